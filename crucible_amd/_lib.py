@@ -63,6 +63,11 @@ SIGNATURES = {
                                          _I64, _I64, _P, _I64, _P], _I),
     "crucible_linear_swiglu_f64acc_prefetch": ([_P, _I64, _P, ctypes.c_float, _P, _P, _I64,
                                                 _I64, _P, _I64, _I64, _P, _I64, _P], _I),
+    "crucible_linear_workspace_bytes": ([_I64, _I64, _I64, _I, _I], _SZ),
+    "crucible_linear_f64acc_ws": ([_P, _I64, _P, ctypes.c_float, _P, _I64, _I64, _P, _P, _I64,
+                                   _I64, _P, _SZ, _P], _I),
+    "crucible_linear_swiglu_f64acc_ws": ([_P, _I64, _P, ctypes.c_float, _P, _P, _I64, _I64, _P,
+                                          _I64, _I64, _P, _SZ, _P], _I),
     "crucible_rmsnorm_rows": ([_P, _I64, _P, ctypes.c_float, _P, _I64, _I64, _I64, _P], _I),
     "crucible_rope_split_qkv": ([_P, _I64, _P, _P, _P, _P, _P, _P] + [_I64] * 5 + [_P], _I),
     "crucible_segments_from_cu_seqlens": ([_P, _I64, _P, _P], _I64),

@@ -148,6 +148,15 @@ __device__ __forceinline__ void lds_dma16(const void* src, uint32_t lds_base) {
                  : "memory", "m0");
 }
 
+// The same with a wave-uniform base and a 32-bit byte offset a lane: no 64-bit address
+// arithmetic on the vector unit.
+__device__ __forceinline__ void lds_dma16_base(const void* base, uint32_t off, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(off), "s"(base), "s"(lds_base)
+                 : "memory", "m0");
+}
+
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {
     return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)p);
 }

@@ -1,0 +1,565 @@
+// Prompt-sized projections with the f64 contract on the int8 matrix cores.
+//
+// The contract is that of model_ops.hip: y = f32(sum_k f64(w[n][k]) * f64(h[m][k])), the
+// reference CPU model's matvec (engine/src/ops.rs:17-32), with RMSNorm, residual and SwiGLU
+// fused. linear_gemm_kernel runs it on the f64 MFMA, whose rate (64 MACs per CU and cycle)
+// bounds it; the int8 MFMA does 4096. So the operands are written as sums of signed 8-bit
+// digits, every digit product is an exact int8 GEMM with int32 sums, and the sums join in
+// f64 at the end:
+//   - a weight is a whole multiple of 2^-24 (fp16's smallest step): w = 2^-24 sum_j w_j
+//     256^(2-j), 3 digits for |w| < 0.498, a 4th (j = -1) up to |w| <= 127;
+//   - a row of activations is scaled by a power of two to |X| < 2^46 and rounded to a whole
+//     number: X = sum_i x_i 256^(5-i), 6 digits. An f32 within 2^22 of its row's largest
+//     value keeps every bit; a smaller one is rounded to 2^-46 of the largest, so its term
+//     is off by at most 2^-47 max|h| |w| (for rows of N(0,1) values about one row in a
+//     thousand holds one such element);
+//   - digit products of equal weight, s = i + j, share an accumulator: 17 products (i, j)
+//     in 7 accumulators. (5, 2), the smallest, is left out: at most 2^-55 max|h| a key, and
+//     nonzero only where the last digit is: elements 2^14 below their row's largest.
+// Rows that this does not fit (a non-finite value, a largest value outside 2^+-60, more than
+// one element in 16 with a last digit) and columns with a weight over 127 or not finite take plain f64 sums instead, 32 x 32
+// outputs at a time.
+//
+// Two launches: digits_kernel writes the digit planes of both operands into the caller's
+// workspace in MFMA operand order, digits_gemm_kernel multiplies them.
+//
+// Included by model_ops.hip, whose floating-point contraction setting (off) it relies on.
+#pragma once
+
+#include "common.hpp"
+
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
+namespace crucible {
+namespace {
+
+enum DigitMode { kDigitPlain = 0, kDigitResidual = 1, kDigitSwiGLU = 2 };
+
+constexpr int kDecodeRows = 32;  // batches up to here keep the decode tilings
+
+struct DigitLinear {
+    const float* x;
+    int64_t ldx;
+    const float* norm_w;  // fused RMSNorm weight, or nullptr
+    double eps;
+    const half_t* w;      // [n_out][k_in]; the gate rows when w2 is set
+    const half_t* w2;     // SwiGLU: the up rows
+    const float* resid;
+    float* out;
+    int64_t ldo;
+    int rows;
+    int n_out;
+    int k_in;
+};
+
+
+typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
+typedef int32_t i32x16_t __attribute__((ext_vector_type(16)));
+
+constexpr int kXDigits = 6;
+constexpr int kWDigits = 4;         // the last one is zero for |w| < 0.498
+constexpr int kBlk = 32;            // rows (columns) of an operand block
+constexpr int kStep = 32;           // K of one MFMA
+constexpr int kFrag = kBlk * kStep; // bytes of one digit of an operand block: 1 KiB
+constexpr int kXBlk = kXDigits * kFrag;
+constexpr int kWBlk = kWDigits * kFrag;
+constexpr int kPart = 128;          // K range of one weight workgroup
+constexpr int kWgRows = 8;          // rows of one activation workgroup
+constexpr int kRowWgs = kBlk / kWgRows;
+constexpr int kMaxK = 16384;        // 4 products of 2^14 a key stay below 2^31
+
+// Workspace: the planes' blocks first (1 KiB aligned), then the rows' scales, then flags.
+//   x planes [row block][K / 32][6][1024], w planes [column block][K / 32][4][1024]
+struct Layout {
+    int64_t row_blks, col_blks, parts;
+    int64_t w_off, scale_off, norm_off, xflag_off, wflag_off, bytes;
+};
+
+Layout make_layout(int64_t rows, int64_t cols, int64_t k_in) {
+    Layout l;
+    const int64_t steps = k_in / kStep;
+    // 64-row and 64-column tiles: both blocks of the last tile exist
+    l.row_blks = (rows + 63) / 64 * 2;
+    l.col_blks = (cols + 63) / 64 * 2;
+    l.parts = (k_in + kPart - 1) / kPart;
+    l.w_off = l.row_blks * steps * kXBlk;
+    l.scale_off = l.w_off + l.col_blks * steps * kWBlk;
+    l.norm_off = l.scale_off + l.row_blks * kBlk * 8;
+    l.xflag_off = l.norm_off + l.row_blks * kBlk * 8;
+    l.wflag_off = l.xflag_off + l.row_blks * kRowWgs * 4;
+    l.bytes = l.wflag_off + l.col_blks * l.parts * 4;
+    return l;
+}
+
+struct DigitArgs {
+    DigitLinear p;
+    unsigned char* ws;
+    Layout l;
+    int row_wgs;    // digits_kernel: workgroups of the activations
+    int row_tiles;  // 64 x 64 output tiles
+    int col_tiles;
+    int per_xcd;
+};
+
+// The weight row behind column c of the product. SwiGLU interleaves 16 gate columns with
+// the up columns of the same outputs, so one 32-column block holds both halves.
+__device__ __forceinline__ const half_t* weight_row(const DigitLinear& p, int c, bool& ok) {
+    if (p.w2) {
+        const int n = (c >> 5) * 16 + (c & 15);
+        ok = n < p.n_out;
+        return ((c & 16) ? p.w2 : p.w) + (int64_t)(ok ? n : 0) * p.k_in;
+    }
+    ok = c < p.n_out;
+    return p.w + (int64_t)(ok ? c : 0) * p.k_in;
+}
+
+// Byte b of four words as one word (v_perm_b32 selects bytes of {first = 7..4, second = 3..0}).
+__device__ __forceinline__ uint32_t bytes_of(uint32_t a0, uint32_t a1, uint32_t a2, uint32_t a3,
+                                             int b) {
+    const uint32_t lo = __builtin_amdgcn_perm(a1, a0, 0x0c0c0400u + 0x0101u * b);
+    const uint32_t hi = __builtin_amdgcn_perm(a3, a2, 0x04000c0cu + 0x01010000u * b);
+    return lo | hi;
+}
+
+// ---------------------------------------------------------------- digit planes
+
+constexpr int kDigitThreads = 256;
+
+// Memory-bound: 4 B read and 6 written per activation, 2 and 4 per weight. A thread
+// handles groups of 16 consecutive K of a row, the 16 bytes one lane supplies to an MFMA for
+// each digit; 8 neighbouring lanes hold 8 rows, so a digit's stores are 128-byte runs (8 rows
+// a workgroup against 16: 4,713 x 2048 22.4 -> 19.4 us, 1,003 x 768 12.6 -> 11.4). The digits need the row's norm and largest value first: with G > 0 (k_in <= 512 G) a thread's
+// groups wait in registers, loaded at once; G = 0 reads the row twice.
+template <int G, bool NORM>
+__global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
+    __shared__ double s_ss[32][kWgRows];
+    __shared__ uint32_t s_mx[32][kWgRows];
+    __shared__ int s_low[32][kWgRows];
+    __shared__ int s_flag;
+    const DigitLinear& p = a.p;
+    const int tid = threadIdx.x;
+    const int steps = p.k_in / kStep;
+    const int r = tid & 7, kg = tid >> 3;  // row (of 8), group of 16 K (of 32)
+
+    if ((int)blockIdx.x >= a.row_wgs) {
+        // ---- weights: 32 rows x kPart
+        const int id = blockIdx.x - a.row_wgs;
+        const int blk = id / (int)a.l.parts, part = id - blk * (int)a.l.parts;
+        if (tid == 0) s_flag = 0;
+        __syncthreads();
+        const int row = tid & 31;
+        const int k = part * kPart + (tid >> 5) * 16;
+        if (k < p.k_in) {
+            bool ok;
+            const half_t* src = weight_row(p, blk * kBlk + row, ok) + k;
+            half8_t v[2];
+            v[0] = *reinterpret_cast<const half8_t*>(src);
+            v[1] = *reinterpret_cast<const half8_t*>(src + 8);
+            uint32_t wv[16];
+            int flag = 0;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const float f = ok ? (float)v[e >> 3][e & 7] : 0.0f;
+                const bool fits = fabsf(f) <= 127.0f;  // false for NaN
+                const int wi = fits ? (int)(f * 16777216.0f) : 0;
+                wv[e] = ((uint32_t)wi + 0x808080u) ^ 0x808080u;
+                flag |= fits ? ((wv[e] >> 24) != 0 ? 1 : 0) : 2;
+            }
+            unsigned char* dst = a.ws + a.l.w_off + ((int64_t)blk * steps + k / kStep) * kWBlk +
+                                 ((k & 16) ? 512 : 0) + row * 16;
+#pragma unroll
+            for (int j = 0; j < kWDigits; ++j) {  // digit j: bytes 2, 1, 0, then 3
+                const int b = j < 3 ? 2 - j : 3;
+                u32x4_t o;
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    o[q] = bytes_of(wv[4 * q], wv[4 * q + 1], wv[4 * q + 2], wv[4 * q + 3], b);
+                *reinterpret_cast<u32x4_t*>(dst + j * kFrag) = o;
+            }
+            if (flag) atomicOr(&s_flag, flag);
+        }
+        __syncthreads();
+        if (tid == 0) reinterpret_cast<int*>(a.ws + a.l.wflag_off)[id] = s_flag;
+        return;
+    }
+
+    // ---- activations: 8 rows, all of K
+    const int row = blockIdx.x * kWgRows + r;
+    const bool ok = row < p.rows;
+    const float* src = p.x + (int64_t)(ok ? row : 0) * p.ldx;
+    const int groups = p.k_in / 16;
+    struct Group {
+        float4_t x[4], nw[NORM ? 4 : 1];
+    };
+    auto load = [&](int g, Group& v) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            v.x[q] = *reinterpret_cast<const float4_t*>(src + g * 16 + 4 * q);
+            if constexpr (NORM)
+                v.nw[q] = *reinterpret_cast<const float4_t*>(p.norm_w + g * 16 + 4 * q);
+        }
+    };
+    // first pass: the f64 sum of squares and a bound of the largest |h|, as float bits (an
+    // infinity or a NaN is the largest)
+    double ss = 0.0;
+    uint32_t mx = 0;
+    auto measure = [&](const Group& v) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float m = v.x[q][e];
+                if constexpr (NORM) {
+                    const double d = (double)m;
+                    ss += d * d;
+                    m *= v.nw[q][e];
+                }
+                mx = max(mx, __builtin_bit_cast(uint32_t, m) & 0x7fffffffu);
+            }
+    };
+    Group held[G > 0 ? G : 1];
+    if constexpr (G > 0) {
+        // a group past the row's end re-reads the last one: its digits are not written
+#pragma unroll
+        for (int i = 0; i < G; ++i) load(min(kg + 32 * i, groups - 1), held[i]);
+#pragma unroll
+        for (int i = 0; i < G; ++i)
+            if (kg + 32 * i < groups) measure(held[i]);
+    } else {
+        for (int g = kg; g < groups; g += 32) {
+            load(g, held[0]);
+            measure(held[0]);
+        }
+    }
+    s_ss[kg][r] = ss;
+    s_mx[kg][r] = mx;
+    __syncthreads();
+    double tot = 0.0;
+    mx = 0;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+        tot += s_ss[i][r];
+        mx = max(mx, s_mx[i][r]);
+    }
+    const double scale = NORM ? 1.0 / sqrt(tot / (double)p.k_in + p.eps) : 1.0;
+    // |h| <= bound (1 + 2^-18 covers the roundings of h), so |h| 2^(21 - e) < 2^22 with e
+    // the exponent of 2^e > bound / 2
+    const float bound = (float)((double)__builtin_bit_cast(float, mx) * scale * 1.00001);
+    const int e = (int)((__builtin_bit_cast(uint32_t, bound) >> 23) & 255) - 127;
+    // Usual magnitudes only: every power of two below is a normal f32.
+    const bool usual = mx < 0x7f800000u && e >= -60 && e <= 60;
+    const bool zero = mx == 0;
+    const float up = usual ? __builtin_bit_cast(float, (uint32_t)(21 - e + 127) << 23) : 0.0f;
+    int low = 0;
+    unsigned char* blk = a.ws + (int64_t)(row >> 5) * steps * kXBlk + (row & 31) * 16;
+    auto write = [&](int g, const Group& v) {
+        uint32_t hi[16], lo[16];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float h = v.x[q][i];
+                if constexpr (NORM) h = (float)((double)h * scale) * v.nw[q][i];
+                const float t = ok && usual ? h * up : 0.0f;        // exact
+                const float th = rintf(t);
+                const float tl = (t - th) * 16777216.0f;            // exact, |tl| <= 2^23
+                const float tr = rintf(tl);                         // rounds below 2^-22 of the largest
+                const uint32_t l = (uint32_t)((int)tr + 0x808080);  // 25 bits, carry on top
+                low += (l & 0xffu) != 0x80u;                        // its last digit is used
+                hi[4 * q + i] = ((uint32_t)((int)th + (int)(l >> 24) + 0x808080)) ^ 0x808080u;
+                lo[4 * q + i] = l ^ 0x808080u;
+            }
+        unsigned char* dst = blk + (int64_t)(g >> 1) * kXBlk + ((g & 1) ? 512 : 0);
+#pragma unroll
+        for (int i = 0; i < kXDigits; ++i) {
+            u32x4_t o;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                o[q] = i < 3 ? bytes_of(hi[4 * q], hi[4 * q + 1], hi[4 * q + 2], hi[4 * q + 3], 2 - i)
+                             : bytes_of(lo[4 * q], lo[4 * q + 1], lo[4 * q + 2], lo[4 * q + 3], 5 - i);
+            *reinterpret_cast<u32x4_t*>(dst + i * kFrag) = o;
+        }
+    };
+    if constexpr (G > 0) {
+#pragma unroll
+        for (int i = 0; i < G; ++i)
+            if (kg + 32 * i < groups) write(kg + 32 * i, held[i]);
+    } else {
+        for (int g = kg; g < groups; g += 32) {
+            load(g, held[0]);
+            write(g, held[0]);
+        }
+    }
+    s_low[kg][r] = low;
+    if (tid == 0) s_flag = 0;
+    __syncthreads();
+    if (kg == 0) {
+#pragma unroll
+        for (int i = 1; i < 32; ++i) low += s_low[i][r];
+        // 2^(e - 45) per unit of X, 2^-24 per unit of W, 2^8 per unit of the last group
+        reinterpret_cast<double*>(a.ws + a.l.scale_off)[row] =
+            usual ? __builtin_bit_cast(double, (uint64_t)(e - 61 + 1023) << 52) : 0.0;
+        reinterpret_cast<double*>(a.ws + a.l.norm_off)[row] = scale;
+        if (ok && !zero && (!usual || low * 16 > p.k_in)) atomicOr(&s_flag, 1);
+    }
+    __syncthreads();
+    if (tid == 0) reinterpret_cast<int*>(a.ws + a.l.xflag_off)[blockIdx.x] = s_flag;
+}
+
+// ---------------------------------------------------------------- digit products
+
+constexpr int kDigitGemmThreads = 256;
+constexpr int kGroups = 8;                 // s = i + j = -1 .. 6
+constexpr int kStageK = 64;                // K of a stage: two MFMA steps
+constexpr int kStageX = 2 * 2 * kXBlk;     // 2 row blocks x 2 steps: 24 KiB
+constexpr int kStage = kStageX + 2 * 2 * 3 * kFrag;  // 2 column blocks x 2 steps, 3 digits
+
+// A 64 x 64 output tile per workgroup of 4 waves, 32 x 32 a wave. MFMA-bound: 17 products of
+// 32x32x32 a wave and step (23 with the fourth weight digit) against 9 KiB of LDS reads.
+// Stages of 64 keys stream into two LDS buffers with direct-to-LDS loads, the next stage's
+// issued between the products; the planes are stored in operand order, so both the copy and
+// the reads are linear in the lane and free of bank conflicts. Two workgroups a CU (73.7 KB
+// of LDS each): one multiplies while the other waits at its barrier. The weights' fourth
+// digit, rare, goes from global memory to registers.
+//
+// With every SIMD busy on random digits the part runs a 32x32x32 product in 20 ns (13.7 with
+// a few CUs busy): 150 us for the gate/up product of 4,713 rows (252 G multiply-adds).
+// Measured slower: steps of 32 in a ring of 4 (2 workgroups a CU) or 8 buffers, operands
+// double-buffered in registers, and 32 x 64 outputs a wave (one wave a SIMD, 512 VGPRs).
+//
+// int8 MFMA 32x32x32: lane l supplies row (column) l & 31 and 16 of the step's 32 keys, the
+// half l >> 5 of them (the same keys for both operands), and holds
+// D[8 (i >> 2) + 4 (l >> 5) + (i & 3)][l & 31].
+template <int MODE>
+__global__ __launch_bounds__(kDigitGemmThreads, 2) void digits_gemm_kernel(DigitArgs a) {
+    __shared__ __align__(1024) unsigned char s_buf[2][kStage];
+    const DigitLinear& p = a.p;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = wave >> 1, wc = wave & 1;
+
+    // Workgroup L runs on XCD L % 8; each XCD takes a contiguous piece of the tile list,
+    // which walks groups of 8 row tiles column by column: the group's x planes (2.4 MB at
+    // K = 768) and a column's w planes stay in the XCD's L2.
+    const int L = blockIdx.x;
+    const int t = (L & 7) * a.per_xcd + (L >> 3);
+    if (t >= a.row_tiles * a.col_tiles) return;  // uniform over the workgroup
+    const int group = t / (8 * a.col_tiles);
+    const int in_group = min(8, a.row_tiles - 8 * group);
+    const int rem = t - group * 8 * a.col_tiles;
+    const int ct = rem / in_group;
+    const int rt = group * 8 + rem - ct * in_group;
+
+    const int steps = p.k_in / kStep;
+    const int n_stage = p.k_in / kStageK;
+    const unsigned char* wp = a.ws + a.l.w_off + (int64_t)(2 * ct) * steps * kWBlk;
+
+    // Flags: f64 for the wave's outputs if its row or column block needs it, a fourth weight
+    // digit if one is nonzero anywhere in the wave's columns.
+    const int* xf = reinterpret_cast<const int*>(a.ws + a.l.xflag_off) + (2 * rt + wr) * kRowWgs;
+    const int* wf = reinterpret_cast<const int*>(a.ws + a.l.wflag_off) +
+                    (int64_t)(2 * ct + wc) * a.l.parts;
+    int wflag = 0;
+    for (int i = 0; i < (int)a.l.parts; ++i) wflag |= wf[i];
+    wflag = __builtin_amdgcn_readfirstlane(wflag);
+    const bool plain = __builtin_amdgcn_readfirstlane(xf[0] | xf[1] | xf[2] | xf[3]) != 0 || (wflag & 2) != 0;
+    const bool four = (wflag & 1) != 0;
+
+    // One stage: 24 + 12 blocks of 1 KiB. x block (row block b, step q, digit i) goes to LDS
+    // slot (b * 2 + q) * 6 + i, w block (b, q, j) to 24 + (b * 2 + q) * 3 + j. Wave w loads
+    // (b, q) = (w >> 1, w & 1): 6 + 3 of them, at fixed distances from two running bases.
+    const unsigned char* xsrc = a.ws + ((int64_t)(2 * rt + wr) * steps + wc) * kXBlk;
+    const unsigned char* wsrc = wp + ((int64_t)wr * steps + wc) * kWBlk;
+    const uint32_t lds0 = lds_offset(&s_buf[0][0]);
+    const uint32_t voff = (uint32_t)lane * 16;
+    auto issue_one = [&](int i, int buf) {  // i = 0 .. 8
+        const uint32_t at = lds0 + (uint32_t)(buf * kStage);
+        if (i < kXDigits) lds_dma16_base(xsrc + i * kFrag, voff, at + (uint32_t)((wave * 6 + i) * kFrag));
+        else lds_dma16_base(wsrc + (i - 6) * kFrag, voff,
+                            at + (uint32_t)(kStageX + (wave * 3 + i - 6) * kFrag));
+    };
+
+    i32x16_t acc[kGroups];
+#pragma unroll
+    for (int s = 0; s < kGroups; ++s)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[s][i] = 0;
+
+    struct Frag {
+        i32x4_t x[kXDigits], w[3];
+    };
+    auto read = [&](int buf, int q, Frag& f) {
+        const unsigned char* base = &s_buf[buf][0] + lane * 16;
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            f.w[j] = *reinterpret_cast<const i32x4_t*>(base + kStageX + ((wc * 2 + q) * 3 + j) * kFrag);
+#pragma unroll
+        for (int i = 0; i < kXDigits; ++i)
+            f.x[i] = *reinterpret_cast<const i32x4_t*>(base + ((wr * 2 + q) * 6 + i) * kFrag);
+    };
+    auto loop = [&](auto four_tag) {
+        constexpr bool kFour = decltype(four_tag)::value;
+        for (int st = 0; st < n_stage; ++st) {
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            // the stage is in LDS, and every wave has read the other buffer (stage st - 1)
+            const int buf = st & 1;
+            Frag f[2];
+            read(buf, 0, f[0]);
+            read(buf, 1, f[1]);
+            // The next stage's loads; the last stage re-reads itself into the free buffer.
+            const bool more = st + 1 < n_stage;
+            xsrc += more ? 2 * kXBlk : 0;
+            wsrc += more ? 2 * kWBlk : 0;
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                i32x4_t w4;
+                if constexpr (kFour)
+                    w4 = *reinterpret_cast<const i32x4_t*>(
+                        wp + ((int64_t)wc * steps + 2 * st + q) * kWBlk + 3 * kFrag + lane * 16);
+                // j outer: consecutive products go to different accumulators
+                int n = 0;
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+#pragma unroll
+                    for (int i = 0; i < kXDigits; ++i) {
+                        if (i + j >= 7) continue;
+                        acc[i + j + 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+                            f[q].x[i], f[q].w[j], acc[i + j + 1], 0, 0, 0);
+                        if (!kFour && q == 0 && (n & 1) == 0 && n < 18) {
+                            __builtin_amdgcn_sched_barrier(0);
+                            issue_one(n >> 1, buf ^ 1);
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                        ++n;
+                    }
+                if constexpr (kFour) {
+#pragma unroll
+                    for (int i = 0; i < kXDigits; ++i)
+                        acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f[q].x[i], w4, acc[i], 0, 0, 0);
+                }
+            }
+            if constexpr (kFour)
+#pragma unroll
+                for (int i = 0; i < 9; ++i) issue_one(i, buf ^ 1);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < 9; ++i) issue_one(i, 0);
+    // The choice is per wave, and both loops pass the same barriers.
+    if (four) loop(std::true_type{});
+    else loop(std::false_type{});
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into LDS outlives the workgroup
+
+    // ---- outputs: column c of the wave's block, rows 8 (i >> 2) + 4 (lane >> 5) + (i & 3)
+    const int r0 = (2 * rt + wr) * kBlk + 4 * (lane >> 5);
+    const double* scales = reinterpret_cast<const double*>(a.ws + a.l.scale_off);
+    const int c = (2 * ct + wc) * kBlk + (lane & 31);
+    bool col_ok;
+    const half_t* wrow = weight_row(p, c, col_ok);
+    const int n = MODE == kDigitSwiGLU ? (c >> 5) * 16 + (c & 15) : c;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int row = r0 + 8 * (i >> 2) + (i & 3);
+        double v = (double)acc[0][i];
+#pragma unroll
+        for (int s = 1; s < kGroups; ++s) v = v * 256.0 + (double)acc[s][i];
+        float y = (float)(v * scales[row]);
+        if (plain) {
+            const double ns = reinterpret_cast<const double*>(a.ws + a.l.norm_off)[row];
+            const float* xr = p.x + (int64_t)min(row, p.rows - 1) * p.ldx;
+            double sum = 0.0;
+            for (int k = 0; k < p.k_in; ++k) {
+                const float h = p.norm_w ? (float)((double)xr[k] * ns) * p.norm_w[k] : xr[k];
+                sum += (double)h * (double)(float)wrow[k];
+            }
+            y = (float)sum;
+        }
+        const bool ok = row < p.rows && col_ok;
+        if constexpr (MODE == kDigitSwiGLU) {
+            const float u = __shfl_xor(y, 16);  // lanes 0..15 gate, 16..31 up
+            if (ok && !(lane & 16)) p.out[(int64_t)row * p.ldo + n] = y / (1.0f + expf(-y)) * u;
+        } else if constexpr (MODE == kDigitResidual) {
+            // out may alias resid: each element is read and written by the same lane
+            if (ok) p.out[(int64_t)row * p.ldo + n] = p.resid[(int64_t)row * p.ldo + n] + y;
+        } else {
+            if (ok) p.out[(int64_t)row * p.ldo + n] = y;
+        }
+    }
+}
+
+// Which form a product takes, by what each costs. The lines are fits, in us, to graph replays
+// of the 120m and 350m decoders' four products (768 and 1024 wide) at 64 to 1,024 rows, within
+// about 15% there; G = 10^9 multiply-adds:
+//   decode tilings     5 + 52 G, with a fused norm or SwiGLU 5 + 115 G (every workgroup
+//                      normalises its rows again; half-width tiles): 512 x 768 x 768 21.4,
+//                      192 x 1152 x 768 with norm 27.0
+//   int8 digits        a digit and a product launch each as long as K: 11 + 0.0155 K, the
+//                      weights' digits 2e-6 a weight, 10 G once the CUs are full:
+//                      24.6 and 21.9 there, 4,713 rows of gate/up 208
+//   f64 output tiles   one workgroup's whole K, 3 + 0.0345 K, or 39 G: 29.5 and 34.0, 554
+struct LinearCost {
+    double tiles, digits, gemm;
+};
+LinearCost linear_cost(int64_t rows, int64_t n_out, int64_t k_in, bool norm, bool swiglu) {
+    const double k = (double)k_in, weights = (double)n_out * k * (swiglu ? 2 : 1);
+    const double g = weights * (double)rows * 1e-9;
+    return {5.0 + (norm || swiglu ? 115.0 : 52.0) * g, 11.0 + 0.0155 * k + 2e-6 * weights + 10.0 * g,
+            std::max(3.0 + 0.0345 * k, 39.0 * g)};
+}
+
+// Whether a product takes the digits, given a workspace. Decode-sized batches never do: k_in
+// whole stages and within the int32 sums' range; the other bounds keep the grids within 2^31.
+bool digit_linear_fits(int64_t rows, int64_t n_out, int64_t k_in, bool norm, bool swiglu) {
+    if (k_in <= 0 || k_in % kStageK != 0 || k_in > kMaxK || rows <= 0 || rows > 16 * 65535 ||
+        n_out <= 0 || n_out > (1 << 20))
+        return false;
+    if (const int v = tuning(CRUCIBLE_TUNE_LINEAR_TILE); v > 0) return v == 64;
+    if (rows <= kDecodeRows) return false;
+    const LinearCost c = linear_cost(rows, n_out, k_in, norm, swiglu);
+    return c.digits < c.tiles && c.digits < c.gemm;
+}
+
+size_t digit_linear_bytes(int64_t rows, int64_t n_out, int64_t k_in, bool swiglu) {
+    return (size_t)make_layout(rows, swiglu ? (n_out + 15) / 16 * 32 : n_out, k_in).bytes;
+}
+
+int launch_digit_linear(const DigitLinear& p, int mode, void* workspace, hipStream_t stream,
+                        const char* what) {
+    const int64_t cols = p.w2 ? (int64_t)(p.n_out + 15) / 16 * 32 : p.n_out;
+    DigitArgs a{};
+    a.p = p;
+    a.ws = static_cast<unsigned char*>(workspace);
+    a.l = make_layout(p.rows, cols, p.k_in);
+    a.row_wgs = (int)a.l.row_blks * kRowWgs;
+    a.row_tiles = (int)a.l.row_blks / 2;
+    a.col_tiles = (int)a.l.col_blks / 2;
+    a.per_xcd = (int)(((int64_t)a.row_tiles * a.col_tiles + 7) / 8);
+    const dim3 digit_grid((unsigned)(a.row_wgs + a.l.col_blks * a.l.parts));
+    auto digits = [&](auto norm_tag) {
+        constexpr bool kNorm = decltype(norm_tag)::value;
+        if (p.k_in <= 1024)
+            hipLaunchKernelGGL((digits_kernel<2, kNorm>), digit_grid, dim3(kDigitThreads), 0, stream, a);
+        else if (p.k_in <= 2048)
+            hipLaunchKernelGGL((digits_kernel<4, kNorm>), digit_grid, dim3(kDigitThreads), 0, stream, a);
+        else
+            hipLaunchKernelGGL((digits_kernel<0, kNorm>), digit_grid, dim3(kDigitThreads), 0, stream, a);
+    };
+    if (p.norm_w) digits(std::true_type{});
+    else digits(std::false_type{});
+    const dim3 grid((unsigned)(8 * a.per_xcd));
+    if (mode == kDigitSwiGLU)
+        hipLaunchKernelGGL(digits_gemm_kernel<kDigitSwiGLU>, grid, dim3(kDigitGemmThreads), 0, stream, a);
+    else if (mode == kDigitResidual)
+        hipLaunchKernelGGL(digits_gemm_kernel<kDigitResidual>, grid, dim3(kDigitGemmThreads), 0, stream, a);
+    else
+        hipLaunchKernelGGL(digits_gemm_kernel<kDigitPlain>, grid, dim3(kDigitGemmThreads), 0, stream, a);
+    return fail_launch(what);
+}
+
+}  // namespace
+}  // namespace crucible

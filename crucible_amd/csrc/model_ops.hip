@@ -26,6 +26,8 @@
 
 #pragma clang fp contract(off)
 
+#include "linear_digits.hpp"
+
 namespace crucible {
 namespace {
 
@@ -703,7 +705,6 @@ __global__ __launch_bounds__(kLinThreads) void linear_wide_kernel(LinArgs a) {
 // the rows plus the weights, instead of every XCD fetching every row.
 constexpr int kGemmWaves = 4;
 constexpr int kGemmThreads = 64 * kGemmWaves;
-constexpr int kGemmMinRows = 128;  // below this the decode tilings are used
 
 template <int RB, int CB, bool NORM>
 struct GemmChunk {
@@ -992,12 +993,15 @@ void launch_gemm(const LinArgs& a, hipStream_t stream) {
                        dim3(kGemmThreads), 0, stream, a, col_tiles, n_tiles, per_xcd);
 }
 
-// Output-tiled products for prompt-sized row counts (k_in a multiple of 64);
+// Output-tiled products where they cost less than the decode tilings (linear_cost; k_in a
+// multiple of 64): a fixed 128 rows as the line left 256 x 768 x 768 at 29.4 us against 12.6.
 // CRUCIBLE_TUNE_LINEAR_TILE = 32 forces them, 4 or 16 the decode tilings.
-bool use_gemm(int64_t rows, int64_t k_in) {
+bool use_gemm(int64_t rows, int64_t n_out, int64_t k_in, bool norm, bool swiglu) {
     if (k_in % 64 != 0) return false;
     if (const int v = tuning(CRUCIBLE_TUNE_LINEAR_TILE); v > 0) return v == 32;
-    return rows >= kGemmMinRows;
+    if (rows <= kDecodeRows) return false;
+    const LinearCost c = linear_cost(rows, n_out, k_in, norm, swiglu);
+    return c.gemm < c.tiles;
 }
 
 template <int MODE>
@@ -1051,10 +1055,19 @@ void set_prefetch(LinArgs& a, const void* pf, int64_t pf_bytes) {
     a.pf_bytes = pf_bytes;
 }
 
+// A workspace the caller brought: large enough and aligned for the products on int8 digits.
+int check_workspace(const char* what, const void* ws, size_t ws_bytes, size_t need) {
+    CRUCIBLE_CHECK(ws_bytes >= need, CRUCIBLE_ERR_WORKSPACE, "%s: workspace %zu bytes, need %zu",
+                   what, ws_bytes, need);
+    CRUCIBLE_CHECK(aligned16(ws), CRUCIBLE_ERR_INVALID, "%s: workspace must be 16-byte aligned",
+                   what);
+    return CRUCIBLE_OK;
+}
+
 int linear_f64acc(const char* what, const float* x, int64_t ldx, const float* norm_w, float eps,
                   const void* w, int64_t n_out, int64_t k_in, const float* resid, float* out,
-                  int64_t ldo, int64_t rows, const void* pf, int64_t pf_bytes,
-                  crucible_stream_t stream) {
+                  int64_t ldo, int64_t rows, const void* pf, int64_t pf_bytes, void* ws,
+                  size_t ws_bytes, crucible_stream_t stream) {
     int rc = check_linear(what, x, ldx, norm_w, w, n_out, k_in, out, ldo, rows);
     if (rc == CRUCIBLE_OK) rc = check_prefetch(what, pf, pf_bytes);
     if (rc != CRUCIBLE_OK) return rc;
@@ -1062,7 +1075,14 @@ int linear_f64acc(const char* what, const float* x, int64_t ldx, const float* no
     LinArgs a{x, ldx, norm_w, (double)eps, static_cast<const half_t*>(w), nullptr, resid, out,
               ldo, (int)rows, (int)n_out, (int)k_in};
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (use_gemm(rows, k_in)) {
+    if (ws && digit_linear_fits(rows, n_out, k_in, norm_w != nullptr, false)) {
+        rc = check_workspace(what, ws, ws_bytes, digit_linear_bytes(rows, n_out, k_in, false));
+        if (rc != CRUCIBLE_OK) return rc;
+        return launch_digit_linear({x, ldx, norm_w, (double)eps, a.w, nullptr, resid, out, ldo,
+                                    a.rows, a.n_out, a.k_in},
+                                   resid ? kDigitResidual : kDigitPlain, ws, s, what);
+    }
+    if (use_gemm(rows, n_out, k_in, norm_w != nullptr, false)) {
         if (resid) launch_gemm_mode<kResidual>(a, s);
         else launch_gemm_mode<kPlain>(a, s);
         return fail_launch(what);
@@ -1129,7 +1149,8 @@ int linear_f64acc(const char* what, const float* x, int64_t ldx, const float* no
 int linear_swiglu_f64acc(const char* what, const float* x, int64_t ldx, const float* norm_w,
                          float eps, const void* w_gate, const void* w_up, int64_t hidden,
                          int64_t k_in, float* out, int64_t ldo, int64_t rows, const void* pf,
-                         int64_t pf_bytes, crucible_stream_t stream) {
+                         int64_t pf_bytes, void* ws, size_t ws_bytes,
+                         crucible_stream_t stream) {
     int rc = check_linear(what, x, ldx, norm_w, w_gate, hidden, k_in, out, ldo, rows);
     if (rc == CRUCIBLE_OK) rc = check_prefetch(what, pf, pf_bytes);
     if (rc != CRUCIBLE_OK) return rc;
@@ -1140,7 +1161,14 @@ int linear_swiglu_f64acc(const char* what, const float* x, int64_t ldx, const fl
               static_cast<const half_t*>(w_up), nullptr, out, ldo, (int)rows, (int)hidden,
               (int)k_in};
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (use_gemm(rows, k_in)) {
+    if (ws && digit_linear_fits(rows, hidden, k_in, norm_w != nullptr, true)) {
+        rc = check_workspace(what, ws, ws_bytes, digit_linear_bytes(rows, hidden, k_in, true));
+        if (rc != CRUCIBLE_OK) return rc;
+        return launch_digit_linear({x, ldx, norm_w, (double)eps, a.w, a.w2, nullptr, out, ldo,
+                                    a.rows, a.n_out, a.k_in},
+                                   kDigitSwiGLU, ws, s, what);
+    }
+    if (use_gemm(rows, hidden, k_in, norm_w != nullptr, true)) {
         launch_gemm_mode<kSwiGLU>(a, s);
         return fail_launch(what);
     }
@@ -1166,7 +1194,7 @@ extern "C" int crucible_linear_f64acc(const float* x, int64_t ldx, const float* 
                                       const float* resid, float* out, int64_t ldo, int64_t rows,
                                       crucible_stream_t stream) {
     return linear_f64acc("crucible_linear_f64acc", x, ldx, norm_w, eps, w, n_out, k_in, resid,
-                         out, ldo, rows, nullptr, 0, stream);
+                         out, ldo, rows, nullptr, 0, nullptr, 0, stream);
 }
 
 extern "C" int crucible_linear_f64acc_prefetch(const float* x, int64_t ldx, const float* norm_w,
@@ -1175,7 +1203,7 @@ extern "C" int crucible_linear_f64acc_prefetch(const float* x, int64_t ldx, cons
                                                int64_t ldo, int64_t rows, const void* prefetch,
                                                int64_t prefetch_bytes, crucible_stream_t stream) {
     return linear_f64acc("crucible_linear_f64acc_prefetch", x, ldx, norm_w, eps, w, n_out, k_in,
-                         resid, out, ldo, rows, prefetch, prefetch_bytes, stream);
+                         resid, out, ldo, rows, prefetch, prefetch_bytes, nullptr, 0, stream);
 }
 
 extern "C" int crucible_linear_swiglu_f64acc(const float* x, int64_t ldx, const float* norm_w,
@@ -1184,7 +1212,7 @@ extern "C" int crucible_linear_swiglu_f64acc(const float* x, int64_t ldx, const 
                                              int64_t ldo, int64_t rows,
                                              crucible_stream_t stream) {
     return linear_swiglu_f64acc("crucible_linear_swiglu_f64acc", x, ldx, norm_w, eps, w_gate,
-                                w_up, hidden, k_in, out, ldo, rows, nullptr, 0, stream);
+                                w_up, hidden, k_in, out, ldo, rows, nullptr, 0, nullptr, 0, stream);
 }
 
 extern "C" int crucible_linear_swiglu_f64acc_prefetch(const float* x, int64_t ldx,
@@ -1197,7 +1225,33 @@ extern "C" int crucible_linear_swiglu_f64acc_prefetch(const float* x, int64_t ld
                                                       crucible_stream_t stream) {
     return linear_swiglu_f64acc("crucible_linear_swiglu_f64acc_prefetch", x, ldx, norm_w, eps,
                                 w_gate, w_up, hidden, k_in, out, ldo, rows, prefetch,
-                                prefetch_bytes, stream);
+                                prefetch_bytes, nullptr, 0, stream);
+}
+
+extern "C" size_t crucible_linear_workspace_bytes(int64_t rows, int64_t n_out, int64_t k_in,
+                                                  int norm, int swiglu) {
+    return digit_linear_fits(rows, n_out, k_in, norm != 0, swiglu != 0)
+               ? digit_linear_bytes(rows, n_out, k_in, swiglu != 0)
+               : 0;
+}
+
+extern "C" int crucible_linear_f64acc_ws(const float* x, int64_t ldx, const float* norm_w,
+                                         float eps, const void* w, int64_t n_out, int64_t k_in,
+                                         const float* resid, float* out, int64_t ldo, int64_t rows,
+                                         void* workspace, size_t workspace_bytes,
+                                         crucible_stream_t stream) {
+    return linear_f64acc("crucible_linear_f64acc_ws", x, ldx, norm_w, eps, w, n_out, k_in, resid,
+                         out, ldo, rows, nullptr, 0, workspace, workspace_bytes, stream);
+}
+
+extern "C" int crucible_linear_swiglu_f64acc_ws(const float* x, int64_t ldx, const float* norm_w,
+                                                float eps, const void* w_gate, const void* w_up,
+                                                int64_t hidden, int64_t k_in, float* out,
+                                                int64_t ldo, int64_t rows, void* workspace,
+                                                size_t workspace_bytes, crucible_stream_t stream) {
+    return linear_swiglu_f64acc("crucible_linear_swiglu_f64acc_ws", x, ldx, norm_w, eps, w_gate,
+                                w_up, hidden, k_in, out, ldo, rows, nullptr, 0, workspace,
+                                workspace_bytes, stream);
 }
 
 extern "C" int crucible_rmsnorm_rows(const float* x, int64_t ldx, const float* w, float eps,

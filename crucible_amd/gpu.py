@@ -146,6 +146,12 @@ class Gpu:
             self._bindings[key] = binding
         return ws
 
+    def _scratch(self, nbytes: int) -> torch.Tensor:
+        """Scratch of one call, from torch's caching allocator on the current stream: the
+        block goes back when the call returns and only later work of the same stream (or
+        graph) can take it, so calls on several streams and threads never share one."""
+        return torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+
     @staticmethod
     def version() -> str:
         return _lib.load().crucible_attn_version().decode()
@@ -365,7 +371,12 @@ class Gpu:
         args = (_ptr(x), k_in, _ptr(norm_w) if norm_w is not None else None, float(eps),
                 _ptr(w), n_out, k_in, _ptr(resid) if resid is not None else None, _ptr(out),
                 n_out, rows)
-        if prefetch is None:
+        nbytes = self.lib.crucible_linear_workspace_bytes(rows, n_out, k_in, norm_w is not None, 0)
+        if nbytes and (prefetch is None or _prefetch_region(prefetch)[0] % 4 == 0):
+            ws = self._scratch(nbytes)
+            _lib.check(self.lib.crucible_linear_f64acc_ws(*args, _ptr(ws), nbytes,
+                                                          self._stream()))
+        elif prefetch is None:
             _lib.check(self.lib.crucible_linear_f64acc(*args, self._stream()))
         else:
             _lib.check(self.lib.crucible_linear_f64acc_prefetch(
@@ -386,7 +397,12 @@ class Gpu:
             _need(norm_w, "norm_w", dtype=torch.float32, numel=k_in)
         args = (_ptr(x), k_in, _ptr(norm_w) if norm_w is not None else None, float(eps),
                 _ptr(w_gate), _ptr(w_up), hidden, k_in, _ptr(out), hidden, rows)
-        if prefetch is None:
+        nbytes = self.lib.crucible_linear_workspace_bytes(rows, hidden, k_in, norm_w is not None, 1)
+        if nbytes and (prefetch is None or _prefetch_region(prefetch)[0] % 4 == 0):
+            ws = self._scratch(nbytes)
+            _lib.check(self.lib.crucible_linear_swiglu_f64acc_ws(*args, _ptr(ws), nbytes,
+                                                                 self._stream()))
+        elif prefetch is None:
             _lib.check(self.lib.crucible_linear_swiglu_f64acc(*args, self._stream()))
         else:
             _lib.check(self.lib.crucible_linear_swiglu_f64acc_prefetch(

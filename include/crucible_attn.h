@@ -89,7 +89,8 @@ enum crucible_tuning_key {
     CRUCIBLE_TUNE_PREFILL_HEAVY_FIRST = 4, /* prefill longest-first grid: 0, 1 */
     CRUCIBLE_TUNE_PREFILL_QB = 5,          /* prefill 16-row blocks per wave: 1, 2 */
     CRUCIBLE_TUNE_PREFILL_BUFS = 6,        /* prefill LDS ring depth in key tiles: 4, 6 */
-    CRUCIBLE_TUNE_LINEAR_TILE = 7,         /* projection tiles: 4 or 16 columns (decode), 32 (prompt rows) */
+    CRUCIBLE_TUNE_LINEAR_TILE = 7,         /* projection tiles: 4 or 16 columns (decode), 32 (prompt rows),
+                                              64 (int8 digits, where a workspace is given) */
     CRUCIBLE_TUNE_DECODE_COMBINE_WIDTH = 8, /* decode splits merged per round trip: 8, 16 */
     CRUCIBLE_TUNE_PREFILL_P16 = 9,         /* prefill P operand: 0 fp16 hi + lo (default), 1 one fp16 */
     CRUCIBLE_TUNE_PREFILL_M32 = 10,        /* prefill 32-row waves on 32x32 MFMAs: 1 (default), 0 */
@@ -429,6 +430,32 @@ int crucible_linear_swiglu_f64acc_prefetch(const float* x, int64_t ldx, const fl
                                            int64_t hidden, int64_t k_in, float* out,
                                            int64_t ldo, int64_t rows, const void* prefetch,
                                            int64_t prefetch_bytes, crucible_stream_t stream);
+
+/* The two products with a caller-owned scratch buffer, for prompt-sized row counts: the same
+ * contract on the int8 matrix cores. Both operands are written into the workspace as signed
+ * 8-bit digits, the digit products accumulate exactly in int32 and join in f64. Weights keep
+ * every bit; a row's activations keep every bit down to 2^-22 of the row's largest and are
+ * rounded to 2^-46 of it below. Rows and columns outside the digits' range (non-finite values,
+ * weights over 127, rows with more than one element in 16 below 2^-14 of the largest) are
+ * summed in f64, so outputs are the plain product's to the order of f64 summation.
+ * crucible_linear_workspace_bytes gives the size (norm, swiglu: whether the call fuses them),
+ * 0 where this form is not used (k_in not a multiple of 64 or above 16384, or few enough
+ * rows that the plain product is faster); the plain product runs then, and also for
+ * workspace = NULL. A workspace of fewer bytes is CRUCIBLE_ERR_WORKSPACE. It needs
+ * 16-byte alignment and no clearing, holds nothing between calls, and belongs to one launch
+ * at a time (launches that share it must be ordered, e.g. on one stream). No counterpart in
+ * the reference, whose prefill multiplies in lower precision (kernels.cu:2402-2526). */
+size_t crucible_linear_workspace_bytes(int64_t rows, int64_t n_out, int64_t k_in, int norm,
+                                       int swiglu);
+int crucible_linear_f64acc_ws(const float* x, int64_t ldx, const float* norm_w, float eps,
+                              const void* w, int64_t n_out, int64_t k_in, const float* resid,
+                              float* out, int64_t ldo, int64_t rows, void* workspace,
+                              size_t workspace_bytes, crucible_stream_t stream);
+int crucible_linear_swiglu_f64acc_ws(const float* x, int64_t ldx, const float* norm_w, float eps,
+                                     const void* w_gate, const void* w_up, int64_t hidden,
+                                     int64_t k_in, float* out, int64_t ldo, int64_t rows,
+                                     void* workspace, size_t workspace_bytes,
+                                     crucible_stream_t stream);
 
 /* RMSNorm of each row (ops.rs:39-52; replaces rmsnorm_batch_f32, kernels.cu:968-996). */
 int crucible_rmsnorm_rows(const float* x, int64_t ldx, const float* w, float eps, float* out,

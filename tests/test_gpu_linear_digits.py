@@ -1,0 +1,162 @@
+"""The projections on int8 digits (linear_tile 64) against the f64 contract.
+
+Sizes sit at the edges of the form: one row and column, either side of its 64 x 64 tiles and
+32-row blocks, one K stage, K in one, two and four register groups and beyond them. Values sit
+at the edges of the digits: weights in three digits (below 0.498), in four (up to 127) and
+past them, rows whose elements span more binades than the six digits, rows with infinities
+and NaN. Products whose operands the digits hold exactly must give the f64 sum rounded once:
+at most 1 ulp (two f64 sums may straddle a rounding boundary) on a handful of elements, as
+test_gpu_model_ops.py asks of the f64 kernels.
+"""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+EPS = np.float32(1e-6)
+
+
+def _ulps(a, b):
+    # signed-magnitude order, so that -0.0 and 0.0 are neighbours of the smallest values
+    def key(x):
+        i = x.astype(np.float32).view(np.int32).astype(np.int64)
+        return np.where(i < 0, -(i & 0x7FFFFFFF), i)
+    return np.abs(key(a) - key(b))
+
+
+def _check(got, want):
+    d = _ulps(got, want)
+    assert d.max() <= 1, f"{d.max()} ulps"
+    assert int((d > 0).sum()) <= max(2, got.size // 20000)
+
+
+def _h(x, nw):
+    if nw is None:
+        return x.astype(np.float64)
+    x64 = x.astype(np.float64)
+    scale = 1.0 / np.sqrt((x64 * x64).mean(axis=1, keepdims=True) + np.float64(EPS))
+    return ((x64 * scale).astype(np.float32) * nw).astype(np.float64)
+
+
+def _run(gpu, dev, x, w, nw=None, resid=None, w_up=None):
+    out = torch.full((x.shape[0], w.shape[0]), np.nan, dtype=torch.float32, device=dev)
+    t = [None if a is None else torch.from_numpy(a).to(dev) for a in (x, w, nw, resid, w_up)]
+    if w_up is not None:
+        gpu.linear_swiglu_f64acc(t[0], t[1], t[4], out, norm_w=t[2], eps=float(EPS))
+    else:
+        gpu.linear_f64acc(t[0], t[1], out, norm_w=t[2], eps=float(EPS), resid=t[3])
+    return out.cpu().numpy()
+
+
+@pytest.mark.parametrize("rows,n_out,k_in", [(1, 1, 64), (31, 33, 128), (64, 64, 64),
+                                             (65, 127, 512), (130, 200, 576), (96, 40, 1088),
+                                             (33, 65, 2048), (40, 130, 2112)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_shapes(gpu, dev, tune, rows, n_out, k_in, norm):
+    tune(linear_tile=64)
+    rng = np.random.default_rng(rows + n_out + k_in)
+    x = rng.standard_normal((rows, k_in), dtype=np.float32)
+    w = (rng.standard_normal((n_out, k_in)) * 0.02).astype(np.float16)
+    nw = (1 + 0.1 * rng.standard_normal(k_in)).astype(np.float32) if norm else None
+    want = (_h(x, nw) @ w.astype(np.float64).T).astype(np.float32)
+    got = _run(gpu, dev, x, w, nw)
+    _check(got, want)
+    assert np.array_equal(got, _run(gpu, dev, x, w, nw)), "not deterministic"
+    r = rng.standard_normal((rows, n_out), dtype=np.float32)
+    assert np.array_equal(_run(gpu, dev, x, w, nw, resid=r), r + got)
+
+
+@pytest.mark.parametrize("rows,hidden,k_in", [(1, 1, 64), (33, 17, 128), (70, 100, 704)])
+def test_swiglu(gpu, dev, tune, rows, hidden, k_in):
+    tune(linear_tile=64)
+    rng = np.random.default_rng(hidden)
+    x = rng.standard_normal((rows, k_in), dtype=np.float32)
+    wg, wu = ((rng.standard_normal((hidden, k_in)) * 0.05).astype(np.float16) for _ in range(2))
+    nw = np.ones(k_in, np.float32)
+    h = _h(x, nw)
+    g, u = ((h @ w.astype(np.float64).T).astype(np.float32) for w in (wg, wu))
+    want = (g / (np.float32(1.0) + np.exp(-g))) * u
+    got = _run(gpu, dev, x, wg, nw, w_up=wu)
+    # exp may differ by an ulp between libraries: a few ulps of the product at most
+    assert np.all(np.abs(got - want) <= 8 * 2.0 ** -24 * np.abs(want) + 1e-30)
+
+
+@pytest.mark.parametrize("scale", [0.45, 0.5, 30.0, 127.0, 128.0, 60000.0])
+def test_weight_ranges(gpu, dev, tune, scale):
+    """Weights up to each digit count's limit and past it (f64 sums there), with fp16
+    subnormals among them, in one column block; the other block keeps three digits."""
+    tune(linear_tile=64)
+    rng = np.random.default_rng(int(scale * 10))
+    x = rng.standard_normal((40, 192), dtype=np.float32)
+    w = (rng.standard_normal((64, 192)) * 0.02).astype(np.float16)
+    w[:32] = (rng.uniform(-1, 1, (32, 192)) * scale).astype(np.float16)
+    w[3, :] = np.float16(scale)
+    w[5, ::2] = np.float16(2.0 ** -24)
+    w[6, ::3] = -np.float16(scale)
+    _check(_run(gpu, dev, x, w), (x.astype(np.float64) @ w.astype(np.float64).T).astype(np.float32))
+
+
+@pytest.mark.parametrize("spread", [1.0, 2.0 ** 10, 2.0 ** 15, 2.0 ** 21, 2.0 ** 40])
+def test_rows_with_outliers(gpu, dev, tune, spread):
+    """One element `spread` times the others: the digits hold every bit up to a spread of
+    2^14; past it every other element would reach the last digit and the row's block takes
+    f64 sums."""
+    tune(linear_tile=64)
+    rng = np.random.default_rng(11)
+    x = rng.uniform(0.5, 1.0, (64, 256)).astype(np.float32)
+    x[::5, 17] *= np.float32(spread)
+    w = (rng.standard_normal((48, 256)) * 0.02).astype(np.float16)
+    w[::2, 17] = 0  # columns that do not see the outlier keep the others' bits
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    got = _run(gpu, dev, x, w)
+    # f64 sums of 256 products: 2^-45 of the products' magnitudes at most, then one rounding
+    bound = 2.0 ** -24 * np.abs(want) + 2.0 ** -45 * (np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T)
+    assert np.all(np.abs(got - want) <= bound)
+
+
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan, 3e38, 1e-38])
+def test_unusual_rows(gpu, dev, tune, bad):
+    """Rows outside the digits' range give what f64 sums give, and leave the other rows' bits
+    alone (a block of 32 rows takes f64 sums together, in another order: 1 ulp)."""
+    tune(linear_tile=64)
+    rng = np.random.default_rng(13)
+    x = rng.standard_normal((70, 128), dtype=np.float32)
+    w = (rng.standard_normal((64, 128)) * 0.02).astype(np.float16)
+    x[5] *= 0 if abs(bad) < 1 else 1
+    x[5, 40] = bad
+    x[6] = 0
+    got = _run(gpu, dev, x, w)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = (x.astype(np.float64) @ w.astype(np.float64).T).astype(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    fine = np.isfinite(want)
+    assert np.array_equal(got[~fine & ~np.isnan(want)], want[~fine & ~np.isnan(want)])
+    d = _ulps(got[fine], want[fine])
+    assert d.max() <= 1
+    assert np.array_equal(got[32:64], _run(gpu, dev, x[32:64], w)), "another block changed"
+
+
+def test_workspace_is_checked(gpu, dev):
+    """A workspace below the size asked for is refused before any launch; a null one means the
+    plain product."""
+    from crucible_amd import _lib
+    lib = _lib.load()
+    rows, n, k = 2048, 768, 768
+    need = lib.crucible_linear_workspace_bytes(rows, n, k, 0, 0)
+    assert need > 0
+    assert lib.crucible_linear_workspace_bytes(16, n, k, 0, 0) == 0
+    x = torch.randn(rows, k, device=dev)
+    w = torch.randn(n, k, device=dev).mul_(0.02).half()
+    out = torch.zeros(rows, n, device=dev)
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    args = (x.data_ptr(), k, None, 1e-6, w.data_ptr(), n, k, None, out.data_ptr(), n, rows)
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.crucible_linear_f64acc_ws(*args, ws.data_ptr(), need - 1, stream) == _lib.ERR_WORKSPACE
+    assert lib.crucible_linear_f64acc_ws(*args, ws.data_ptr() + 8, need, stream) == _lib.ERR_INVALID
+    assert not out.any()
+    assert lib.crucible_linear_f64acc_ws(*args, None, 0, stream) == 0
+    plain = out.clone()
+    assert lib.crucible_linear_f64acc_ws(*args, ws.data_ptr(), need, stream) == 0
+    d = (out.view(torch.int32).long() - plain.view(torch.int32).long()).abs()
+    assert int(d.max()) <= 1 and int((d > 0).sum()) <= out.numel() // 20000
