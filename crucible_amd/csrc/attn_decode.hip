@@ -40,6 +40,7 @@
 // at a fixed place at its start).
 #include "common.hpp"
 #include "generic_attend.hpp"
+#include "hd_attend.hpp"
 
 #include <atomic>
 #include <cmath>
@@ -1121,6 +1122,276 @@ __global__ __launch_bounds__(kGenericThreads) void decode_generic_kernel(DecodeA
     });
 }
 
+// head_dim a multiple of 32 (hd_attend.hpp): a workgroup takes a split of 16 pages, a pair a wave at a time,
+// of one (request, kv head, block of 16 query heads), so each K/V byte is read once per
+// GQA group. With scratch for the partials the grid holds every split and
+// decode_hd_combine_kernel joins them; without (a.po null) a workgroup walks its unit's splits.
+// Both join the splits in the same order with the same steps, so they give the same bits.
+// A second kernel instead of decode_kernel's counters: the scratch needs no clearing, and
+// callers of these dimensions never had to clear or own one. HBM-bound at large batches,
+// latency-bound below; the split is small because one CU streams only 25-50 GB/s. 16 requests
+// of 64..2048 tokens, 12/3 heads of 128, fused append (26 MB): 70 us a layer in three launches
+// with attend_generic, 22.5 here, 13.5 of it in this kernel (traced) and 5 in the combine. Up to
+// 128 dims the registers are capped at 128, so that two workgroups share a CU (a few of the
+// f32-query form spill; uncapped it took 22 us against 19).
+constexpr int kHdSplitPages = 16;
+
+//
+// APPEND: the appended row (rotated when RoPE tables are given) goes from k_new / v_new into the
+// operands of every wave that reads its page, and one of them stores it, so the pools and the
+// outputs are those of the separate appends followed by the attention. Loading and storing it
+// apart from the page loads, in two more dependent round trips each, cost 5.5 us a launch.
+
+// Channels d .. d + N - 1 of the appended K row of request b, kv head g, as the append stores
+// them: N <= 8 channels of one half of the head.
+template <int HD, int N>
+__device__ __forceinline__ void hd_new_k(const DecodeArgs& a, int b, int g, int d, half_t (&out)[N]) {
+    const int64_t at = (int64_t)b * a.kv_new_stride + g * HD;
+    auto load = [&](int from, float (&x)[N]) {
+        if constexpr (N == 8) {  // 16-byte aligned (hd_decode_fits)
+            if (a.kv_new_f16) hd_load8<false>(a.k_new, at + from, x);
+            else hd_load8<true>(a.k_new, at + from, x);
+        } else {
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+                x[i] = a.kv_new_f16 ? (float)static_cast<const half_t*>(a.k_new)[at + from + i]
+                                    : static_cast<const float*>(a.k_new)[at + from + i];
+        }
+    };
+    float x[N];
+    load(d, x);
+    if (a.rope_cos) {
+        constexpr int kHalf = HD / 2;
+        const bool low = d < kHalf;
+        float y[N];
+        load(low ? d + kHalf : d - kHalf, y);
+        const int64_t t = (int64_t)min(max(a.positions[b], 0), a.rope_max_pos - 1) * kHalf + (low ? d : d - kHalf);
+        float c[N], sn[N];
+        if constexpr (N == 8) {
+            hd_load8<true>(a.rope_cos, t, c);
+            hd_load8<true>(a.rope_sin, t, sn);
+        } else {
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                c[i] = a.rope_cos[t + i];
+                sn[i] = a.rope_sin[t + i];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            float lo = low ? x[i] : y[i], hi = low ? y[i] : x[i];
+            rope_pair(lo, hi, c[i], sn[i]);
+            x[i] = low ? lo : hi;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) out[i] = (half_t)x[i];
+}
+
+template <int HD>
+__device__ __forceinline__ half_t hd_new_v(const DecodeArgs& a, int b, int g, int d) {
+    const int64_t at = (int64_t)b * a.kv_new_stride + g * HD + d;
+    return a.kv_new_f16 ? static_cast<const half_t*>(a.v_new)[at]
+                        : (half_t) static_cast<const float*>(a.v_new)[at];
+}
+
+template <int HD, bool QF32, bool APPEND, bool WHOLE>
+__global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 ? 4 : 1) void decode_hd_kernel(DecodeArgs a, int col_blocks) {
+    constexpr int W = hd_waves(HD);
+    __shared__ HdLds<HD, W, 1> lds;
+    const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = blockIdx.x / col_blocks;
+    const int c0 = (blockIdx.x - g * col_blocks) * 16;  // first query head of the group
+    const int b = blockIdx.y;
+    const int n_cols = min(16, a.n_rep - c0);
+    const uniform_i32_ptr table =
+        a.tables ? (uniform_i32_ptr)(a.tables + (int64_t)b * a.table_stride) : nullptr;
+    auto page_of = [&](int i) { return table ? (int64_t)table[min(i, a.max_pages - 1)] : (int64_t)i; };
+    const int s0 = WHOLE ? 0 : (int)blockIdx.z;
+    const int first = s0 * kHdSplitPages + 2 * wave;
+    int id0 = (int)page_of(first), id1 = (int)page_of(first + 1);
+    asm volatile("" : "+s"(id0), "+s"(id1));  // issued with the length's load, not behind its branch
+    int64_t page0 = id0, page1 = id1;
+    const int len = request_len(a, b);
+    const int apos = APPEND ? a.positions[b] : -1;
+    // The append of a position that is not attended (at or past the length). As
+    // crucible_cache_store_rows_paged: outside the table it is skipped and its entry not read;
+    // past the last split it belongs to that split.
+    auto append_only = [&]() {
+        const int ap = apos >> kPageShift;
+        if (!APPEND || apos < 0 || apos < len || ap >= a.table_stride || c0 != 0 ||
+            min(ap / kHdSplitPages, (int)gridDim.z - 1) != (int)blockIdx.z)
+            return;
+        const int64_t base = block_base(a.addr, (int64_t)table[ap]);
+        const int slot = apos & kPageMask;
+        for (int d = threadIdx.x; d < HD; d += 64 * W) {
+            half_t k[1];
+            hd_new_k<HD, 1>(a, b, g, d, k);
+            a.k_pool[base + (int64_t)slot * a.addr.kv_dim + g * HD + d] = k[0];
+            a.v_pool[base + (int64_t)(g * HD + d) * kPageTokens + slot] = hd_new_v<HD>(a, b, g, d);
+        }
+    };
+    const int n_pages = len > 0 ? (len + kPageMask) >> kPageShift : 0;
+    const int n_active = (n_pages + kHdSplitPages - 1) / kHdSplitPages;
+    if (s0 >= n_active) {  // past the end, or an inactive request: its output is untouched
+        append_only();
+        return;
+    }
+
+    // The first pages are requested before the queries are waited for.
+    HdPair<HD> kv;
+    auto load = [&](int p) {  // a page past the end re-reads the first one, its keys masked
+        if (p >= n_pages) return;
+        const int64_t base0 = block_base(a.addr, page0);
+        const int64_t base1 = block_base(a.addr, p + 1 < n_pages ? page1 : page0);
+        kv.load(a.k_pool, a.v_pool, base0, base1, a.addr.kv_dim, g * HD, col, grp);
+        if (!APPEND || apos >= len || (apos >> 1) >> kPageShift != p >> 1 || apos < 0) return;
+        // The appended row's page (uniform): every lane loads its share of the row beside the
+        // page loads; the lanes whose operand slots it fills take it and, once per kv head,
+        // store it.
+        const int slot = apos & kPageMask, pg = (apos >> kPageShift) & 1;
+        const int64_t base = pg ? base1 : base0;
+        half_t nk[HD / 32][8], nv[HD / 16];
+#pragma unroll
+        for (int k = 0; k < HD / 32; ++k) hd_new_k<HD, 8>(a, b, g, 32 * k + 8 * grp, nk[k]);
+#pragma unroll
+        for (int d = 0; d < HD / 16; ++d) nv[d] = hd_new_v<HD>(a, b, g, 16 * d + col);
+        const bool has_k = col == slot, has_v = grp == slot >> 2;
+#pragma unroll
+        for (int k = 0; k < HD / 32; ++k) {
+            half8_t row;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) row[e] = nk[k][e];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                if (has_k && pg == i) kv.k[i][k] = row;
+            if (has_k && c0 == 0)
+                *reinterpret_cast<half8_t*>(a.k_pool + base + (int64_t)slot * a.addr.kv_dim + g * HD +
+                                            32 * k + 8 * grp) = row;
+        }
+#pragma unroll
+        for (int d = 0; d < HD / 16; ++d) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (has_v && pg == i && (slot & 3) == r) kv.v[i][d][r] = nv[d];
+            if (has_v && c0 == 0)
+                a.v_pool[base + (int64_t)(g * HD + 16 * d + col) * kPageTokens + slot] = nv[d];
+        }
+    };
+    load(first);
+    __builtin_amdgcn_sched_barrier(0);
+    const int h = g * a.n_rep + c0 + min(col, n_cols - 1);
+    HdQuery<HD, QF32> q;
+    {
+        const int64_t qoff = (int64_t)b * a.q_row_stride + (int64_t)h * HD;
+        float x[HD / 32][8];
+#pragma unroll
+        for (int k = 0; k < HD / 32; ++k) {
+            const int d = 32 * k + 8 * grp;
+            hd_load8<QF32>(a.q, qoff + d, x[k]);
+            if (a.rope_cos) {  // pairs (i, i + HD / 2), both loaded by either side
+                constexpr int kHalf = HD / 2;
+                float y[8];
+                hd_load8<QF32>(a.q, qoff + (d < kHalf ? d + kHalf : d - kHalf), y);
+                const int pos = min(max(a.positions[b], 0), a.rope_max_pos - 1);
+                const int64_t t = (int64_t)pos * kHalf + (d < kHalf ? d : d - kHalf);
+                float c[8], sn[8];
+                hd_load8<true>(a.rope_cos, t, c);
+                hd_load8<true>(a.rope_sin, t, sn);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    float lo = d < kHalf ? x[k][i] : y[i], hi = d < kHalf ? y[i] : x[k][i];
+                    rope_pair(lo, hi, c[i], sn[i]);
+                    x[k][i] = d < kHalf ? lo : hi;
+                }
+            }
+        }
+        q.set(x, a.scale_log2);
+    }
+
+    HdState<HD> total, s[1];
+    for (int sp = s0;; ++sp) {
+        s[0].clear();
+#pragma unroll
+        for (int i = 0; i < kHdSplitPages / 2; i += W) {
+            const int p = sp * kHdSplitPages + 2 * (i + wave);
+            if ((WHOLE && sp > 0) || i > 0) {
+                page0 = page_of(p);
+                page1 = page_of(p + 1);
+                load(p);
+            }
+            if (p >= n_pages) break;
+            const int key0 = p * kPageTokens;
+            if (key0 + 2 * kPageTokens > len) kv.zero_tail(key0, len, grp);
+            hd_attend_pair(s[0], q, kv, key0, len - 1, grp);
+        }
+        hd_merge_waves<HD, W, 1>(lds, s, wave, col, grp, n_cols);
+        if constexpr (!WHOLE) break;
+        if (sp == 0) total = s[0];
+        else total.merge(s[0]);
+        if (sp + 1 == n_active) break;
+    }
+    append_only();
+    const int64_t out = (int64_t)b * a.out_row_stride + (int64_t)h * HD;
+    const bool mine = wave == 0 && col < n_cols;
+    if (WHOLE || n_active == 1) {
+        if (mine) hd_store(a.out, a.out_f16, out, WHOLE ? total : s[0], grp);
+    } else if (mine) {
+        const int64_t slot = ((int64_t)b * a.n_head + h) * a.n_splits + s0;
+#pragma unroll
+        for (int i = 0; i < HD / 16; ++i)
+            *reinterpret_cast<float4_t*>(a.po + slot * HD + 16 * i + 4 * grp) = s[0].o[i];
+        if (grp == 0) {
+            a.pm[slot] = s[0].m;
+            a.pl[slot] = s[0].l;
+        }
+    }
+}
+
+// Joins the splits' partials in order, one thread per (request, query head, 4 dims).
+__global__ __launch_bounds__(256) void decode_hd_combine_kernel(DecodeArgs a, int hd) {
+    const int quads = hd >> 2;
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (int64_t)a.batch * a.n_head * quads) return;
+    const int64_t row = i / quads;  // b * n_head + h
+    const int d = 4 * (int)(i - row * quads);
+    const int b = (int)(row / a.n_head);
+    const int64_t slot = row * a.n_splits;
+    // The first splits' partials are requested beside the length, whether or not it reaches
+    // them (those it does not are not used).
+    constexpr int kAhead = 8;  // splits a round trip
+    HdState<16> t[kAhead];
+    auto load = [&](int j0) {
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) {
+            const int64_t at = slot + min(j0 + j, a.n_splits - 1);
+            t[j].m = a.pm[at];
+            t[j].l = a.pl[at];
+            t[j].o[0] = *reinterpret_cast<const float4_t*>(a.po + at * hd + d);
+        }
+    };
+    load(0);
+    const int len = request_len(a, b);
+    if (len <= 0) return;
+    const int n_active = ((len + kPageMask) / kPageTokens + kHdSplitPages - 1) / kHdSplitPages;
+    if (n_active == 1) return;  // written by its only split
+    HdState<16> total;  // one quad of dims
+    for (int j0 = 0; j0 < n_active; j0 += kAhead) {
+        if (j0 > 0) load(j0);
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) {
+            if (j0 + j >= n_active) break;
+            if (j0 + j == 0) total = t[0];
+            else total.merge(t[j]);
+        }
+    }
+    store_out4(a, (int64_t)b * a.out_row_stride + (row - (int64_t)b * a.n_head) * hd + d,
+               total.o[0] * (1.0f / total.l));
+}
+
 // The qkv entry's two appends for head_dim other than 64: row b's K (rotated at
 // positions[b] when RoPE tables are given) and its V, f32 rows of stride kv_new_stride,
 // rounded to fp16 and stored at positions[b] as crucible_rope_split_qkv followed by
@@ -1355,14 +1626,75 @@ DecodeArgs common_args(const void* q, const void* k, const void* v, void* out, i
     return a;
 }
 
-// head_dim other than 64: decode_generic_kernel over (request, query head). Appends, where
-// the entry has them, are launched before it on the same stream.
-int launch_decode_generic(const DecodeArgs& a, int hd, bool q_f32, hipStream_t stream,
-                          const char* what) {
+// Whether decode_hd_kernel takes the call: its vector accesses need 16-byte rows, its grid
+// the counts below. Everything else stays with decode_generic_kernel.
+bool hd_decode_fits(const DecodeArgs& a, int hd, bool q_f32) {
+    return hd_mfma_ok(hd) && aligned16(a.q) && aligned16(a.out) && aligned16(a.rope_cos) &&
+           aligned16(a.rope_sin) &&
+           a.q_row_stride % (q_f32 ? 4 : 8) == 0 &&
+           (!a.positions || (aligned16(a.k_new) && a.kv_new_stride % (a.kv_new_f16 ? 8 : 4) == 0)) &&
+           a.batch <= 65535 && a.n_kv_head <= 65535 &&
+           a.max_pages <= kHdSplitPages * 65535;
+}
+
+template <int HD>
+void launch_decode_hd(const DecodeArgs& a, bool q_f32, hipStream_t stream) {
+    const int blocks = (a.n_rep + 15) / 16;
+    const dim3 grid((unsigned)(a.n_kv_head * blocks), (unsigned)a.batch,
+                    (unsigned)(a.po ? a.n_splits : 1));
+    auto go = [&](auto f32_tag, auto append_tag) {
+        constexpr bool kF32 = decltype(f32_tag)::value, kAppend = decltype(append_tag)::value;
+        if (a.po)
+            hipLaunchKernelGGL((decode_hd_kernel<HD, kF32, kAppend, false>), grid,
+                               dim3(64 * hd_waves(HD)), 0, stream, a, blocks);
+        else
+            hipLaunchKernelGGL((decode_hd_kernel<HD, kF32, kAppend, true>), grid,
+                               dim3(64 * hd_waves(HD)), 0, stream, a, blocks);
+    };
+    if (a.positions && q_f32) go(std::true_type{}, std::true_type{});
+    else if (a.positions) go(std::false_type{}, std::true_type{});
+    else if (q_f32) go(std::true_type{}, std::false_type{});
+    else go(std::false_type{}, std::false_type{});
+}
+
+// head_dim other than 64: decode_hd_kernel for multiples of 32, else decode_generic_kernel
+// over (request, query head). Appends, where the entry has them, are launched before it on
+// the same stream (decode_hd_kernel makes them itself). The workspace is optional scratch for the splits' partials, uncleared:
+// what crucible_attention_decode_workspace_bytes asks for holds them (its 4-page splits of
+// 64 + 2 floats and fixed region against 16-page splits of at most 256 + 2).
+int launch_decode_generic(DecodeArgs a, int hd, bool q_f32, void* workspace,
+                          size_t workspace_bytes, hipStream_t stream, const char* what) {
     CRUCIBLE_CHECK(a.n_head <= 65535, CRUCIBLE_ERR_INVALID, "%s: n_head %d too large", what,
                    a.n_head);
     CRUCIBLE_CHECK(aligned16(a.k_pool) && aligned16(a.v_pool), CRUCIBLE_ERR_INVALID,
                    "%s: pools must be 16-byte aligned", what);
+    if (hd_decode_fits(a, hd, q_f32)) {
+        a.po = nullptr;
+        a.n_splits = (a.max_pages + kHdSplitPages - 1) / kHdSplitPages;
+        const int64_t partials = checked_mul(a.batch, a.n_head, a.n_splits);
+        const int64_t bytes = checked_mul(partials, (hd + 2) * (int64_t)sizeof(float));
+        if (workspace && aligned16(workspace) && a.n_splits > 1 && bytes > 0 &&
+            partials * (hd / 4) <= (int64_t)INT32_MAX && (uint64_t)bytes <= workspace_bytes) {
+            a.po = static_cast<float*>(workspace);
+            a.pm = a.po + partials * hd;
+            a.pl = a.pm + partials;
+        }
+        switch (hd) {
+            case 32: launch_decode_hd<32>(a, q_f32, stream); break;
+            case 96: launch_decode_hd<96>(a, q_f32, stream); break;
+            case 128: launch_decode_hd<128>(a, q_f32, stream); break;
+            case 160: launch_decode_hd<160>(a, q_f32, stream); break;
+            case 192: launch_decode_hd<192>(a, q_f32, stream); break;
+            case 224: launch_decode_hd<224>(a, q_f32, stream); break;
+            default: launch_decode_hd<256>(a, q_f32, stream); break;
+        }
+        if (const int rc = fail_launch(what)) return rc;
+        if (!a.po) return CRUCIBLE_OK;
+        const int64_t threads = (int64_t)a.batch * a.n_head * (hd / 4);
+        hipLaunchKernelGGL(decode_hd_combine_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256),
+                           0, stream, a, hd);
+        return fail_launch(what);
+    }
     const dim3 grid((unsigned)a.batch, (unsigned)a.n_head);
     if (q_f32)
         hipLaunchKernelGGL(decode_generic_kernel<true>, grid, dim3(kGenericThreads), 0, stream, a, hd);
@@ -1525,7 +1857,8 @@ extern "C" int crucible_attention_decode_paged(
                    (long long)n_layer, (long long)kv_dim);
     a.table_stride = (int32_t)table_stride;
     if (head_dim != kHeadDim)
-        return launch_decode_generic(a, (int)head_dim, q_dtype == CRUCIBLE_F32, stream, what);
+        return launch_decode_generic(a, (int)head_dim, q_dtype == CRUCIBLE_F32, workspace, workspace_bytes,
+                                     stream, what);
     return decode_with_workspace(a, q_dtype == CRUCIBLE_F32, workspace, workspace_bytes, stream,
                                  what);
 }
@@ -1569,8 +1902,10 @@ extern "C" int crucible_attention_decode_paged_append(
                    (long long)n_layer, (long long)kv_dim);
     a.table_stride = (int32_t)table_stride;
     if (head_dim != kHeadDim) {
-        if (const int rc = append_rows_generic(a, kv_dtype, n_layer, layer, stream)) return rc;
-        return launch_decode_generic(a, (int)head_dim, q_dtype == CRUCIBLE_F32, stream, what);
+        if (!hd_decode_fits(a, (int)head_dim, q_dtype == CRUCIBLE_F32))
+            if (const int rc = append_rows_generic(a, kv_dtype, n_layer, layer, stream)) return rc;
+        return launch_decode_generic(a, (int)head_dim, q_dtype == CRUCIBLE_F32, workspace, workspace_bytes,
+                                     stream, what);
     }
     return decode_with_workspace(a, q_dtype == CRUCIBLE_F32, workspace, workspace_bytes, stream,
                                  what);
@@ -1615,8 +1950,10 @@ extern "C" int crucible_attention_decode_paged_append_noalloc(
                    (long long)n_layer, (long long)kv_dim);
     a.table_stride = (int32_t)table_stride;
     if (head_dim != kHeadDim) {  // the generic kernels use no scratch
-        if (const int rc = append_rows_generic(a, kv_dtype, n_layer, layer, stream)) return rc;
-        return launch_decode_generic(a, (int)head_dim, q_dtype == CRUCIBLE_F32, stream, what);
+        if (!hd_decode_fits(a, (int)head_dim, q_dtype == CRUCIBLE_F32))
+            if (const int rc = append_rows_generic(a, kv_dtype, n_layer, layer, stream)) return rc;
+        return launch_decode_generic(a, (int)head_dim, q_dtype == CRUCIBLE_F32, nullptr, 0,
+                                     stream, what);
     }
     CRUCIBLE_CHECK(aligned16(a.q) && aligned16(a.k_pool) && aligned16(a.v_pool) &&
                        aligned16(a.out) && aligned16(a.k_new) && aligned16(a.v_new),
@@ -1710,10 +2047,12 @@ extern "C" int crucible_attention_decode_qkv_paged_append(
         const int64_t threads = batch * n_kv_head * (head_dim / 2);
         CRUCIBLE_CHECK(threads <= (int64_t)INT32_MAX * 256, CRUCIBLE_ERR_INVALID, "%s: too many rows",
                        what);
-        hipLaunchKernelGGL(append_rope_generic_kernel, dim3((unsigned)((threads + 255) / 256)),
-                           dim3(256), 0, stream, a, (int)head_dim);
-        if (const int rc = fail_launch(what)) return rc;
-        return launch_decode_generic(a, (int)head_dim, true, stream, what);
+        if (!hd_decode_fits(a, (int)head_dim, true)) {
+            hipLaunchKernelGGL(append_rope_generic_kernel, dim3((unsigned)((threads + 255) / 256)),
+                               dim3(256), 0, stream, a, (int)head_dim);
+            if (const int rc = fail_launch(what)) return rc;
+        }
+        return launch_decode_generic(a, (int)head_dim, true, workspace, workspace_bytes, stream, what);
     }
     return decode_with_workspace(a, true, workspace, workspace_bytes, stream, what);
 }
@@ -1781,7 +2120,8 @@ extern "C" int crucible_attention_decode(const void* q, int q_dtype, const void*
     a.addr.page_stride = kPageTokens * cache_stride;
     a.addr.layer_off = layer_base;
     if (head_dim != kHeadDim)
-        return launch_decode_generic(a, (int)head_dim, q_dtype == CRUCIBLE_F32, stream, what);
+        return launch_decode_generic(a, (int)head_dim, q_dtype == CRUCIBLE_F32, workspace, workspace_bytes,
+                                     stream, what);
     return decode_with_workspace(a, q_dtype == CRUCIBLE_F32, workspace, workspace_bytes, stream,
                                  what);
 }
@@ -1814,7 +2154,8 @@ extern "C" int crucible_attention_split(const void* q, int q_dtype, const void* 
     // head_dim other than 64: the generic kernel writes the output in one pass (the partial
     // buffers are left as they are)
     if (head_dim != kHeadDim)
-        return launch_decode_generic(a, (int)head_dim, q_dtype == CRUCIBLE_F32, stream, what);
+        return launch_decode_generic(a, (int)head_dim, q_dtype == CRUCIBLE_F32, nullptr, 0,
+                                     stream, what);
     // 128-position chunks as in the reference (gpu.rs:37 ATTN_CHUNK): 4 waves x 2 pages,
     // partials in the caller's buffers, combined by a second kernel.
     const DecodeShape sh{2, 4};

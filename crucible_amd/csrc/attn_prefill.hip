@@ -38,6 +38,7 @@
 // makes two passes, each masking the rows of the other request.
 #include "common.hpp"
 #include "generic_attend.hpp"
+#include "hd_attend.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -1734,6 +1735,129 @@ __global__ __launch_bounds__(kGenericThreads) void prefill_generic_kernel(Prefil
     }
 }
 
+// head_dim a multiple of 32 (hd_attend.hpp): a workgroup takes 16 QB query rows of one head; its W
+// waves take every W-th pair of pages of the rows' key range and merge at the end. K and V
+// stream from L2 once per 16 QB rows (attend_generic reads them once a row), so 32 rows a
+// workgroup where the registers hold them, and 4 waves, whose 512 registers a lane do: prompts
+// of 1000, 333, 777 and 64 tokens, 12/3 heads of 128, 41.8 us (8 waves of 32 rows spill: 59.9;
+// 8 waves of 16 rows 59.0; attend_generic 820). Later row tiles,
+// whose key ranges are longer, are dispatched first.
+//
+// An OWNERS tile may hold rows of several requests: each owner's rows are attended, merged and
+// stored on their own, so no value of one request reaches another's rows.
+template <int HD, int W, int QB, bool QF32, bool HYB>
+__global__ __launch_bounds__(64 * W) void prefill_hd_kernel(PrefillArgs a) {
+    __shared__ HdLds<HD, W, QB> lds;
+    const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int h = blockIdx.x;
+    const int64_t tile = (int64_t)gridDim.y - 1 - blockIdx.y;
+    const int64_t stride = (int64_t)a.n_head * HD;
+    int row[QB], owner[QB], pos[QB];
+    bool pending[QB];
+    HdQuery<HD, QF32> q[QB];
+    bool any = false;
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+        tile_row(a, blockIdx.z, tile * (16 * QB) + 16 * b + col, row[b], owner[b], pos[b]);
+        pending[b] = row[b] >= 0;
+        any |= pending[b];
+    }
+    if (__ballot(any) == 0) return;  // the same rows in every wave
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+        float x[HD / 32][8];
+        const int64_t off = (int64_t)max(row[b], 0) * stride + (int64_t)h * HD + 8 * grp;
+#pragma unroll
+        for (int k = 0; k < HD / 32; ++k) hd_load8<QF32>(a.q, off + 32 * k, x[k]);
+        q[b].set(x, a.scale_log2);
+    }
+    const int head_off = (h / a.n_rep) * HD;
+    for (;;) {
+        // the first pending row's owner, the rows that share it, and their last position
+        int who = 0, last = -1;
+        bool found = false;
+#pragma unroll
+        for (int b = 0; b < QB; ++b) {
+            const uint64_t mask = __ballot(pending[b]);
+            if (!found && mask) {
+                who = __builtin_amdgcn_readlane(owner[b], __builtin_ctzll(mask));
+                found = true;
+            }
+        }
+        if (!found) return;
+        int see[QB];  // last key the column sees
+#pragma unroll
+        for (int b = 0; b < QB; ++b) {
+            const bool mine = pending[b] && owner[b] == who;
+            see[b] = mine ? pos[b] : -1;
+            pending[b] = pending[b] && !mine;
+            last = max(last, see[b]);
+        }
+#pragma unroll
+        for (int off = 1; off < 16; off <<= 1) last = max(last, __shfl_xor(last, off));
+        last = __builtin_amdgcn_readfirstlane(last);
+
+        const uniform_i32_ptr table =
+            a.tables ? (uniform_i32_ptr)(a.tables + (int64_t)who * a.table_stride) : nullptr;
+        const int n_pages = (last >> kPageShift) + 1;
+        // Hybrid: keys from the segment's absolute start on are the chunk's own rows, and a page
+        // that holds only such keys has neither its table entry nor its pool block read; the
+        // first page stands in for it (or, with no history at all, nothing is loaded).
+        const int astart = HYB ? a.segments[4 * blockIdx.z + 2] : INT32_MAX;
+        const int row0 = HYB ? a.segments[4 * blockIdx.z] : 0;
+        const int pool_pages = HYB ? min(n_pages, (astart + kPageMask) >> kPageShift) : n_pages;
+        auto page_of = [&](int i) {  // past the end: the last page, its keys masked
+            if (HYB && pool_pages == 0) return (int64_t)0;
+            i = min(i, pool_pages - 1);
+            return table ? (int64_t)table[i] : (int64_t)i;
+        };
+        HdState<HD> s[QB];
+#pragma unroll
+        for (int b = 0; b < QB; ++b) s[b].clear();
+        int64_t page0 = page_of(2 * wave), page1 = page_of(2 * wave + 1);
+        for (int p = 2 * wave; p < n_pages; p += 2 * W) {
+            HdPair<HD> kv;
+            if (!HYB || p < pool_pages)
+                kv.load(a.k_pool, a.v_pool, block_base(a.addr, page0), block_base(a.addr, page1),
+                        a.addr.kv_dim, head_off, col, grp);
+            if constexpr (HYB)
+                kv.load_rows(a.cur_k, a.cur_v, row0, astart, last, p * kPageTokens, a.addr.kv_dim,
+                             head_off, col, grp);
+            page0 = page_of(p + 2 * W);  // beside the K/V loads, not before the next ones
+            page1 = page_of(p + 2 * W + 1);
+            const int key0 = p * kPageTokens;
+            if (key0 + 2 * kPageTokens > last + 1) kv.zero_tail(key0, last + 1, grp);
+#pragma unroll
+            for (int b = 0; b < QB; ++b) hd_attend_pair(s[b], q[b], kv, key0, see[b], grp);
+        }
+        hd_merge_waves<HD, W, QB>(lds, s, wave, col, grp, 16 * QB);
+        if (wave == 0)
+#pragma unroll
+            for (int b = 0; b < QB; ++b)
+                if (see[b] >= 0)
+                    hd_store(a.out, a.out_f16, (int64_t)row[b] * stride + (int64_t)h * HD, s[b], grp);
+    }
+}
+
+template <int HD, int W, int QB>
+void launch_prefill_hd(const PrefillArgs& a, int64_t rows, int64_t z, bool q_f32, hipStream_t stream) {
+    auto go = [&](auto qb_tag, auto f32_tag, auto hyb_tag) {
+        constexpr int kQB = decltype(qb_tag)::value;
+        const dim3 grid((unsigned)a.n_head, (unsigned)((rows + 16 * kQB - 1) / (16 * kQB)), (unsigned)z);
+        hipLaunchKernelGGL((prefill_hd_kernel<HD, W, kQB, decltype(f32_tag)::value, decltype(hyb_tag)::value>),
+                           grid, dim3(64 * W), 0, stream, a);
+    };
+    // a column's arithmetic does not depend on its neighbours, so hybrid segments, with 16
+    // rows a workgroup, give the pool form's bits
+    using one = std::integral_constant<int, 1>;
+    using qb = std::integral_constant<int, QB>;
+    if (a.hybrid && q_f32) go(one{}, std::true_type{}, std::true_type{});
+    else if (a.hybrid) go(one{}, std::false_type{}, std::true_type{});
+    else if (q_f32) go(qb{}, std::true_type{}, std::false_type{});
+    else go(qb{}, std::false_type{}, std::false_type{});
+}
+
 int launch_prefill_generic(PrefillArgs a, int hd, int64_t tile_rows_total, int64_t z, bool q_f32,
                            hipStream_t stream, const char* what) {
     CRUCIBLE_CHECK(a.n_head <= INT32_MAX && z <= 65535, CRUCIBLE_ERR_INVALID,
@@ -1741,6 +1865,21 @@ int launch_prefill_generic(PrefillArgs a, int hd, int64_t tile_rows_total, int64
     CRUCIBLE_CHECK(((uintptr_t)a.k_pool & 15) == 0 && ((uintptr_t)a.v_pool & 15) == 0,
                    CRUCIBLE_ERR_INVALID, "%s: pools must be 16-byte aligned", what);
     a.scale_log2 = (float)(1.4426950408889634 / std::sqrt((double)hd));
+    // prefill_hd_kernel where its vector accesses and grid allow; every other head_dim stays
+    // with prefill_generic_kernel
+    if (hd_mfma_ok(hd) && ((uintptr_t)a.q & 15) == 0 && ((uintptr_t)a.out & 15) == 0 &&
+        tile_rows_total <= 16 * 65535) {
+        switch (hd) {
+            case 32: launch_prefill_hd<32, 8, 2>(a, tile_rows_total, z, q_f32, stream); break;
+            case 96: launch_prefill_hd<96, 4, 2>(a, tile_rows_total, z, q_f32, stream); break;
+            case 128: launch_prefill_hd<128, 4, 2>(a, tile_rows_total, z, q_f32, stream); break;
+            case 160: launch_prefill_hd<160, 4, 1>(a, tile_rows_total, z, q_f32, stream); break;
+            case 192: launch_prefill_hd<192, 4, 1>(a, tile_rows_total, z, q_f32, stream); break;
+            case 224: launch_prefill_hd<224, 4, 1>(a, tile_rows_total, z, q_f32, stream); break;
+            default: launch_prefill_hd<256, 4, 1>(a, tile_rows_total, z, q_f32, stream); break;
+        }
+        return fail_launch(what);
+    }
     const dim3 grid((unsigned)a.n_head, (unsigned)std::min<int64_t>(tile_rows_total, 65535),
                     (unsigned)z);
     if (q_f32)

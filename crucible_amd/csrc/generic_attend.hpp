@@ -2,8 +2,9 @@
 //
 // The reference kernels take any head_dim (kernels.cu:1741-1756, 2100-2276: loops over d in
 // steps of the warp). The MFMA kernels of attn_decode.hip / attn_prefill.hip are built for
-// head_dim 64, the dimension of every preset. Other dimensions (a multiple of 8 up to 256)
-// run through this workgroup-level routine instead: plain wave64 code, f32 accumulation,
+// head_dim 64, the dimension of every preset; hd_attend.hpp has those of the other multiples of
+// 32. The remaining dimensions (multiples of 8 up to 256), and calls whose buffers are not
+// 16-byte aligned, run through this workgroup-level routine instead: plain wave64 code, f32 accumulation,
 // fp16 K/V read from the same pool layout, online softmax in base 2.
 //
 // One workgroup of kGenericThreads threads attends one (query row, query head) over keys

@@ -152,6 +152,15 @@ class Gpu:
         graph) can take it, so calls on several streams and threads never share one."""
         return torch.empty(nbytes, dtype=torch.uint8, device=self.device)
 
+    def _decode_scratch(self, workspace, batch, n_head, head_dim, max_seq, pools=None):
+        """The workspace of a decode call: the caller's or the cached one for head_dim 64. The
+        other dimensions keep nothing between calls and never needed calls to be ordered, so
+        theirs is scratch of the call's own."""
+        if head_dim != 64:
+            return self._scratch(max(16, self.lib.crucible_attention_decode_workspace_bytes(
+                batch, n_head, max_seq)))
+        return workspace if workspace is not None else self.workspace(batch, n_head, max_seq, pools)
+
     @staticmethod
     def version() -> str:
         return _lib.load().crucible_attn_version().decode()
@@ -210,8 +219,7 @@ class Gpu:
         _need(v_pool, "v_pool", dtype=torch.float16)
         _need(page_tables, "page_tables", dtype=torch.int32, numel=batch * table_stride)
         _need(seq_lens, "seq_lens", dtype=torch.int32, numel=batch)
-        ws = workspace if workspace is not None else self.workspace(batch, n_head, max_seq,
-                                                                   (k_pool, v_pool))
+        ws = self._decode_scratch(workspace, batch, n_head, head_dim, max_seq, (k_pool, v_pool))
         _need(ws, "workspace")
         _lib.check(self.lib.crucible_attention_decode_paged(
             _ptr(q), _dtype(q, "q"), _ptr(k_pool), _ptr(v_pool), _ptr(out), _dtype(out, "out"),
@@ -234,8 +242,7 @@ class Gpu:
         _need(page_tables, "page_tables", dtype=torch.int32, numel=batch * table_stride)
         _need(positions, "positions", dtype=torch.int32, numel=batch)
         _need(seq_lens, "seq_lens", dtype=torch.int32, numel=batch)
-        ws = workspace if workspace is not None else self.workspace(batch, n_head, max_seq,
-                                                                   (k_pool, v_pool))
+        ws = self._decode_scratch(workspace, batch, n_head, head_dim, max_seq, (k_pool, v_pool))
         _lib.check(self.lib.crucible_attention_decode_paged_append(
             _ptr(q), _dtype(q, "q"), _ptr(k_new), _ptr(v_new), _dtype(k_new, "k_new"),
             _ptr(k_pool), _ptr(v_pool), _ptr(out), _dtype(out, "out"), _ptr(page_tables),
@@ -263,8 +270,7 @@ class Gpu:
             _need(rope_cos, "rope_cos", dtype=torch.float32)
             _need(rope_sin, "rope_sin", dtype=torch.float32, numel=rope_cos.numel())
             max_pos = rope_cos.shape[0]
-        ws = workspace if workspace is not None else self.workspace(batch, n_head, max_seq,
-                                                                   (k_pool, v_pool))
+        ws = self._decode_scratch(workspace, batch, n_head, head_dim, max_seq, (k_pool, v_pool))
         _lib.check(self.lib.crucible_attention_decode_qkv_paged_append(
             _ptr(qkv), row_stride, _ptr(rope_cos), _ptr(rope_sin), max_pos, _ptr(k_pool),
             _ptr(v_pool), _ptr(out), _dtype(out, "out"), _ptr(page_tables), _ptr(positions),
@@ -279,7 +285,7 @@ class Gpu:
         _need(k_cache, "k_cache", dtype=torch.float16)
         _need(v_cache, "v_cache", dtype=torch.float16)
         _need(params, "params", dtype=torch.int32, numel=6)
-        ws = workspace if workspace is not None else self.workspace(1, n_head, max_seq)
+        ws = self._decode_scratch(workspace, 1, n_head, head_dim, max_seq)
         _lib.check(self.lib.crucible_attention_decode(
             _ptr(q), _dtype(q, "q"), _ptr(k_cache), _ptr(v_cache), _ptr(out), _dtype(out, "out"),
             n_head, n_kv_head, head_dim, _ptr(params), max_seq, cache_stride, layer_base,

@@ -149,12 +149,16 @@ int crucible_cache_store_packed_paged(const void* src, int src_dtype, void* pool
  * q is [batch][n_head * head_dim] (q_dtype), out is [batch][n_head * head_dim]
  * (out_dtype). n_head is a multiple of n_kv_head; query head h reads KV head
  * h / (n_head / n_kv_head). head_dim 64 (every preset) runs the MFMA kernels, with
- * n_head / n_kv_head <= 16. Any other head_dim that is a multiple of 8 up to 256 runs a
- * generic kernel (one workgroup per request and query head, f32 arithmetic, same pool
- * layout and the same results to the tolerance of f32 accumulation); it uses no
- * workspace, the fused entries run their appends as two cache_store_rows_paged launches
- * (RoPE rows: one append launch) before it, and attention_split leaves its partial
- * buffers untouched. The same holds for the prefill entries below.
+ * n_head / n_kv_head <= 16. Any other multiple of 32 up to 256 runs MFMA kernels of its own
+ * when q, out, the new rows and the RoPE tables are 16-byte aligned (and rows of q and of the
+ * new keys start there): splits of 16 pages, joined by a second launch when the call brings a
+ * workspace (used as plain scratch: it needs no clearing and nothing is kept in it) and by the
+ * same workgroup, with the same bits, when it does not. The remaining multiples of 8, and
+ * unaligned buffers, run a generic kernel (one workgroup per request and query head, f32
+ * arithmetic, no workspace). For every head_dim other than 64 the pool layout and the results
+ * are the same to the tolerance of f32 accumulation, the fused entries write the bytes of the
+ * separate appends, and attention_split leaves its partial buffers untouched. The same holds
+ * for the prefill entries below.
  * The split-K partials live in a caller-provided workspace of at least
  * crucible_attention_decode_workspace_bytes(...) bytes (no allocation here; 0 for an
  * empty batch, SIZE_MAX for a shape past the entry points' limits), 16-byte aligned.

@@ -1,0 +1,139 @@
+"""The MFMA attention of head dimensions that are multiples of 32 (hd_attend.hpp) against the
+one-row generic kernels, which take the same calls when a buffer is not 16-byte aligned.
+
+Both compute the same attention over the same fp16 pages; they differ in the order of f32 sums
+and in carrying P (and an f32 query) as fp16 hi + lo, about 2^-22 of each: outputs of N(0,1)
+values agree to 1e-5. Sizes sit at the edges: one key, one page, either side of a 16-page split
+and of a 32-row tile, more than 16 query heads a group, every dimension.
+"""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5
+
+
+def _unaligned(t):
+    """The same values one element into a larger buffer."""
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    out = flat[1:].view(t.shape)
+    out.copy_(t)
+    return out
+
+
+def _case(dev, seed, hd, n_head, n_kv, lens, n_layer=2, dtype=torch.float32):
+    g = torch.Generator(device=dev)
+    g.manual_seed(seed)
+    stride = max(-(-max(max(lens), 1) // 16), 1) + 1
+    n_pages = len(lens) * stride + 3
+    kv = n_kv * hd
+    pools = [torch.randn(n_pages * n_layer * 16 * kv, generator=g, device=dev).half() for _ in "kv"]
+    perm = torch.randperm(n_pages, generator=g, device=dev)[:len(lens) * stride]
+    tables = perm.view(len(lens), stride).int().contiguous()
+    q = torch.randn(len(lens), n_head * hd, generator=g, device=dev).to(dtype)
+    return g, stride, kv, pools, tables, q
+
+
+@pytest.mark.parametrize("hd,n_head,n_kv", [(32, 4, 4), (32, 24, 1), (96, 12, 3), (128, 40, 2),
+                                            (160, 6, 2), (192, 4, 1), (224, 2, 2), (256, 8, 2)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_decode_against_generic(gpu, dev, hd, n_head, n_kv, dtype):
+    lens = [1, 15, 16, 17, 255, 256, 257, 0, 600]
+    b, layer = len(lens), 1
+    g, stride, kv, (kp, vp), tables, q = _case(dev, hd + n_head, hd, n_head, n_kv, lens, dtype=dtype)
+    d_len = torch.tensor(lens, dtype=torch.int32, device=dev)
+
+    def run(q, k, v):
+        out = torch.full((b, n_head * hd), 7.0, device=dev)
+        gpu.attention_decode_paged(q, k, v, out, tables, d_len, b, n_head, n_kv, hd, stride, 2,
+                                   layer, kv, stride * 16)
+        return out
+
+    got, want = run(q, kp, vp), run(_unaligned(q), kp, vp)
+    assert torch.all(got[7] == 7.0), "an inactive request's output was written"
+    assert float((got - want).abs().max()) <= TOL
+    # without scratch one workgroup walks the splits: the same bits
+    from crucible_amd import _lib
+    lib = _lib.load()
+    alone = torch.full_like(got, 7.0)
+    _lib.check(lib.crucible_attention_decode_paged(
+        q.data_ptr(), 0 if dtype == torch.float32 else 1, kp.data_ptr(), vp.data_ptr(),
+        alone.data_ptr(), 0, tables.data_ptr(), d_len.data_ptr(), b, n_head, n_kv, hd, stride, 2,
+        layer, kv, stride * 16, None, 0, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(alone, got)
+
+
+@pytest.mark.parametrize("hd,n_head,n_kv", [(32, 24, 1), (96, 12, 3), (128, 12, 3), (256, 4, 2)])
+@pytest.mark.parametrize("kv_dtype", [torch.float32, torch.float16])
+def test_append_against_separate_calls(gpu, dev, hd, n_head, n_kv, kv_dtype):
+    """Positions inside the attended keys, just past them, in a page the length does not reach,
+    in the table's last page and outside it; inactive requests append too."""
+    lens = [1, 16, 17, 300, 40, 0, 260, 30]
+    pos = [0, 15, 16, 299, 40, 3, 16 * 19 - 1, 10 ** 6]
+    b, layer = len(lens), 0
+    g, stride, kv, (kp, vp), tables, q = _case(dev, hd, hd, n_head, n_kv, lens)
+    assert stride == 20
+    d_len = torch.tensor(lens, dtype=torch.int32, device=dev)
+    d_pos = torch.tensor(pos, dtype=torch.int32, device=dev)
+    new = [torch.randn(b, kv, generator=g, device=dev).to(kv_dtype) for _ in "kv"]
+    k1, v1, k2, v2 = kp.clone(), vp.clone(), kp.clone(), vp.clone()
+    o1 = torch.full((b, n_head * hd), 7.0, device=dev)
+    o2 = o1.clone()
+    gpu.attention_decode_paged_append(q, new[0], new[1], k1, v1, o1, tables, d_pos, d_len, b, n_head,
+                                      n_kv, hd, stride, 2, layer, kv, 300)
+    for src, pool, kind in ((new[0], k2, "k"), (new[1], v2, "v")):
+        gpu.cache_store_rows_paged(src, pool, tables, d_pos, b, kv, stride, 2, layer, kind=kind)
+    gpu.attention_decode_paged(q, k2, v2, o2, tables, d_len, b, n_head, n_kv, hd, stride, 2, layer,
+                               kv, 300)
+    assert torch.equal(k1, k2) and torch.equal(v1, v2)
+    assert torch.equal(o1, o2)
+
+
+@pytest.mark.parametrize("hd", [32, 96, 128, 160, 256])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_prefill_against_generic(gpu, dev, hd, dtype):
+    lens = [1, 16, 31, 32, 33, 65, 300]
+    n_head, n_kv, layer = 4, 2, 1
+    g, stride, kv, (kp, vp), tables, _ = _case(dev, hd, hd, n_head, n_kv, lens)
+    owners = np.repeat(np.arange(len(lens), dtype=np.int32), lens)
+    positions = np.concatenate([np.arange(n, dtype=np.int32) for n in lens])
+    rows = len(owners)
+    q = torch.randn(rows, n_head * hd, generator=g, device=dev).to(dtype)
+    d_own, d_pos = (torch.from_numpy(a).to(dev) for a in (owners, positions))
+
+    def run(q, v):
+        out = torch.full((rows, n_head * hd), 7.0, device=dev)
+        gpu.attention_prefill_packed(q, kp, v, out, tables, d_own, d_pos, rows, stride, n_head, n_kv,
+                                     hd, 2, layer, kv, stride * 16)
+        return out
+
+    got = run(q, vp)
+    assert float((got - run(_unaligned(q), vp)).abs().max()) <= TOL
+    # packed tiles hold rows of several requests: one request's NaN stays its own
+    bad = vp.clone().view(-1, 2, kv, 16)
+    bad[tables[2, :1].long(), layer] = float("nan")
+    touched = torch.from_numpy(owners == 2).to(dev)
+    other = run(q, bad.view(-1))
+    assert torch.equal(other[~touched], got[~touched])
+    assert torch.all(torch.isnan(other[touched]))
+
+
+def test_large_and_tiny_f32_queries(gpu, dev):
+    """f32 queries outside fp16's range: the operands are scaled by a power of two."""
+    hd, n_head, n_kv, lens = 128, 4, 2, [70, 33]
+    g, stride, kv, (kp, vp), tables, q = _case(dev, 5, hd, n_head, n_kv, lens)
+    d_len = torch.tensor(lens, dtype=torch.int32, device=dev)
+    for factor in (2.0 ** -60, 1e-6, 1e5):
+        kp2 = (kp.float() * min(1.0, 1.0 / factor)).half() if factor > 1 else kp
+        qq = (q * factor).contiguous()
+        outs = []
+        for x in (qq, _unaligned(qq)):
+            out = torch.zeros(2, n_head * hd, device=dev)
+            gpu.attention_decode_paged(x, kp2, vp, out, tables, d_len, 2, n_head, n_kv, hd, stride, 2,
+                                       0, kv, stride * 16)
+            outs.append(out)
+        assert torch.isfinite(outs[0]).all()
+        # scores of 1e5 x 1e-5 products keep 2^-22 of their magnitude (about 11): 1e-4 of weight
+        assert float((outs[0] - outs[1]).abs().max()) <= (1e-4 if factor > 1 else TOL)
