@@ -122,6 +122,9 @@ class Gpu:
 
     # ------------------------------------------------------------- plumbing
     def _stream(self) -> int:
+        # the raw handle, without building a Stream object, for a device known by its index
+        if self.device.index is not None:
+            return torch._C._cuda_getCurrentRawStream(self.device.index)
         return torch.cuda.current_stream(self.device).cuda_stream
 
     def workspace(self, batch: int, n_head: int, max_seq: int, pools=None) -> torch.Tensor:
