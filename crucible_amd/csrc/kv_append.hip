@@ -32,13 +32,28 @@ struct AppendArgs {
     int mode;
 };
 
+// K threads walk a row's channels, so a wave stores whole rows. V threads (a.v_kind) walk 16
+// rows of one channel group first: consecutive positions share a page, whose channel rows are
+// 16 slots of 2 bytes, so the lanes of one store instruction fill 32-byte runs (4,713 rows of
+// 192 channels, K and V: 5.8 us each with the K order).
 template <int VEC>
 __global__ __launch_bounds__(256) void kv_append_kernel(AppendArgs a) {
-    const int64_t per_row = a.addr.kv_dim / VEC;
+    const uint32_t per_row = (uint32_t)(a.addr.kv_dim / VEC);
+    // launch_append keeps the blocks below 2^31, not the threads: one 64-bit step, then 32-bit
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= a.rows * per_row) return;
-    const int64_t row = i / per_row;
-    const int c0 = (int)(i - row * per_row) * VEC;
+    int64_t row;
+    uint32_t group;
+    if (a.v_kind) {
+        const int64_t n = i >> 4;
+        const int64_t block = n <= UINT32_MAX ? (int64_t)((uint32_t)n / per_row) : n / per_row;
+        row = block * 16 + (i & 15);
+        group = (uint32_t)(n - block * per_row);
+    } else {
+        row = i <= UINT32_MAX ? (int64_t)((uint32_t)i / per_row) : i / per_row;
+        group = (uint32_t)(i - row * per_row);
+    }
+    if (row >= a.rows) return;
+    const int c0 = (int)group * VEC;
 
     int64_t pos;
     int64_t page;
@@ -99,7 +114,9 @@ __global__ __launch_bounds__(256) void kv_append_kernel(AppendArgs a) {
 int launch_append(AppendArgs a, hipStream_t stream, const char* what) {
     if (a.rows == 0) return CRUCIBLE_OK;
     const bool vec = (a.addr.kv_dim % 8) == 0;
-    const int64_t threads = a.rows * (vec ? a.addr.kv_dim / 8 : a.addr.kv_dim);
+    // V: whole groups of 16 rows
+    const int64_t rows = a.v_kind ? (a.rows + 15) / 16 * 16 : a.rows;
+    const int64_t threads = rows * (vec ? a.addr.kv_dim / 8 : a.addr.kv_dim);
     const int64_t blocks = (threads + 255) / 256;
     CRUCIBLE_CHECK(blocks <= INT32_MAX, CRUCIBLE_ERR_INVALID, "%s: too many rows", what);
     if (vec)

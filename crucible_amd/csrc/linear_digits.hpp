@@ -327,7 +327,8 @@ constexpr int kStage = kStageX + 2 * 2 * 3 * kFrag;  // 2 column blocks x 2 step
 // With every SIMD busy on random digits the part runs a 32x32x32 product in 20 ns (13.7 with
 // a few CUs busy): 150 us for the gate/up product of 4,713 rows (252 G multiply-adds).
 // Measured slower: steps of 32 in a ring of 4 (2 workgroups a CU) or 8 buffers, operands
-// double-buffered in registers, and 32 x 64 outputs a wave (one wave a SIMD, 512 VGPRs).
+// double-buffered in registers, 32 x 64 outputs a wave (one wave a SIMD, 512 VGPRs), and, for
+// grids below the CU count, a second set of 4 waves on every other stage of K.
 //
 // int8 MFMA 32x32x32: lane l supplies row (column) l & 31 and 16 of the step's 32 keys, the
 // half l >> 5 of them (the same keys for both operands), and holds

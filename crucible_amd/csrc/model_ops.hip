@@ -957,6 +957,49 @@ __global__ void rope_split_kernel(const float* __restrict__ qkv, int64_t ld, flo
     dst[i + half] = lo * s + hi * c;
 }
 
+// The same for head_dim a multiple of 8 and 16-byte rows: 4 pairs a thread in 16-byte accesses
+// and one 32-bit division (the scalar form's two 64-bit ones and 4-byte accesses took 14 us for
+// 4,713 rows of 12 + 2 x 3 heads, 43 MB).
+__global__ __launch_bounds__(256) void rope_split4_kernel(
+    const float* __restrict__ qkv, int64_t ld, float* q, float* k, float* v,
+    const float* __restrict__ cos_t, const float* __restrict__ sin_t,
+    const int32_t* __restrict__ positions, int rows, int n_head, int n_kv_head, int head_dim,
+    int max_pos) {
+    const int half = head_dim >> 1;
+    const uint32_t quads = (uint32_t)half >> 2;                     // a head
+    const uint32_t per_row = (uint32_t)(n_head + 2 * n_kv_head) * quads;
+    const uint32_t at = blockIdx.x * 256 + threadIdx.x;             // of the row
+    const int row = blockIdx.y;
+    if (at >= per_row) return;
+    const int head = (int)(at / quads);
+    const int i = 4 * (int)(at - (uint32_t)head * quads);
+    const float* src = qkv + (int64_t)row * ld + (int64_t)head * head_dim + i;
+    const float4_t lo = *reinterpret_cast<const float4_t*>(src);
+    const float4_t hi = *reinterpret_cast<const float4_t*>(src + half);
+    float* dst;
+    if (head < n_head) dst = q + ((int64_t)row * n_head + head) * head_dim;
+    else if (head < n_head + n_kv_head) dst = k + ((int64_t)row * n_kv_head + head - n_head) * head_dim;
+    else dst = v + ((int64_t)row * n_kv_head + head - n_head - n_kv_head) * head_dim;
+    float4_t a = lo, b = hi;
+    if (head < n_head + n_kv_head) {
+        const int pos = positions[row];
+        if (pos < 0 || pos >= max_pos) {
+            const float nan = __builtin_nanf("");
+            a = b = float4_t{nan, nan, nan, nan};
+        } else {
+            const float4_t c = *reinterpret_cast<const float4_t*>(cos_t + (int64_t)pos * half + i);
+            const float4_t s = *reinterpret_cast<const float4_t*>(sin_t + (int64_t)pos * half + i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                a[e] = lo[e] * c[e] - hi[e] * s[e];
+                b[e] = lo[e] * s[e] + hi[e] * c[e];
+            }
+        }
+    }
+    *reinterpret_cast<float4_t*>(dst + i) = a;
+    *reinterpret_cast<float4_t*>(dst + i + half) = b;
+}
+
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 // The prefetch's lines a workgroup: the region spread evenly over the grid, at most
@@ -1286,6 +1329,15 @@ extern "C" int crucible_rope_split_qkv(const float* qkv, int64_t ld, float* q, f
                        max_pos <= INT32_MAX && rows >= 0 && rows <= (1 << 24),
                    CRUCIBLE_ERR_INVALID, "%s: bad shape", what);
     if (rows == 0) return CRUCIBLE_OK;
+    if (head_dim % 8 == 0 && ld % 4 == 0 && rows <= 65535 && aligned16(qkv) && aligned16(q) &&
+        aligned16(k) && aligned16(v) && aligned16(cos_table) && aligned16(sin_table)) {
+        const int64_t per_row = (n_head + 2 * n_kv_head) * (head_dim / 8);
+        hipLaunchKernelGGL(rope_split4_kernel, dim3((unsigned)((per_row + 255) / 256), (unsigned)rows),
+                           dim3(256), 0, reinterpret_cast<hipStream_t>(stream), qkv, ld, q, k, v,
+                           cos_table, sin_table, positions, (int)rows, (int)n_head, (int)n_kv_head,
+                           (int)head_dim, (int)max_pos);
+        return fail_launch(what);
+    }
     const int64_t threads = rows * (n_head + 2 * n_kv_head) * (head_dim / 2);
     hipLaunchKernelGGL(rope_split_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
                        reinterpret_cast<hipStream_t>(stream), qkv, ld, q, k, v, cos_table,
