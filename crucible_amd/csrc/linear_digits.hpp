@@ -16,9 +16,9 @@
 //   - digit products of equal weight, s = i + j, share an accumulator: 17 products (i, j)
 //     in 7 accumulators. (5, 2), the smallest, is left out: at most 2^-55 max|h| a key, and
 //     nonzero only where the last digit is: elements 2^14 below their row's largest.
-// Rows that this does not fit (a non-finite value, a largest value outside 2^+-60, more than
-// one element in 16 with a last digit) and columns with a weight over 127 or not finite take plain f64 sums instead, 32 x 32
-// outputs at a time.
+// Rows that this does not fit (a non-finite value, a largest value outside 2^-60 .. 2^22, more
+// than one nonzero element in 16 small enough to reach the last digit or be rounded) and columns
+// with a weight over 127 or not finite take plain f64 sums instead, 32 x 32 outputs at a time.
 //
 // Two launches: digits_kernel writes the digit planes of both operands into the caller's
 // workspace in MFMA operand order, digits_gemm_kernel multiplies them.
@@ -248,11 +248,13 @@ __global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
     // the exponent of 2^e > bound / 2
     const float bound = (float)((double)__builtin_bit_cast(float, mx) * scale * 1.00001);
     const int e = (int)((__builtin_bit_cast(uint32_t, bound) >> 23) & 255) - 127;
-    // Usual magnitudes only: every power of two below is a normal f32.
-    const bool usual = mx < 0x7f800000u && e >= -60 && e <= 60;
-    const bool zero = mx == 0;
+    // Usual magnitudes only: every power of two below is a normal f32, and the scaling up exact.
+    // x * norm_w below the normal range bounds nothing: the row's scale may lift h out of it.
+    const bool usual = mx >= 0x00800000u && mx < 0x7f800000u && e >= -60 && e <= 21;  // up >= 1
+    const bool zero = mx == 0 && (!NORM || tot == 0.0);
     const float up = usual ? __builtin_bit_cast(float, (uint32_t)(21 - e + 127) << 23) : 0.0f;
-    int low = 0;
+    // Elements of |t| < 2^7, whose bits reach the last digit or past it, and the zeros of them.
+    int small = 0, none = 0;
     unsigned char* blk = a.ws + (int64_t)(row >> 5) * steps * kXBlk + (row & 31) * 16;
     auto write = [&](int g, const Group& v) {
         uint32_t hi[16], lo[16];
@@ -267,7 +269,8 @@ __global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
                 const float tl = (t - th) * 16777216.0f;            // exact, |tl| <= 2^23
                 const float tr = rintf(tl);                         // rounds below 2^-22 of the largest
                 const uint32_t l = (uint32_t)((int)tr + 0x808080);  // 25 bits, carry on top
-                low += (l & 0xffu) != 0x80u;                        // its last digit is used
+                small += fabsf(t) < 128.0f;
+                none += t == 0.0f;
                 hi[4 * q + i] = ((uint32_t)((int)th + (int)(l >> 24) + 0x808080)) ^ 0x808080u;
                 lo[4 * q + i] = l ^ 0x808080u;
             }
@@ -292,6 +295,7 @@ __global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
             write(g, held[0]);
         }
     }
+    int low = small | none << 16;  // k_in < 2^15
     s_low[kg][r] = low;
     if (tid == 0) s_flag = 0;
     __syncthreads();
@@ -302,7 +306,7 @@ __global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
         reinterpret_cast<double*>(a.ws + a.l.scale_off)[row] =
             usual ? __builtin_bit_cast(double, (uint64_t)(e - 61 + 1023) << 52) : 0.0;
         reinterpret_cast<double*>(a.ws + a.l.norm_off)[row] = scale;
-        if (ok && !zero && (!usual || low * 16 > p.k_in)) atomicOr(&s_flag, 1);
+        if (ok && !zero && (!usual || ((low & 0xffff) - (low >> 16)) * 16 > p.k_in - (low >> 16))) atomicOr(&s_flag, 1);
     }
     __syncthreads();
     if (tid == 0) reinterpret_cast<int*>(a.ws + a.l.xflag_off)[blockIdx.x] = s_flag;

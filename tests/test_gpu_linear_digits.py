@@ -137,6 +137,34 @@ def test_unusual_rows(gpu, dev, tune, bad):
     assert np.array_equal(got[32:64], _run(gpu, dev, x[32:64], w)), "another block changed"
 
 
+@pytest.mark.parametrize("spread,others", [(2.0 ** 47, 255), (2.0 ** 60, 255), (2.0 ** 100, 255),
+                                           (2.0 ** 40, 10), (2.0 ** 60, 1)])
+def test_outliers_out_of_sight(gpu, dev, tune, spread, others):
+    """Elements below the last digit of their row's largest, all of them or the few that are not
+    zero: columns that do not see the largest get the others' f64 sums."""
+    tune(linear_tile=64)
+    rng = np.random.default_rng(17)
+    x = np.zeros((64, 256), np.float32)
+    x[:, :others] = rng.uniform(0.5, 1.0, (64, others)) * 2.0 ** -41
+    x[:, 255] = spread * 2.0 ** -41
+    w = (rng.standard_normal((48, 256)) * 0.02).astype(np.float16)
+    w[::2, 255] = 0
+    _check(_run(gpu, dev, x, w), (x.astype(np.float64) @ w.astype(np.float64).T).astype(np.float32))
+
+
+@pytest.mark.parametrize("size,weight", [(1e-38, 1e-8), (1e-37, 2e-6), (0.0, 1.0)])
+def test_norm_lifts_products_out_of_the_subnormals(gpu, dev, tune, size, weight):
+    """x * norm_w is zero or subnormal, the normalised row is not."""
+    tune(linear_tile=64)
+    rng = np.random.default_rng(19)
+    x = (rng.uniform(0.5, 1.0, (40, 128)) * size).astype(np.float32)
+    nw = np.full(128, weight, np.float32)
+    w = (rng.uniform(50, 100, (40, 128))).astype(np.float16)
+    want = (_h(x, nw) @ w.astype(np.float64).T).astype(np.float32)
+    assert (size == 0.0) == (not want.any())
+    _check(_run(gpu, dev, x, w, nw), want)
+
+
 def test_workspace_is_checked(gpu, dev):
     """A workspace below the size asked for is refused before any launch; a null one means the
     plain product."""
