@@ -1659,9 +1659,11 @@ void launch_decode_hd(const DecodeArgs& a, bool q_f32, hipStream_t stream) {
 
 // head_dim other than 64: decode_hd_kernel for multiples of 32, else decode_generic_kernel
 // over (request, query head). Appends, where the entry has them, are launched before it on
-// the same stream (decode_hd_kernel makes them itself). The workspace is optional scratch for the splits' partials, uncleared:
-// what crucible_attention_decode_workspace_bytes asks for holds them (its 4-page splits of
-// 64 + 2 floats and fixed region against 16-page splits of at most 256 + 2).
+// the same stream (decode_hd_kernel makes them itself). The workspace is optional, uncleared
+// scratch for the splits' partials. They go where the partials of head_dim 64 do, behind the
+// counters and the unit plan, which a caller's other launches rely on. What
+// crucible_attention_decode_workspace_bytes asks for holds them up to head_dim 160 (its 4-page
+// splits of 64 + 2 floats against 16-page splits of hd + 2); wider heads may need one split more.
 int launch_decode_generic(DecodeArgs a, int hd, bool q_f32, void* workspace,
                           size_t workspace_bytes, hipStream_t stream, const char* what) {
     CRUCIBLE_CHECK(a.n_head <= 65535, CRUCIBLE_ERR_INVALID, "%s: n_head %d too large", what,
@@ -1674,8 +1676,9 @@ int launch_decode_generic(DecodeArgs a, int hd, bool q_f32, void* workspace,
         const int64_t partials = checked_mul(a.batch, a.n_head, a.n_splits);
         const int64_t bytes = checked_mul(partials, (hd + 2) * (int64_t)sizeof(float));
         if (workspace && aligned16(workspace) && a.n_splits > 1 && bytes > 0 &&
-            partials * (hd / 4) <= (int64_t)INT32_MAX && (uint64_t)bytes <= workspace_bytes) {
-            a.po = static_cast<float*>(workspace);
+            partials * (hd / 4) <= (int64_t)INT32_MAX && workspace_bytes >= kCounterBytes + kPlanBytes &&
+            (uint64_t)bytes <= workspace_bytes - (kCounterBytes + kPlanBytes)) {
+            a.po = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes + kPlanBytes);
             a.pm = a.po + partials * hd;
             a.pl = a.pm + partials;
         }

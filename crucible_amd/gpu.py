@@ -160,8 +160,9 @@ class Gpu:
         other dimensions keep nothing between calls and never needed calls to be ordered, so
         theirs is scratch of the call's own."""
         if head_dim != 64:
+            # one split more than head_dim 64's need: wider heads round up to larger splits
             return self._scratch(max(16, self.lib.crucible_attention_decode_workspace_bytes(
-                batch, n_head, max_seq)))
+                batch, n_head, max_seq) + 4 * batch * n_head * (head_dim + 2)))
         return workspace if workspace is not None else self.workspace(batch, n_head, max_seq, pools)
 
     @staticmethod

@@ -152,8 +152,9 @@ int crucible_cache_store_packed_paged(const void* src, int src_dtype, void* pool
  * n_head / n_kv_head <= 16. Any other multiple of 32 up to 256 runs MFMA kernels of its own
  * when q, out, the new rows and the RoPE tables are 16-byte aligned (and rows of q and of the
  * new keys start there): splits of 16 pages, joined by a second launch when the call brings a
- * workspace (used as plain scratch: it needs no clearing and nothing is kept in it) and by the
- * same workgroup, with the same bits, when it does not. The remaining multiples of 8, and
+ * workspace that holds them (uncleared; only its partials' part, behind the counters and the
+ * plan described below, is written) and by the same workgroup, with the same bits, when it does
+ * not. The remaining multiples of 8, and
  * unaligned buffers, run a generic kernel (one workgroup per request and query head, f32
  * arithmetic, no workspace). For every head_dim other than 64 the pool layout and the results
  * are the same to the tolerance of f32 accumulation, the fused entries write the bytes of the

@@ -137,3 +137,36 @@ def test_large_and_tiny_f32_queries(gpu, dev):
         assert torch.isfinite(outs[0]).all()
         # scores of 1e5 x 1e-5 products keep 2^-22 of their magnitude (about 11): 1e-4 of weight
         assert float((outs[0] - outs[1]).abs().max()) <= (1e-4 if factor > 1 else TOL)
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+def test_workspace_shared_with_head_dim_64(gpu, dev, hd):
+    """Calls of other head dimensions leave the counters and the unit plan of a workspace alone,
+    so a caller's head_dim 64 launches around them give the bits they give by themselves."""
+    from crucible_amd import _lib
+    lib = _lib.load()
+    lens, n_head, n_kv = [600, 33, 257], 12, 3
+    b = len(lens)
+    d_len = torch.tensor(lens, dtype=torch.int32, device=dev)
+    wide, usual = (_case(dev, d, d, n_head, n_kv, lens) for d in (hd, 64))
+    max_seq = usual[1] * 16
+    nbytes = lib.crucible_attention_decode_workspace_bytes(b, n_head, max_seq) + 4 * b * n_head * (hd + 2)
+    fixed = lib.crucible_attention_decode_workspace_bytes(1, 1, 1) - 4 * 66  # one split's partials
+    ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
+
+    def run(case, d):
+        _, stride, kv, (kp, vp), tables, q = case
+        out = torch.zeros(b, n_head * d, device=dev)
+        _lib.check(lib.crucible_attention_decode_paged(
+            q.data_ptr(), 0, kp.data_ptr(), vp.data_ptr(), out.data_ptr(), 0, tables.data_ptr(),
+            d_len.data_ptr(), b, n_head, n_kv, d, stride, 2, 1, kv, max_seq, ws.data_ptr(), nbytes,
+            torch.cuda.current_stream().cuda_stream))
+        return out
+
+    before = ws.clone()
+    first = run(wide, hd)
+    assert torch.equal(ws[:fixed], before[:fixed]), "the counters or the plan were written"
+    assert not torch.equal(ws[fixed:], before[fixed:]), "the partials are not where they should be"
+    want = run(usual, 64)
+    assert torch.equal(run(wide, hd), first)
+    assert torch.equal(run(usual, 64), want)
