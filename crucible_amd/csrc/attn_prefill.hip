@@ -1746,7 +1746,7 @@ __global__ __launch_bounds__(kGenericThreads) void prefill_generic_kernel(Prefil
 // An OWNERS tile may hold rows of several requests: each owner's rows are attended, merged and
 // stored on their own, so no value of one request reaches another's rows.
 template <int HD, int W, int QB, bool QF32, bool HYB>
-__global__ __launch_bounds__(64 * W) void prefill_hd_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(64 * W, W == 8 ? 4 : 1) void prefill_hd_kernel(PrefillArgs a) {
     __shared__ HdLds<HD, W, QB> lds;
     const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1816,7 +1816,17 @@ __global__ __launch_bounds__(64 * W) void prefill_hd_kernel(PrefillArgs a) {
 #pragma unroll
         for (int b = 0; b < QB; ++b) s[b].clear();
         int64_t page0 = page_of(2 * wave), page1 = page_of(2 * wave + 1);
-        for (int p = 2 * wave; p < n_pages; p += 2 * W) {
+        // Pairs that every row of this owner sees whole go first, without masks (other columns
+        // are attended too and dropped); the tile's diagonal follows.
+        int whole = INT32_MAX;  // the smallest last key
+#pragma unroll
+        for (int b = 0; b < QB; ++b) whole = min(whole, see[b] >= 0 ? see[b] : INT32_MAX);
+#pragma unroll
+        for (int off = 1; off < 16; off <<= 1) whole = min(whole, __shfl_xor(whole, off));
+        const int whole_pages = (__builtin_amdgcn_readfirstlane(whole) + 1) >> kPageShift;
+        int p = 2 * wave;
+        auto attend = [&](auto mask_tag) {
+            constexpr bool kMask = decltype(mask_tag)::value;
             HdPair<HD> kv;
             if (!HYB || p < pool_pages)
                 kv.load(a.k_pool, a.v_pool, block_base(a.addr, page0), block_base(a.addr, page1),
@@ -1827,10 +1837,20 @@ __global__ __launch_bounds__(64 * W) void prefill_hd_kernel(PrefillArgs a) {
             page0 = page_of(p + 2 * W);  // beside the K/V loads, not before the next ones
             page1 = page_of(p + 2 * W + 1);
             const int key0 = p * kPageTokens;
-            if (key0 + 2 * kPageTokens > last + 1) kv.zero_tail(key0, last + 1, grp);
+            if constexpr (kMask) {
+                if (key0 + 2 * kPageTokens > last + 1) kv.zero_tail(key0, last + 1, grp);
+                if (__ballot(kv.v_not_finite()) != 0) {
 #pragma unroll
-            for (int b = 0; b < QB; ++b) hd_attend_pair(s[b], q[b], kv, key0, see[b], grp);
-        }
+                    for (int b = 0; b < QB; ++b) hd_spoil(s[b], kv, key0, see[b], grp);
+                    kv.zero_not_finite();
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < QB; ++b)
+                hd_attend_pair<HD, QF32, kMask>(s[b], q[b], kv, key0, see[b], grp);
+        };
+        for (; p + 2 <= whole_pages; p += 2 * W) attend(std::false_type{});
+        for (; p < n_pages; p += 2 * W) attend(std::true_type{});
         hd_merge_waves<HD, W, QB>(lds, s, wave, col, grp, 16 * QB);
         if (wave == 0)
 #pragma unroll

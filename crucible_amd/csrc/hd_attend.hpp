@@ -153,11 +153,35 @@ struct HdPair {
 #pragma unroll
                     for (int i = 0; i < HD / 16; ++i) v[p][i][r] = (half_t)0.0f;
     }
+    // Whether the lane holds an infinite or NaN V value.
+    __device__ __forceinline__ bool v_not_finite() const {
+        // an exponent of all ones carries into its half's top bit
+        uint32_t bad = 0;
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int i = 0; i < HD / 16; ++i) {
+                struct Words { uint32_t w[2]; };
+                const Words x = __builtin_bit_cast(Words, v[p][i]);
+                bad |= ((x.w[0] & 0x7c007c00u) + 0x04000400u) | ((x.w[1] & 0x7c007c00u) + 0x04000400u);
+            }
+        return (bad & 0x80008000u) != 0;
+    }
+    __device__ __forceinline__ void zero_not_finite() {
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int i = 0; i < HD / 16; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if ((__builtin_bit_cast(uint16_t, (half_t)v[p][i][r]) & 0x7c00) == 0x7c00)
+                        v[p][i][r] = (half_t)0.0f;
+    }
 };
 
-// One pair into a column block's state: the column sees keys up to `last` (-1: none).
-// s.l is the lane's own sum until finish().
-template <int HD, bool F32>
+// One pair into a column block's state: the column sees keys up to `last` (-1: none), or the
+// whole pair (MASK false). s.l is the lane's own sum until hd_merge_waves.
+template <int HD, bool F32, bool MASK = true>
 __device__ __forceinline__ void hd_attend_pair(HdState<HD>& s, const HdQuery<HD, F32>& q,
                                                const HdPair<HD>& kv, int key0, int last, int grp) {
     float4_t st[2];
@@ -175,7 +199,7 @@ __device__ __forceinline__ void hd_attend_pair(HdState<HD>& s, const HdQuery<HD,
     for (int p = 0; p < 2; ++p)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            st[p][r] = key0 + 16 * p + 4 * grp + r <= last ? st[p][r] : -INFINITY;
+            if constexpr (MASK) st[p][r] = key0 + 16 * p + 4 * grp + r <= last ? st[p][r] : -INFINITY;
             mx = fmaxf(mx, st[p][r]);
         }
     const float mn = fmaxf(s.m, group_max4(mx) * q.scale);
@@ -206,6 +230,31 @@ __device__ __forceinline__ void hd_attend_pair(HdState<HD>& s, const HdQuery<HD,
         const half8_t va = __builtin_shufflevector(kv.v[0][i], kv.v[1][i], 0, 1, 2, 3, 4, 5, 6, 7);
         s.o[i] = mfma_16x16x32(va, ph, s.o[i] * alpha);
         s.o[i] = mfma_16x16x32(va, pl, s.o[i]);
+    }
+}
+
+// A masked key's weight of 0 does not cancel an infinite or NaN V. Where a pair has such values
+// and some columns see only a part of it, this makes the outputs NaN whose column sees one (the
+// count of those is a product of two 0/1 operands), and the values are zeroed before
+// hd_attend_pair.
+template <int HD>
+__device__ __forceinline__ void hd_spoil(HdState<HD>& s, const HdPair<HD>& kv, int key0, int last,
+                                         int grp) {
+    half8_t sees;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        sees[e] = key0 + 16 * (e >> 2) + 4 * grp + (e & 3) <= last ? (half_t)1.0f : (half_t)0.0f;
+#pragma unroll
+    for (int i = 0; i < HD / 16; ++i) {
+        half8_t bad;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            bad[e] = (__builtin_bit_cast(uint16_t, (half_t)kv.v[e >> 2][i][e & 3]) & 0x7c00) == 0x7c00
+                         ? (half_t)1.0f : (half_t)0.0f;
+        const float4_t n = mfma_16x16x32(bad, sees, float4_t{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (n[r] > 0.0f) s.o[i][r] = __builtin_nanf("");
     }
 }
 

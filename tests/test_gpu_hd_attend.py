@@ -120,6 +120,34 @@ def test_prefill_against_generic(gpu, dev, hd, dtype):
     assert torch.all(torch.isnan(other[touched]))
 
 
+@pytest.mark.parametrize("hd", [32, 128, 256])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_prefill_rows_before_an_infinite_value(gpu, dev, hd, bad):
+    """V values that are not finite reach the rows that see them, and no earlier row of the tile;
+    positions descend within the second request."""
+    lens, at = [70, 40], [37, 8]
+    n_head, n_kv, layer = 4, 2, 1
+    g, stride, kv, (kp, vp), tables, _ = _case(dev, hd + 1, hd, n_head, n_kv, lens)
+    owners = np.repeat(np.arange(2, dtype=np.int32), lens)
+    positions = np.concatenate([np.arange(70), np.arange(40)[::-1]]).astype(np.int32)
+    pool = vp.view(-1, 2, kv, 16)
+    for r, t in enumerate(at):
+        pool[tables[r, t // 16].long(), layer, :, t % 16] = bad
+    q = torch.randn(110, n_head * hd, generator=g, device=dev)
+    d_own, d_pos = (torch.from_numpy(a).to(dev) for a in (owners, positions))
+
+    def run(q):
+        out = torch.full((110, n_head * hd), 7.0, device=dev)
+        gpu.attention_prefill_packed(q, kp, vp, out, tables, d_own, d_pos, 110, stride, n_head, n_kv,
+                                     hd, 2, layer, kv, stride * 16)
+        return out
+
+    got, want = run(q), run(_unaligned(q))
+    sees = torch.from_numpy(positions >= np.array(at)[owners]).to(dev)
+    assert not torch.isfinite(got[sees]).any() and not torch.isfinite(want[sees]).any()
+    assert float((got[~sees] - want[~sees]).abs().max()) <= TOL
+
+
 def test_large_and_tiny_f32_queries(gpu, dev):
     """f32 queries outside fp16's range: the operands are scaled by a power of two."""
     hd, n_head, n_kv, lens = 128, 4, 2, [70, 33]
