@@ -1739,9 +1739,10 @@ __global__ __launch_bounds__(kGenericThreads) void prefill_generic_kernel(Prefil
 // waves take every W-th pair of pages of the rows' key range and merge at the end. K and V
 // stream from L2 once per 16 QB rows (attend_generic reads them once a row), so 32 rows a
 // workgroup where the registers hold them, and 4 waves, whose 512 registers a lane do: prompts
-// of 1000, 333, 777 and 64 tokens, 12/3 heads of 128, 41.8 us (8 waves of 32 rows spill: 59.9;
-// 8 waves of 16 rows 59.0; attend_generic 820). Later row tiles,
-// whose key ranges are longer, are dispatched first.
+// of 1000, 333, 777 and 64 tokens, 12/3 heads of 128, 42.5 us (8 waves of 32 rows spill: 59.9;
+// 8 waves of 16 rows 59.0; attend_generic 820). With 8 waves (32 dims) the registers are capped
+// at 128, so that two workgroups share a CU. Later row tiles, whose key ranges are longer, are
+// dispatched first.
 //
 // An OWNERS tile may hold rows of several requests: each owner's rows are attended, merged and
 // stored on their own, so no value of one request reaches another's rows.
