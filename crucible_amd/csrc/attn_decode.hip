@@ -1122,80 +1122,21 @@ __global__ __launch_bounds__(kGenericThreads) void decode_generic_kernel(DecodeA
     });
 }
 
-// head_dim a multiple of 32 (hd_attend.hpp): a workgroup takes a split of 16 pages, a pair a wave at a time,
-// of one (request, kv head, block of 16 query heads), so each K/V byte is read once per
+// head_dim a multiple of 32 (hd_attend.hpp): a workgroup takes a split of 16 pages, a pair a wave
+// at a time, of one (request, kv head, block of 16 query heads), so each K/V byte is read once per
 // GQA group. With scratch for the partials the grid holds every split and
 // decode_hd_combine_kernel joins them; without (a.po null) a workgroup walks its unit's splits.
 // Both join the splits in the same order with the same steps, so they give the same bits.
 // A second kernel instead of decode_kernel's counters: the scratch needs no clearing, and
 // callers of these dimensions never had to clear or own one. HBM-bound at large batches,
 // latency-bound below; the split is small because one CU streams only 25-50 GB/s. 16 requests
-// of 64..2048 tokens, 12/3 heads of 128, fused append (26 MB): 70 us a layer in three launches
-// with attend_generic, 22.5 here, 13.5 of it in this kernel (traced) and 5 in the combine. Up to
+// of 64..2048 tokens, 12/3 heads of 128, fused append (26 MB): 70 us a layer with
+// attend_generic, 22.2 here with the append and the combine launches. Up to
 // 128 dims the registers are capped at 128, so that two workgroups share a CU (a few of the
 // f32-query form spill; uncapped it took 22 us against 19).
 constexpr int kHdSplitPages = 16;
 
-//
-// APPEND: the appended row (rotated when RoPE tables are given) goes from k_new / v_new into the
-// operands of every wave that reads its page, and one of them stores it, so the pools and the
-// outputs are those of the separate appends followed by the attention. Loading and storing it
-// apart from the page loads, in two more dependent round trips each, cost 5.5 us a launch.
-
-// Channels d .. d + N - 1 of the appended K row of request b, kv head g, as the append stores
-// them: N <= 8 channels of one half of the head.
-template <int HD, int N>
-__device__ __forceinline__ void hd_new_k(const DecodeArgs& a, int b, int g, int d, half_t (&out)[N]) {
-    const int64_t at = (int64_t)b * a.kv_new_stride + g * HD;
-    auto load = [&](int from, float (&x)[N]) {
-        if constexpr (N == 8) {  // 16-byte aligned (hd_decode_fits)
-            if (a.kv_new_f16) hd_load8<false>(a.k_new, at + from, x);
-            else hd_load8<true>(a.k_new, at + from, x);
-        } else {
-#pragma unroll
-            for (int i = 0; i < N; ++i)
-                x[i] = a.kv_new_f16 ? (float)static_cast<const half_t*>(a.k_new)[at + from + i]
-                                    : static_cast<const float*>(a.k_new)[at + from + i];
-        }
-    };
-    float x[N];
-    load(d, x);
-    if (a.rope_cos) {
-        constexpr int kHalf = HD / 2;
-        const bool low = d < kHalf;
-        float y[N];
-        load(low ? d + kHalf : d - kHalf, y);
-        const int64_t t = (int64_t)min(max(a.positions[b], 0), a.rope_max_pos - 1) * kHalf + (low ? d : d - kHalf);
-        float c[N], sn[N];
-        if constexpr (N == 8) {
-            hd_load8<true>(a.rope_cos, t, c);
-            hd_load8<true>(a.rope_sin, t, sn);
-        } else {
-#pragma unroll
-            for (int i = 0; i < N; ++i) {
-                c[i] = a.rope_cos[t + i];
-                sn[i] = a.rope_sin[t + i];
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            float lo = low ? x[i] : y[i], hi = low ? y[i] : x[i];
-            rope_pair(lo, hi, c[i], sn[i]);
-            x[i] = low ? lo : hi;
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < N; ++i) out[i] = (half_t)x[i];
-}
-
-template <int HD>
-__device__ __forceinline__ half_t hd_new_v(const DecodeArgs& a, int b, int g, int d) {
-    const int64_t at = (int64_t)b * a.kv_new_stride + g * HD + d;
-    return a.kv_new_f16 ? static_cast<const half_t*>(a.v_new)[at]
-                        : (half_t) static_cast<const float*>(a.v_new)[at];
-}
-
-template <int HD, bool QF32, bool APPEND, bool WHOLE>
+template <int HD, bool QF32, bool WHOLE>
 __global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 ? 4 : 1) void decode_hd_kernel(DecodeArgs a, int col_blocks) {
     constexpr int W = hd_waves(HD);
     __shared__ HdLds<HD, W, 1> lds;
@@ -1214,30 +1155,9 @@ __global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 ? 4 : 1) void decode_h
     asm volatile("" : "+s"(id0), "+s"(id1));  // issued with the length's load, not behind its branch
     int64_t page0 = id0, page1 = id1;
     const int len = request_len(a, b);
-    const int apos = APPEND ? a.positions[b] : -1;
-    // The append of a position that is not attended (at or past the length). As
-    // crucible_cache_store_rows_paged: outside the table it is skipped and its entry not read;
-    // past the last split it belongs to that split.
-    auto append_only = [&]() {
-        const int ap = apos >> kPageShift;
-        if (!APPEND || apos < 0 || apos < len || ap >= a.table_stride || c0 != 0 ||
-            min(ap / kHdSplitPages, (int)gridDim.z - 1) != (int)blockIdx.z)
-            return;
-        const int64_t base = block_base(a.addr, (int64_t)table[ap]);
-        const int slot = apos & kPageMask;
-        for (int d = threadIdx.x; d < HD; d += 64 * W) {
-            half_t k[1];
-            hd_new_k<HD, 1>(a, b, g, d, k);
-            a.k_pool[base + (int64_t)slot * a.addr.kv_dim + g * HD + d] = k[0];
-            a.v_pool[base + (int64_t)(g * HD + d) * kPageTokens + slot] = hd_new_v<HD>(a, b, g, d);
-        }
-    };
     const int n_pages = len > 0 ? (len + kPageMask) >> kPageShift : 0;
     const int n_active = (n_pages + kHdSplitPages - 1) / kHdSplitPages;
-    if (s0 >= n_active) {  // past the end, or an inactive request: its output is untouched
-        append_only();
-        return;
-    }
+    if (s0 >= n_active) return;  // past the end, or an inactive request: its output is untouched
 
     // The first pages are requested before the queries are waited for.
     HdPair<HD> kv;
@@ -1246,40 +1166,6 @@ __global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 ? 4 : 1) void decode_h
         const int64_t base0 = block_base(a.addr, page0);
         const int64_t base1 = block_base(a.addr, p + 1 < n_pages ? page1 : page0);
         kv.load(a.k_pool, a.v_pool, base0, base1, a.addr.kv_dim, g * HD, col, grp);
-        if (!APPEND || apos >= len || (apos >> 1) >> kPageShift != p >> 1 || apos < 0) return;
-        // The appended row's page (uniform): every lane loads its share of the row beside the
-        // page loads; the lanes whose operand slots it fills take it and, once per kv head,
-        // store it.
-        const int slot = apos & kPageMask, pg = (apos >> kPageShift) & 1;
-        const int64_t base = pg ? base1 : base0;
-        half_t nk[HD / 32][8], nv[HD / 16];
-#pragma unroll
-        for (int k = 0; k < HD / 32; ++k) hd_new_k<HD, 8>(a, b, g, 32 * k + 8 * grp, nk[k]);
-#pragma unroll
-        for (int d = 0; d < HD / 16; ++d) nv[d] = hd_new_v<HD>(a, b, g, 16 * d + col);
-        const bool has_k = col == slot, has_v = grp == slot >> 2;
-#pragma unroll
-        for (int k = 0; k < HD / 32; ++k) {
-            half8_t row;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) row[e] = nk[k][e];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-                if (has_k && pg == i) kv.k[i][k] = row;
-            if (has_k && c0 == 0)
-                *reinterpret_cast<half8_t*>(a.k_pool + base + (int64_t)slot * a.addr.kv_dim + g * HD +
-                                            32 * k + 8 * grp) = row;
-        }
-#pragma unroll
-        for (int d = 0; d < HD / 16; ++d) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (has_v && pg == i && (slot & 3) == r) kv.v[i][d][r] = nv[d];
-            if (has_v && c0 == 0)
-                a.v_pool[base + (int64_t)(g * HD + 16 * d + col) * kPageTokens + slot] = nv[d];
-        }
     };
     load(first);
     __builtin_amdgcn_sched_barrier(0);
@@ -1334,7 +1220,6 @@ __global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 ? 4 : 1) void decode_h
         else total.merge(s[0]);
         if (sp + 1 == n_active) break;
     }
-    append_only();
     const int64_t out = (int64_t)b * a.out_row_stride + (int64_t)h * HD;
     const bool mine = wave == 0 && col < n_cols;
     if (WHOLE || n_active == 1) {
@@ -1392,12 +1277,15 @@ __global__ __launch_bounds__(256) void decode_hd_combine_kernel(DecodeArgs a, in
                total.o[0] * (1.0f / total.l));
 }
 
-// The qkv entry's two appends for head_dim other than 64: row b's K (rotated at
-// positions[b] when RoPE tables are given) and its V, f32 rows of stride kv_new_stride,
-// rounded to fp16 and stored at positions[b] as crucible_rope_split_qkv followed by
-// crucible_cache_store_rows_paged stores them (a row whose position lies outside its table
-// is skipped). One thread per (row, kv head, pair).
-__global__ __launch_bounds__(256) void append_rope_generic_kernel(DecodeArgs a, int hd) {
+// The fused entries' two appends for head_dim other than 64: row b's K (rotated at positions[b]
+// when RoPE tables are given) and its V, rows of stride kv_new_stride, rounded to fp16 and stored
+// at positions[b] as crucible_rope_split_qkv followed by crucible_cache_store_rows_paged stores
+// them (a row whose position lies outside its table is skipped). One thread per (row, kv head,
+// pair). A launch of its own: the attention that follows may read any row's append, as rows of
+// one batch may share pages (several positions of one sequence), and a workgroup of the same
+// launch could not wait for the others' stores.
+template <bool F16>
+__global__ __launch_bounds__(256) void append_new_rows_kernel(DecodeArgs a, int hd) {
     const int half = hd >> 1;
     const int64_t per_row = (int64_t)a.n_kv_head * half;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1411,16 +1299,25 @@ __global__ __launch_bounds__(256) void append_rope_generic_kernel(DecodeArgs a, 
     const int64_t base = block_base(a.addr, a.tables[(int64_t)b * a.table_stride + (pos >> kPageShift)]);
     const int slot = pos & kPageMask;
     const int c = g * hd + e;  // channel of the pair's first element
-    const float* kr = static_cast<const float*>(a.k_new) + (int64_t)b * a.kv_new_stride;
-    const float* vr = static_cast<const float*>(a.v_new) + (int64_t)b * a.kv_new_stride;
-    float lo = kr[c], hi = kr[c + half];
-    if (a.rope_cos) {
-        const int p = min(pos, a.rope_max_pos - 1);
-        rope_pair(lo, hi, a.rope_cos[(int64_t)p * half + e], a.rope_sin[(int64_t)p * half + e]);
+    using T = std::conditional_t<F16, half_t, float>;
+    const T* kr = static_cast<const T*>(a.k_new) + (int64_t)b * a.kv_new_stride;
+    const T* vr = static_cast<const T*>(a.v_new) + (int64_t)b * a.kv_new_stride;
+    half_t k0, k1;
+    if constexpr (F16) {  // copied, not converted: the bytes of a NaN stay
+        k0 = kr[c];
+        k1 = kr[c + half];
+    } else {
+        float lo = kr[c], hi = kr[c + half];
+        if (a.rope_cos) {
+            const int p = min(pos, a.rope_max_pos - 1);
+            rope_pair(lo, hi, a.rope_cos[(int64_t)p * half + e], a.rope_sin[(int64_t)p * half + e]);
+        }
+        k0 = (half_t)lo;
+        k1 = (half_t)hi;
     }
     const int kv_dim = a.addr.kv_dim;
-    a.k_pool[base + (int64_t)slot * kv_dim + c] = (half_t)lo;
-    a.k_pool[base + (int64_t)slot * kv_dim + c + half] = (half_t)hi;
+    a.k_pool[base + (int64_t)slot * kv_dim + c] = k0;
+    a.k_pool[base + (int64_t)slot * kv_dim + c + half] = k1;
     a.v_pool[base + (int64_t)c * kPageTokens + slot] = (half_t)vr[c];
     a.v_pool[base + (int64_t)(c + half) * kPageTokens + slot] = (half_t)vr[c + half];
 }
@@ -1632,7 +1529,6 @@ bool hd_decode_fits(const DecodeArgs& a, int hd, bool q_f32) {
     return hd_mfma_ok(hd) && aligned16(a.q) && aligned16(a.out) && aligned16(a.rope_cos) &&
            aligned16(a.rope_sin) &&
            a.q_row_stride % (q_f32 ? 4 : 8) == 0 &&
-           (!a.positions || (aligned16(a.k_new) && a.kv_new_stride % (a.kv_new_f16 ? 8 : 4) == 0)) &&
            a.batch <= 65535 && a.n_kv_head <= 65535 &&
            a.max_pages <= kHdSplitPages * 65535;
 }
@@ -1642,24 +1538,22 @@ void launch_decode_hd(const DecodeArgs& a, bool q_f32, hipStream_t stream) {
     const int blocks = (a.n_rep + 15) / 16;
     const dim3 grid((unsigned)(a.n_kv_head * blocks), (unsigned)a.batch,
                     (unsigned)(a.po ? a.n_splits : 1));
-    auto go = [&](auto f32_tag, auto append_tag) {
-        constexpr bool kF32 = decltype(f32_tag)::value, kAppend = decltype(append_tag)::value;
+    auto go = [&](auto f32_tag) {
+        constexpr bool kF32 = decltype(f32_tag)::value;
         if (a.po)
-            hipLaunchKernelGGL((decode_hd_kernel<HD, kF32, kAppend, false>), grid,
-                               dim3(64 * hd_waves(HD)), 0, stream, a, blocks);
+            hipLaunchKernelGGL((decode_hd_kernel<HD, kF32, false>), grid, dim3(64 * hd_waves(HD)),
+                               0, stream, a, blocks);
         else
-            hipLaunchKernelGGL((decode_hd_kernel<HD, kF32, kAppend, true>), grid,
-                               dim3(64 * hd_waves(HD)), 0, stream, a, blocks);
+            hipLaunchKernelGGL((decode_hd_kernel<HD, kF32, true>), grid, dim3(64 * hd_waves(HD)),
+                               0, stream, a, blocks);
     };
-    if (a.positions && q_f32) go(std::true_type{}, std::true_type{});
-    else if (a.positions) go(std::false_type{}, std::true_type{});
-    else if (q_f32) go(std::true_type{}, std::false_type{});
-    else go(std::false_type{}, std::false_type{});
+    if (q_f32) go(std::true_type{});
+    else go(std::false_type{});
 }
 
 // head_dim other than 64: decode_hd_kernel for multiples of 32, else decode_generic_kernel
 // over (request, query head). Appends, where the entry has them, are launched before it on
-// the same stream (decode_hd_kernel makes them itself). The workspace is optional, uncleared
+// the same stream. The workspace is optional, uncleared
 // scratch for the splits' partials. They go where the partials of head_dim 64 do, behind the
 // counters and the unit plan, which a caller's other launches rely on. What
 // crucible_attention_decode_workspace_bytes asks for holds them up to head_dim 160 (its 4-page
@@ -1706,20 +1600,18 @@ int launch_decode_generic(DecodeArgs a, int hd, bool q_f32, void* workspace,
     return fail_launch(what);
 }
 
-// The two appends of the fused entries for head_dim other than 64, f32 or fp16 rows of
-// stride kv_dim: the library's own crucible_cache_store_rows_paged, so the pools get the
-// bytes the separate calls store.
-int append_rows_generic(const DecodeArgs& a, int kv_dtype, int64_t n_layer, int64_t layer,
-                        hipStream_t stream) {
-    for (int kind : {CRUCIBLE_POOL_K, CRUCIBLE_POOL_V}) {
-        const bool k = kind == CRUCIBLE_POOL_K;
-        if (const int rc = crucible_cache_store_rows_paged(
-                k ? a.k_new : a.v_new, kv_dtype, k ? a.k_pool : a.v_pool, kind, a.tables,
-                a.positions, a.batch, a.addr.kv_dim, a.table_stride, n_layer, layer,
-                reinterpret_cast<crucible_stream_t>(stream)))
-            return rc;
-    }
-    return CRUCIBLE_OK;
+// The fused entries' K and V appends (positions, tables, k_new, v_new of `a`) for head_dim other
+// than 64, in one launch before the attention.
+int append_new_rows(const DecodeArgs& a, int hd, hipStream_t stream, const char* what) {
+    const int64_t threads = (int64_t)a.batch * a.n_kv_head * (hd / 2);
+    CRUCIBLE_CHECK(threads <= (int64_t)INT32_MAX * 256, CRUCIBLE_ERR_INVALID, "%s: too many rows",
+                   what);
+    const dim3 grid((unsigned)((threads + 255) / 256));
+    if (a.kv_new_f16)
+        hipLaunchKernelGGL(append_new_rows_kernel<true>, grid, dim3(256), 0, stream, a, hd);
+    else
+        hipLaunchKernelGGL(append_new_rows_kernel<false>, grid, dim3(256), 0, stream, a, hd);
+    return fail_launch(what);
 }
 
 // Split the request into workgroups, bind the workspace and launch.
@@ -1905,8 +1797,7 @@ extern "C" int crucible_attention_decode_paged_append(
                    (long long)n_layer, (long long)kv_dim);
     a.table_stride = (int32_t)table_stride;
     if (head_dim != kHeadDim) {
-        if (!hd_decode_fits(a, (int)head_dim, q_dtype == CRUCIBLE_F32))
-            if (const int rc = append_rows_generic(a, kv_dtype, n_layer, layer, stream)) return rc;
+        if (const int rc = append_new_rows(a, (int)head_dim, stream, what)) return rc;
         return launch_decode_generic(a, (int)head_dim, q_dtype == CRUCIBLE_F32, workspace, workspace_bytes,
                                      stream, what);
     }
@@ -1953,8 +1844,7 @@ extern "C" int crucible_attention_decode_paged_append_noalloc(
                    (long long)n_layer, (long long)kv_dim);
     a.table_stride = (int32_t)table_stride;
     if (head_dim != kHeadDim) {  // the generic kernels use no scratch
-        if (!hd_decode_fits(a, (int)head_dim, q_dtype == CRUCIBLE_F32))
-            if (const int rc = append_rows_generic(a, kv_dtype, n_layer, layer, stream)) return rc;
+        if (const int rc = append_new_rows(a, (int)head_dim, stream, what)) return rc;
         return launch_decode_generic(a, (int)head_dim, q_dtype == CRUCIBLE_F32, nullptr, 0,
                                      stream, what);
     }
@@ -2047,14 +1937,7 @@ extern "C" int crucible_attention_decode_qkv_paged_append(
                    (long long)n_layer, (long long)kv_dim);
     a.table_stride = (int32_t)table_stride;
     if (head_dim != kHeadDim) {
-        const int64_t threads = batch * n_kv_head * (head_dim / 2);
-        CRUCIBLE_CHECK(threads <= (int64_t)INT32_MAX * 256, CRUCIBLE_ERR_INVALID, "%s: too many rows",
-                       what);
-        if (!hd_decode_fits(a, (int)head_dim, true)) {
-            hipLaunchKernelGGL(append_rope_generic_kernel, dim3((unsigned)((threads + 255) / 256)),
-                               dim3(256), 0, stream, a, (int)head_dim);
-            if (const int rc = fail_launch(what)) return rc;
-        }
+        if (const int rc = append_new_rows(a, (int)head_dim, stream, what)) return rc;
         return launch_decode_generic(a, (int)head_dim, true, workspace, workspace_bytes, stream, what);
     }
     return decode_with_workspace(a, true, workspace, workspace_bytes, stream, what);

@@ -236,7 +236,8 @@ class Gpu:
                                       table_stride, n_layer, layer, kv_dim, max_seq,
                                       workspace=None):
         """Fused gpu_model.rs:1434-1507 sequence: append K and V rows at positions[b], then
-        decode with seq_lens, in one launch (same pool bytes and output as the three calls)."""
+        decode with seq_lens (same pool bytes and output as the three calls). At head_dim 64
+        it is one launch, and no row may attend to a slot that another row appends."""
         _need(q, "q", numel=batch * n_head * head_dim)
         _need(out, "out", numel=batch * n_head * head_dim)
         _need(k_new, "k_new", numel=batch * kv_dim)

@@ -150,8 +150,7 @@ int crucible_cache_store_packed_paged(const void* src, int src_dtype, void* pool
  * (out_dtype). n_head is a multiple of n_kv_head; query head h reads KV head
  * h / (n_head / n_kv_head). head_dim 64 (every preset) runs the MFMA kernels, with
  * n_head / n_kv_head <= 16. Any other multiple of 32 up to 256 runs MFMA kernels of its own
- * when q, out, the new rows and the RoPE tables are 16-byte aligned (and rows of q and of the
- * new keys start there): splits of 16 pages, joined by a second launch when the call brings a
+ * when q, out and the RoPE tables are 16-byte aligned and rows of q start there: splits of 16 pages, joined by a second launch when the call brings a
  * workspace that holds them (uncleared; only its partials' part, behind the counters and the
  * plan described below, is written) and by the same workgroup, with the same bits, when it does
  * not. The remaining multiples of 8, and
@@ -216,11 +215,14 @@ int crucible_attention_decode_paged(const void* q, int q_dtype, const void* k_po
  *   Gpu::cache_store_rows_paged(k_new -> k_pool, positions)   (gpu.rs:1405-1439)
  *   Gpu::cache_store_rows_paged(v_new -> v_pool, positions)
  *   Gpu::attention_decode_paged(q, ..., seq_lens)             (gpu.rs:1441-1500)
- * in one launch. Row b < batch is appended at positions[b] (k_new/v_new are
- * [batch][kv_dim] in kv_dtype, rounded to fp16); the pools receive exactly the
- * bytes the two appends write, and `out` is what attention_decode_paged computes
- * after them (seq_lens[b] <= 0: no output for b, the row is still appended).
- * Same workspace as attention_decode_paged. */
+ * in one launch at head_dim 64, after one launch of both appends at any other. Row b < batch
+ * is appended at positions[b] (k_new/v_new are [batch][kv_dim] in kv_dtype, rounded to fp16);
+ * the pools receive exactly the bytes the two appends write, and `out` is what
+ * attention_decode_paged computes after them (seq_lens[b] <= 0: no output for b, the row is
+ * still appended). At head_dim 64 the launch does not order one row's append before another
+ * row's reads: no row may attend to a slot that another row of the call appends (two positions
+ * of one sequence); make the separate calls for such a batch. Other head dimensions have no
+ * such rule. Same workspace as attention_decode_paged. */
 int crucible_attention_decode_paged_append(
     const void* q, int q_dtype, const void* k_new, const void* v_new, int kv_dtype,
     void* k_pool, void* v_pool, void* out, int out_dtype, const int32_t* page_tables,

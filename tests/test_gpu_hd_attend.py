@@ -91,6 +91,46 @@ def test_append_against_separate_calls(gpu, dev, hd, n_head, n_kv, kv_dtype):
     assert torch.equal(o1, o2)
 
 
+@pytest.mark.parametrize("hd", [32, 96, 128, 160, 192, 224, 256])
+@pytest.mark.parametrize("entry", ["append", "noalloc", "qkv"])
+def test_rows_of_one_batch_that_share_pages(gpu, dev, hd, entry):
+    """Sixteen consecutive positions of one sequence in one call, as in the verification of
+    several tokens: every row sees the earlier rows' appends, and the outputs are those of the
+    separate calls. Four more rows share a page of another sequence in descending order."""
+    from crucible_amd import _lib
+    lib = _lib.load()
+    n_head, n_kv, layer = 4, 2, 1
+    pos = list(range(500, 516)) + [43, 42, 41, 40]
+    lens = [p + 1 for p in pos]
+    b = len(pos)
+    g, stride, kv, (kp, vp), two, _ = _case(dev, hd + 3, hd, n_head, n_kv, [516, 44])
+    tables = two[torch.tensor([0] * 16 + [1] * 4, device=dev)].contiguous()
+    qkv = torch.randn(b, n_head * hd + 2 * kv, generator=g, device=dev)
+    q = qkv[:, :n_head * hd].contiguous()
+    new = [qkv[:, n_head * hd + i * kv:n_head * hd + (i + 1) * kv].contiguous() for i in range(2)]
+    d_len, d_pos = (torch.tensor(x, dtype=torch.int32, device=dev) for x in (lens, pos))
+    k1, v1, k2, v2 = kp.clone(), vp.clone(), kp.clone(), vp.clone()
+    for src, pool, kind in ((new[0], k2, "k"), (new[1], v2, "v")):
+        gpu.cache_store_rows_paged(src, pool, tables, d_pos, b, kv, stride, 2, layer, kind=kind)
+    o1, o2, o3 = (torch.full((b, n_head * hd), 7.0, device=dev) for _ in range(3))
+    geometry = (b, n_head, n_kv, hd, stride, 2, layer, kv, stride * 16)
+    gpu.attention_decode_paged(q, k2, v2, o2, tables, d_len, *geometry)
+    gpu.attention_decode_paged(_unaligned(q), k2, v2, o3, tables, d_len, *geometry)
+    if entry == "append":
+        gpu.attention_decode_paged_append(q, *new, k1, v1, o1, tables, d_pos, d_len, *geometry)
+    elif entry == "qkv":
+        gpu.attention_decode_qkv_paged_append(qkv, None, None, k1, v1, o1, tables, d_pos, d_len,
+                                              *geometry)
+    else:
+        _lib.check(lib.crucible_attention_decode_paged_append_noalloc(
+            q.data_ptr(), 0, new[0].data_ptr(), new[1].data_ptr(), 0, k1.data_ptr(), v1.data_ptr(),
+            o1.data_ptr(), 0, tables.data_ptr(), d_pos.data_ptr(), d_len.data_ptr(), *geometry,
+            torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(k1, k2) and torch.equal(v1, v2)
+    assert torch.equal(o1, o2)
+    assert float((o1 - o3).abs().max()) <= TOL
+
+
 @pytest.mark.parametrize("hd", [32, 96, 128, 160, 256])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 def test_prefill_against_generic(gpu, dev, hd, dtype):
