@@ -10,15 +10,15 @@
 //     256^(2-j), 3 digits for |w| < 0.498, a 4th (j = -1) up to |w| <= 127;
 //   - a row of activations is scaled by a power of two to |X| < 2^46 and rounded to a whole
 //     number: X = sum_i x_i 256^(5-i), 6 digits. An f32 within 2^22 of its row's largest
-//     value keeps every bit; a smaller one is rounded to 2^-46 of the largest, so its term
-//     is off by at most 2^-47 max|h| |w| (for rows of N(0,1) values about one row in a
-//     thousand holds one such element);
-//   - digit products of equal weight, s = i + j, share an accumulator: 17 products (i, j)
-//     in 7 accumulators. (5, 2), the smallest, is left out: at most 2^-55 max|h| a key, and
-//     nonzero only where the last digit is: elements 2^14 below their row's largest.
-// Rows that this does not fit (a non-finite value, a largest value outside 2^-60 .. 2^22, more
-// than one nonzero element in 16 small enough to reach the last digit or be rounded) and columns
-// with a weight over 127 or not finite take plain f64 sums instead, 32 x 32 outputs at a time.
+//     value keeps every bit; what the rounding of a smaller one drops is listed, up to 16
+//     elements a row, and multiplied in f64 with the sums (of rows of 768 N(0,1) values about
+//     one in three thousand has such an element, of SwiGLU outputs one in thirty);
+//   - digit products of equal weight, s = i + j, share an accumulator: 18 products (i, j)
+//     in 8 accumulators (a ninth with the fourth weight digit).
+// So every product is exact, and the sums are joined in f64. Rows that this does not fit (a
+// non-finite value, a largest value outside 2^-60 .. 2^22, more than 16 rounded elements) and
+// columns with a weight over 127 or not finite take plain f64 sums instead, 32 x 32 outputs at
+// a time.
 //
 // Two launches: digits_kernel writes the digit planes of both operands into the caller's
 // workspace in MFMA operand order, digits_gemm_kernel multiplies them.
@@ -69,12 +69,20 @@ constexpr int kPart = 128;          // K range of one weight workgroup
 constexpr int kWgRows = 8;          // rows of one activation workgroup
 constexpr int kRowWgs = kBlk / kWgRows;
 constexpr int kMaxK = 16384;        // 4 products of 2^14 a key stay below 2^31
+constexpr int kRests = 16;          // listed elements of a row
 
-// Workspace: the planes' blocks first (1 KiB aligned), then the rows' scales, then flags.
+// What the digits of element k leave of it, in units of X.
+struct Rest {
+    int k;
+    float r;
+};
+
+// Workspace: the planes' blocks first (1 KiB aligned), then the rows' scales and rests, then
+// flags (rows: 1 f64 sums, 2 some row has rests; columns: 1 a fourth digit, 2 f64 sums).
 //   x planes [row block][K / 32][6][1024], w planes [column block][K / 32][4][1024]
 struct Layout {
     int64_t row_blks, col_blks, parts;
-    int64_t w_off, scale_off, norm_off, xflag_off, wflag_off, bytes;
+    int64_t w_off, scale_off, norm_off, rest_off, count_off, xflag_off, wflag_off, bytes;
 };
 
 Layout make_layout(int64_t rows, int64_t cols, int64_t k_in) {
@@ -87,7 +95,9 @@ Layout make_layout(int64_t rows, int64_t cols, int64_t k_in) {
     l.w_off = l.row_blks * steps * kXBlk;
     l.scale_off = l.w_off + l.col_blks * steps * kWBlk;
     l.norm_off = l.scale_off + l.row_blks * kBlk * 8;
-    l.xflag_off = l.norm_off + l.row_blks * kBlk * 8;
+    l.rest_off = l.norm_off + l.row_blks * kBlk * 8;
+    l.count_off = l.rest_off + l.row_blks * kBlk * kRests * (int64_t)sizeof(Rest);
+    l.xflag_off = l.count_off + l.row_blks * kBlk * 4;
     l.wflag_off = l.xflag_off + l.row_blks * kRowWgs * 4;
     l.bytes = l.wflag_off + l.col_blks * l.parts * 4;
     return l;
@@ -136,7 +146,8 @@ template <int G, bool NORM>
 __global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
     __shared__ double s_ss[32][kWgRows];
     __shared__ uint32_t s_mx[32][kWgRows];
-    __shared__ int s_low[32][kWgRows];
+    __shared__ Rest s_rest[kWgRows][kRests];
+    __shared__ int s_rests[kWgRows];
     __shared__ int s_flag;
     const DigitLinear& p = a.p;
     const int tid = threadIdx.x;
@@ -235,6 +246,8 @@ __global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
     }
     s_ss[kg][r] = ss;
     s_mx[kg][r] = mx;
+    if (tid < kWgRows) s_rests[tid] = 0;
+    if (tid == 0) s_flag = 0;
     __syncthreads();
     double tot = 0.0;
     mx = 0;
@@ -253,8 +266,6 @@ __global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
     const bool usual = mx >= 0x00800000u && mx < 0x7f800000u && e >= -60 && e <= 21;  // up >= 1
     const bool zero = mx == 0 && (!NORM || tot == 0.0);
     const float up = usual ? __builtin_bit_cast(float, (uint32_t)(21 - e + 127) << 23) : 0.0f;
-    // Elements of |t| < 2^7, whose bits reach the last digit or past it, and the zeros of them.
-    int small = 0, none = 0;
     unsigned char* blk = a.ws + (int64_t)(row >> 5) * steps * kXBlk + (row & 31) * 16;
     auto write = [&](int g, const Group& v) {
         uint32_t hi[16], lo[16];
@@ -269,8 +280,10 @@ __global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
                 const float tl = (t - th) * 16777216.0f;            // exact, |tl| <= 2^23
                 const float tr = rintf(tl);                         // rounds below 2^-22 of the largest
                 const uint32_t l = (uint32_t)((int)tr + 0x808080);  // 25 bits, carry on top
-                small += fabsf(t) < 128.0f;
-                none += t == 0.0f;
+                if (tl != tr) {
+                    const int at = atomicAdd(&s_rests[r], 1);
+                    if (at < kRests) s_rest[r][at] = {g * 16 + 4 * q + i, tl - tr};  // exact
+                }
                 hi[4 * q + i] = ((uint32_t)((int)th + (int)(l >> 24) + 0x808080)) ^ 0x808080u;
                 lo[4 * q + i] = l ^ 0x808080u;
             }
@@ -295,18 +308,23 @@ __global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
             write(g, held[0]);
         }
     }
-    int low = small | none << 16;  // k_in < 2^15
-    s_low[kg][r] = low;
-    if (tid == 0) s_flag = 0;
     __syncthreads();
+    const int n_rest = s_rests[r];
     if (kg == 0) {
-#pragma unroll
-        for (int i = 1; i < 32; ++i) low += s_low[i][r];
-        // 2^(e - 45) per unit of X, 2^-24 per unit of W, 2^8 per unit of the last group
+        // 2^(e - 45) per unit of X, 2^-24 per unit of W
         reinterpret_cast<double*>(a.ws + a.l.scale_off)[row] =
-            usual ? __builtin_bit_cast(double, (uint64_t)(e - 61 + 1023) << 52) : 0.0;
+            usual ? __builtin_bit_cast(double, (uint64_t)(e - 69 + 1023) << 52) : 0.0;
         reinterpret_cast<double*>(a.ws + a.l.norm_off)[row] = scale;
-        if (ok && !zero && (!usual || ((low & 0xffff) - (low >> 16)) * 16 > p.k_in - (low >> 16))) atomicOr(&s_flag, 1);
+        reinterpret_cast<int*>(a.ws + a.l.count_off)[row] = min(n_rest, kRests);
+        if (ok && !zero && (!usual || n_rest > kRests)) atomicOr(&s_flag, 1);
+        if (n_rest > 0) atomicOr(&s_flag, 2);
+    }
+    // in the order of k, whatever order the threads came in
+    if (kg < min(n_rest, kRests)) {
+        const Rest mine = s_rest[r][kg];
+        int rank = 0;
+        for (int i = 0; i < min(n_rest, kRests); ++i) rank += s_rest[r][i].k < mine.k;
+        reinterpret_cast<Rest*>(a.ws + a.l.rest_off)[(int64_t)row * kRests + rank] = mine;
     }
     __syncthreads();
     if (tid == 0) reinterpret_cast<int*>(a.ws + a.l.xflag_off)[blockIdx.x] = s_flag;
@@ -315,13 +333,13 @@ __global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
 // ---------------------------------------------------------------- digit products
 
 constexpr int kDigitGemmThreads = 256;
-constexpr int kGroups = 8;                 // s = i + j = -1 .. 6
+constexpr int kGroups = 9;                 // s = i + j = -1 .. 7
 constexpr int kStageK = 64;                // K of a stage: two MFMA steps
 constexpr int kStageX = 2 * 2 * kXBlk;     // 2 row blocks x 2 steps: 24 KiB
 constexpr int kStage = kStageX + 2 * 2 * 3 * kFrag;  // 2 column blocks x 2 steps, 3 digits
 
-// A 64 x 64 output tile per workgroup of 4 waves, 32 x 32 a wave. MFMA-bound: 17 products of
-// 32x32x32 a wave and step (23 with the fourth weight digit) against 9 KiB of LDS reads.
+// A 64 x 64 output tile per workgroup of 4 waves, 32 x 32 a wave. MFMA-bound: 18 products of
+// 32x32x32 a wave and step (24 with the fourth weight digit) against 9 KiB of LDS reads.
 // Stages of 64 keys stream into two LDS buffers with direct-to-LDS loads, the next stage's
 // issued between the products; the planes are stored in operand order, so both the copy and
 // the reads are linear in the lane and free of bank conflicts. Two workgroups a CU (73.7 KB
@@ -369,7 +387,8 @@ __global__ __launch_bounds__(kDigitGemmThreads, 2) void digits_gemm_kernel(Digit
     int wflag = 0;
     for (int i = 0; i < (int)a.l.parts; ++i) wflag |= wf[i];
     wflag = __builtin_amdgcn_readfirstlane(wflag);
-    const bool plain = __builtin_amdgcn_readfirstlane(xf[0] | xf[1] | xf[2] | xf[3]) != 0 || (wflag & 2) != 0;
+    const int xflag = __builtin_amdgcn_readfirstlane(xf[0] | xf[1] | xf[2] | xf[3]);
+    const bool plain = (xflag & 1) != 0 || (wflag & 2) != 0;
     const bool four = (wflag & 1) != 0;
 
     // One stage: 24 + 12 blocks of 1 KiB. x block (row block b, step q, digit i) goes to LDS
@@ -432,7 +451,6 @@ __global__ __launch_bounds__(kDigitGemmThreads, 2) void digits_gemm_kernel(Digit
                 for (int j = 0; j < 3; ++j)
 #pragma unroll
                     for (int i = 0; i < kXDigits; ++i) {
-                        if (i + j >= 7) continue;
                         acc[i + j + 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
                             f[q].x[i], f[q].w[j], acc[i + j + 1], 0, 0, 0);
                         if (!kFour && q == 0 && (n & 1) == 0 && n < 18) {
@@ -467,13 +485,43 @@ __global__ __launch_bounds__(kDigitGemmThreads, 2) void digits_gemm_kernel(Digit
     bool col_ok;
     const half_t* wrow = weight_row(p, c, col_ok);
     const int n = MODE == kDigitSwiGLU ? (c >> 5) * 16 + (c & 15) : c;
+    double sums[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        sums[i] = (double)acc[0][i];
+#pragma unroll
+        for (int s = 1; s < kGroups; ++s) sums[i] = sums[i] * 256.0 + (double)acc[s][i];
+    }
+    if (xflag & 2) {  // what the rows' digits left out, a row of the block at a time
+        const int64_t first = (int64_t)(2 * rt + wr) * kBlk;
+        const int count = reinterpret_cast<const int*>(a.ws + a.l.count_off)[first + (lane & 31)];
+        const Rest* rests = reinterpret_cast<const Rest*>(a.ws + a.l.rest_off) + first * kRests;
+        for (uint32_t left = (uint32_t)__ballot(count > 0); left != 0; left &= left - 1) {
+            const int row = __builtin_ctz(left);
+            const int n_rest = __builtin_amdgcn_readlane(count, row);
+            const Rest mine = rests[row * kRests + (lane & (kRests - 1))];
+            double sum = 0.0;
+            for (int j0 = 0; j0 < n_rest; j0 += 4) {  // 4 weights a round trip
+                float r[4], w[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int at = min(j0 + j, n_rest - 1);
+                    const int bits = __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine.r), at);
+                    r[j] = j0 + j < n_rest ? __builtin_bit_cast(float, bits) : 0.0f;
+                    w[j] = (float)wrow[__builtin_amdgcn_readlane(mine.k, at)];
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) sum += (double)r[j] * (double)(w[j] * 16777216.0f);
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                if (8 * (i >> 2) + 4 * (lane >> 5) + (i & 3) == row) sums[i] += sum;
+        }
+    }
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const int row = r0 + 8 * (i >> 2) + (i & 3);
-        double v = (double)acc[0][i];
-#pragma unroll
-        for (int s = 1; s < kGroups; ++s) v = v * 256.0 + (double)acc[s][i];
-        float y = (float)(v * scales[row]);
+        float y = (float)(sums[i] * scales[row]);
         if (plain) {
             const double ns = reinterpret_cast<const double*>(a.ws + a.l.norm_off)[row];
             const float* xr = p.x + (int64_t)min(row, p.rows - 1) * p.ldx;

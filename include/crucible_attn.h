@@ -441,11 +441,11 @@ int crucible_linear_swiglu_f64acc_prefetch(const float* x, int64_t ldx, const fl
 /* The two products with a caller-owned scratch buffer, for prompt-sized row counts: the same
  * contract on the int8 matrix cores. Both operands are written into the workspace as signed
  * 8-bit digits, the digit products accumulate exactly in int32 and join in f64. Weights keep
- * every bit; a row's activations keep every bit down to 2^-22 of the row's largest and are
- * rounded to 2^-46 of it below. Rows and columns outside the digits' range (non-finite values,
- * weights over 127, rows with a value past 2^22 or with more than one nonzero element in 16 below
- * 2^-14 of the largest) are
- * summed in f64, so outputs are the plain product's to the order of f64 summation.
+ * every bit; a row's activations keep every bit down to 2^-22 of the row's largest, and what is
+ * rounded off smaller ones is added in f64. Rows and columns outside the digits' range
+ * (non-finite values, weights over 127, rows whose largest value is outside 2^-60 .. 2^22 or
+ * with more than 16 rounded elements) are summed in f64, so outputs are the plain product's to
+ * the order of f64 summation.
  * crucible_linear_workspace_bytes gives the size (norm, swiglu: whether the call fuses them),
  * 0 where this form is not used (k_in not a multiple of 64 or above 16384, or few enough
  * rows that the plain product is faster); the plain product runs then, and also for

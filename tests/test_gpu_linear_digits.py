@@ -165,6 +165,49 @@ def test_norm_lifts_products_out_of_the_subnormals(gpu, dev, tune, size, weight)
     _check(_run(gpu, dev, x, w, nw), want)
 
 
+@pytest.mark.parametrize("small", [2.0 ** -20, 1e-8, 1e-10, 1e-12, 1e-14, 1e-30])
+@pytest.mark.parametrize("count", [1, 2, 5, 16, 17, 40])
+@pytest.mark.parametrize("norm", [False, True])
+def test_columns_that_see_only_small_elements(gpu, dev, tune, small, count, norm):
+    """`count` elements of a row far below its largest (what the digits round off, listed up to
+    16 a row, f64 sums past that), and columns whose weights are nonzero only there, one-hot
+    columns among them: the f64 sum, rounded once."""
+    tune(linear_tile=64)
+    rng = np.random.default_rng(count)
+    rows, k_in = 70, 768
+    x = rng.standard_normal((rows, k_in), dtype=np.float32)
+    x[::3] = np.abs(x[::3]) + 0.5  # rows without small elements of their own
+    w = (rng.standard_normal((96, k_in)) * 0.02).astype(np.float16)
+    at = rng.choice(k_in, count, replace=False)
+    x[1:, at] = (rng.uniform(0.5, 1.0, (rows - 1, count)) * small).astype(np.float32)
+    x[2:, at[0]] *= -1
+    keep = w[:40, at].copy()
+    w[:40] = 0
+    w[:40, at] = keep
+    w[40:50] = 0
+    w[np.arange(40, 50), at[np.arange(10) % count]] = 1
+    nw = (1 + 0.1 * rng.standard_normal(k_in)).astype(np.float32) if norm else None
+    want = (_h(x, nw) @ w.astype(np.float64).T).astype(np.float32)
+    got = _run(gpu, dev, x, w, nw)
+    _check(got, want)
+    assert np.array_equal(got, _run(gpu, dev, x, w, nw)), "not deterministic"
+
+
+@pytest.mark.parametrize("rows", [40, 130])
+def test_identity_weights_give_the_rows_back(gpu, dev, tune, rows):
+    """One-hot columns: every element of every row is an exact product by itself, whatever its
+    size beside the row's largest."""
+    tune(linear_tile=64)
+    rng = np.random.default_rng(23)
+    k_in = 512
+    x = rng.standard_normal((rows, k_in), dtype=np.float32)
+    x[1::4] *= rng.standard_normal(x[1::4].shape, dtype=np.float32) ** 2
+    x[2::4] = np.exp(x[2::4] * 3)
+    x[3::4, 7] *= 3000
+    w = np.eye(k_in, dtype=np.float16)
+    assert np.array_equal(_run(gpu, dev, x, w), x)
+
+
 def test_workspace_is_checked(gpu, dev):
     """A workspace below the size asked for is refused before any launch; a null one means the
     plain product."""
