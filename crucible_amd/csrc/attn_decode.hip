@@ -1078,16 +1078,12 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(DecodeArgs a) {
 }
 
 // ---------------------------------------------------------------- head_dim other than 64
-// One workgroup per (request, query head) through attend_generic (generic_attend.hpp).
-// ROPE (the qkv entry, f32 rows): q's pairs (i, i + hd/2) are rotated at positions[b], as
+// One workgroup per (request, query head) through attend_generic (generic_attend.hpp). With RoPE
+// tables (the qkv entry, f32 rows) q's pairs (i, i + hd/2) are rotated at positions[b], as
 // crucible_rope_split_qkv rotates them.
 template <bool QF32>
-__global__ __launch_bounds__(kGenericThreads) void decode_generic_kernel(DecodeArgs a, int hd) {
-    __shared__ GenericLds lds;
-    const int b = blockIdx.x;
-    const int h = blockIdx.y;
-    const int len = request_len(a, b);
-    if (len <= 0) return;  // inactive request: output untouched
+__device__ __forceinline__ void decode_generic_head(GenericLds& lds, const DecodeArgs& a, int hd, int b,
+                                                    int h, int len) {
     const int half = hd >> 1;
     const int64_t qoff = (int64_t)b * a.q_row_stride + (int64_t)h * hd;
     if (a.rope_cos) {
@@ -1120,6 +1116,16 @@ __global__ __launch_bounds__(kGenericThreads) void decode_generic_kernel(DecodeA
         else
             static_cast<float*>(a.out)[ooff + d] = v;
     });
+}
+
+template <bool QF32>
+__global__ __launch_bounds__(kGenericThreads) void decode_generic_kernel(DecodeArgs a, int hd) {
+    __shared__ GenericLds lds;
+    const int b = blockIdx.x;
+    const int h = blockIdx.y;
+    const int len = request_len(a, b);
+    if (len <= 0) return;  // inactive request: output untouched
+    decode_generic_head<QF32>(lds, a, hd, b, h, len);
 }
 
 // head_dim a multiple of 32 (hd_attend.hpp): a workgroup takes a split of 16 pages, a pair a wave
@@ -1220,11 +1226,9 @@ __global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 ? 4 : 1) void decode_h
         else total.merge(s[0]);
         if (sp + 1 == n_active) break;
     }
-    const int64_t out = (int64_t)b * a.out_row_stride + (int64_t)h * HD;
     const bool mine = wave == 0 && col < n_cols;
-    if (WHOLE || n_active == 1) {
-        if (mine) hd_store(a.out, a.out_f16, out, WHOLE ? total : s[0], grp);
-    } else if (mine) {
+    if constexpr (!WHOLE) {
+        if (!mine) return;
         const int64_t slot = ((int64_t)b * a.n_head + h) * a.n_splits + s0;
 #pragma unroll
         for (int i = 0; i < HD / 16; ++i)
@@ -1233,48 +1237,81 @@ __global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 ? 4 : 1) void decode_h
             a.pm[slot] = s[0].m;
             a.pl[slot] = s[0].l;
         }
+    } else {
+        __shared__ GenericLds again;
+        __shared__ uint32_t s_again;
+        if (wave == 0) {
+            const uint32_t cols = hd_not_finite(total, mine);
+            if (lane == 0) s_again = cols;
+        }
+        if (mine) hd_store(a.out, a.out_f16, (int64_t)b * a.out_row_stride + (int64_t)h * HD, total, grp);
+        __syncthreads();
+        for (uint32_t left = s_again; left != 0; left &= left - 1) {
+            const DecodeArgs& c = cold_args<DecodeArgs>();
+            decode_generic_head<QF32>(again, c, HD, blockIdx.y, g * c.n_rep + c0 + __builtin_ctz(left), len);
+        }
     }
 }
 
-// Joins the splits' partials in order, one thread per (request, query head, 4 dims).
-__global__ __launch_bounds__(256) void decode_hd_combine_kernel(DecodeArgs a, int hd) {
+// Joins the splits' partials in order, one thread per (request, query head, 4 dims), whole rows
+// a workgroup. Rows that come out with an infinity or a NaN are attended once more by
+// decode_generic_head: a visible infinity times a weight's zero lo half leaves NaN where the f32
+// product is infinite.
+template <bool QF32>
+__global__ __launch_bounds__(kGenericThreads) void decode_hd_combine_kernel(DecodeArgs a, int hd) {
+    __shared__ GenericLds again;
+    __shared__ uint32_t s_again;  // of the workgroup's rows, at most 32
     const int quads = hd >> 2;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (int64_t)a.batch * a.n_head * quads) return;
-    const int64_t row = i / quads;  // b * n_head + h
-    const int d = 4 * (int)(i - row * quads);
-    const int b = (int)(row / a.n_head);
-    const int64_t slot = row * a.n_splits;
-    // The first splits' partials are requested beside the length, whether or not it reaches
-    // them (those it does not are not used).
-    constexpr int kAhead = 8;  // splits a round trip
-    HdState<16> t[kAhead];
-    auto load = [&](int j0) {
+    const int rows = kGenericThreads / quads;
+    const int mine = threadIdx.x / quads;
+    const int64_t row0 = (int64_t)blockIdx.x * rows;
+    const int64_t row = row0 + mine;  // b * n_head + h
+    if (threadIdx.x == 0) s_again = 0;
+    __syncthreads();
+    if (mine < rows && row < (int64_t)a.batch * a.n_head) {
+        const int d = 4 * (threadIdx.x - mine * quads);
+        const int b = (int)(row / a.n_head);
+        const int64_t slot = row * a.n_splits;
+        // The first splits' partials are requested beside the length, whether or not it reaches
+        // them (those it does not are not used).
+        constexpr int kAhead = 8;  // splits a round trip
+        HdState<16> t[kAhead];
+        auto load = [&](int j0) {
 #pragma unroll
-        for (int j = 0; j < kAhead; ++j) {
-            const int64_t at = slot + min(j0 + j, a.n_splits - 1);
-            t[j].m = a.pm[at];
-            t[j].l = a.pl[at];
-            t[j].o[0] = *reinterpret_cast<const float4_t*>(a.po + at * hd + d);
-        }
-    };
-    load(0);
-    const int len = request_len(a, b);
-    if (len <= 0) return;
-    const int n_active = ((len + kPageMask) / kPageTokens + kHdSplitPages - 1) / kHdSplitPages;
-    if (n_active == 1) return;  // written by its only split
-    HdState<16> total;  // one quad of dims
-    for (int j0 = 0; j0 < n_active; j0 += kAhead) {
-        if (j0 > 0) load(j0);
+            for (int j = 0; j < kAhead; ++j) {
+                const int64_t at = slot + min(j0 + j, a.n_splits - 1);
+                t[j].m = a.pm[at];
+                t[j].l = a.pl[at];
+                t[j].o[0] = *reinterpret_cast<const float4_t*>(a.po + at * hd + d);
+            }
+        };
+        load(0);
+        const int len = request_len(a, b);
+        if (len > 0) {
+            const int n_active = ((len + kPageMask) / kPageTokens + kHdSplitPages - 1) / kHdSplitPages;
+            HdState<16> total;  // one quad of dims
+            for (int j0 = 0; j0 < n_active; j0 += kAhead) {
+                if (j0 > 0) load(j0);
 #pragma unroll
-        for (int j = 0; j < kAhead; ++j) {
-            if (j0 + j >= n_active) break;
-            if (j0 + j == 0) total = t[0];
-            else total.merge(t[j]);
+                for (int j = 0; j < kAhead; ++j) {
+                    if (j0 + j >= n_active) break;
+                    if (j0 + j == 0) total = t[0];
+                    else total.merge(t[j]);
+                }
+            }
+            const float4_t v = total.o[0] * (1.0f / total.l);
+            store_out4(a, (int64_t)b * a.out_row_stride + (row - (int64_t)b * a.n_head) * hd + d, v);
+            const float z = ((v[0] * 0.0f + v[1] * 0.0f) + v[2] * 0.0f) + v[3] * 0.0f;
+            if (!(z == 0.0f)) atomicOr(&s_again, 1u << mine);
         }
     }
-    store_out4(a, (int64_t)b * a.out_row_stride + (row - (int64_t)b * a.n_head) * hd + d,
-               total.o[0] * (1.0f / total.l));
+    __syncthreads();
+    for (uint32_t left = s_again; left != 0; left &= left - 1) {
+        const DecodeArgs& c = cold_args<DecodeArgs>();
+        const int64_t at = (int64_t)blockIdx.x * rows + __builtin_ctz(left);
+        const int b = (int)(at / c.n_head);
+        decode_generic_head<QF32>(again, c, hd, b, (int)(at - (int64_t)b * c.n_head), request_len(c, b));
+    }
 }
 
 // The fused entries' two appends for head_dim other than 64: row b's K (rotated at positions[b]
@@ -1587,9 +1624,12 @@ int launch_decode_generic(DecodeArgs a, int hd, bool q_f32, void* workspace,
         }
         if (const int rc = fail_launch(what)) return rc;
         if (!a.po) return CRUCIBLE_OK;
-        const int64_t threads = (int64_t)a.batch * a.n_head * (hd / 4);
-        hipLaunchKernelGGL(decode_hd_combine_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256),
-                           0, stream, a, hd);
+        const int64_t rows = kGenericThreads / (hd / 4);  // a workgroup
+        const dim3 grid((unsigned)(((int64_t)a.batch * a.n_head + rows - 1) / rows));
+        if (q_f32)
+            hipLaunchKernelGGL(decode_hd_combine_kernel<true>, grid, dim3(kGenericThreads), 0, stream, a, hd);
+        else
+            hipLaunchKernelGGL(decode_hd_combine_kernel<false>, grid, dim3(kGenericThreads), 0, stream, a, hd);
         return fail_launch(what);
     }
     const dim3 grid((unsigned)a.batch, (unsigned)a.n_head);

@@ -1696,16 +1696,13 @@ void launch_kb(const PrefillArgs& a, int kb, dim3 grid, hipStream_t stream) {
 // through the same row modes (tile_row) and, for hybrid segments, the chunk's own K/V rows
 // from the segment's absolute start.
 template <bool QF32>
-__global__ __launch_bounds__(kGenericThreads) void prefill_generic_kernel(PrefillArgs a, int hd,
-                                                                          int64_t rows_y) {
-    __shared__ GenericLds lds;
-    const int h = blockIdx.x;
-    const int64_t req = blockIdx.z;
-    const int64_t stride = (int64_t)a.n_head * hd;
+__device__ __forceinline__ void prefill_generic_row(GenericLds& lds, const PrefillArgs& a, int hd, int h,
+                                                    int64_t req, int row, int owner, int pos) {
     GenericKeys ks{};
     ks.k_pool = a.k_pool;
     ks.v_pool = a.v_pool;
     ks.addr = a.addr;
+    ks.table = a.tables ? a.tables + (int64_t)owner * a.table_stride : nullptr;
     ks.g = h / a.n_rep;
     ks.hd = hd;
     ks.astart = INT32_MAX;
@@ -1716,22 +1713,30 @@ __global__ __launch_bounds__(kGenericThreads) void prefill_generic_kernel(Prefil
         ks.cur_k = a.cur_k;
         ks.cur_v = a.cur_v;
     }
+    const int64_t qoff = ((int64_t)row * a.n_head + h) * hd;
+    for (int d = threadIdx.x; d < hd; d += kGenericThreads)
+        lds.q[d] = QF32 ? static_cast<const float*>(a.q)[qoff + d]
+                        : (float)static_cast<const half_t*>(a.q)[qoff + d];
+    __syncthreads();
+    attend_generic(lds, ks, pos + 1, a.scale_log2, [&](int d, float v) {
+        if (a.out_f16)
+            static_cast<half_t*>(a.out)[qoff + d] = (half_t)v;
+        else
+            static_cast<float*>(a.out)[qoff + d] = v;
+    });
+}
+
+template <bool QF32>
+__global__ __launch_bounds__(kGenericThreads) void prefill_generic_kernel(PrefillArgs a, int hd,
+                                                                          int64_t rows_y) {
+    __shared__ GenericLds lds;
+    const int h = blockIdx.x;
+    const int64_t req = blockIdx.z;
     for (int64_t local = blockIdx.y; local < rows_y; local += gridDim.y) {
         int row, owner, pos;
         tile_row(a, req, local, row, owner, pos);
         if (row < 0) continue;  // uniform: the same row for the whole workgroup
-        const int64_t qoff = (int64_t)row * stride + (int64_t)h * hd;
-        for (int d = threadIdx.x; d < hd; d += kGenericThreads)
-            lds.q[d] = QF32 ? static_cast<const float*>(a.q)[qoff + d]
-                            : (float)static_cast<const half_t*>(a.q)[qoff + d];
-        __syncthreads();
-        ks.table = a.tables ? a.tables + (int64_t)owner * a.table_stride : nullptr;
-        attend_generic(lds, ks, pos + 1, a.scale_log2, [&](int d, float v) {
-            if (a.out_f16)
-                static_cast<half_t*>(a.out)[qoff + d] = (half_t)v;
-            else
-                static_cast<float*>(a.out)[qoff + d] = v;
-        });
+        prefill_generic_row<QF32>(lds, a, hd, h, req, row, owner, pos);
     }
 }
 
@@ -1749,6 +1754,9 @@ __global__ __launch_bounds__(kGenericThreads) void prefill_generic_kernel(Prefil
 template <int HD, int W, int QB, bool QF32, bool HYB>
 __global__ __launch_bounds__(64 * W, W == 8 ? 4 : 1) void prefill_hd_kernel(PrefillArgs a) {
     __shared__ HdLds<HD, W, QB> lds;
+    __shared__ GenericLds again;
+    __shared__ uint32_t s_again[QB];
+    __shared__ int s_row[16 * QB], s_owner[16 * QB], s_pos[16 * QB];
     const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = blockIdx.x;
@@ -1765,6 +1773,9 @@ __global__ __launch_bounds__(64 * W, W == 8 ? 4 : 1) void prefill_hd_kernel(Pref
         any |= pending[b];
     }
     if (__ballot(any) == 0) return;  // the same rows in every wave
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int b = 0; b < QB; ++b) s_again[b] = 0;
 #pragma unroll
     for (int b = 0; b < QB; ++b) {
         float x[HD / 32][8];
@@ -1786,7 +1797,7 @@ __global__ __launch_bounds__(64 * W, W == 8 ? 4 : 1) void prefill_hd_kernel(Pref
                 found = true;
             }
         }
-        if (!found) return;
+        if (!found) break;
         int see[QB];  // last key the column sees
 #pragma unroll
         for (int b = 0; b < QB; ++b) {
@@ -1838,14 +1849,8 @@ __global__ __launch_bounds__(64 * W, W == 8 ? 4 : 1) void prefill_hd_kernel(Pref
             page0 = page_of(p + 2 * W);  // beside the K/V loads, not before the next ones
             page1 = page_of(p + 2 * W + 1);
             const int key0 = p * kPageTokens;
-            if constexpr (kMask) {
+            if constexpr (kMask)
                 if (key0 + 2 * kPageTokens > last + 1) kv.zero_tail(key0, last + 1, grp);
-                if (__ballot(kv.v_not_finite()) != 0) {
-#pragma unroll
-                    for (int b = 0; b < QB; ++b) hd_spoil(s[b], kv, key0, see[b], grp);
-                    kv.zero_not_finite();
-                }
-            }
 #pragma unroll
             for (int b = 0; b < QB; ++b)
                 hd_attend_pair<HD, QF32, kMask>(s[b], q[b], kv, key0, see[b], grp);
@@ -1855,10 +1860,30 @@ __global__ __launch_bounds__(64 * W, W == 8 ? 4 : 1) void prefill_hd_kernel(Pref
         hd_merge_waves<HD, W, QB>(lds, s, wave, col, grp, 16 * QB);
         if (wave == 0)
 #pragma unroll
-            for (int b = 0; b < QB; ++b)
-                if (see[b] >= 0)
+            for (int b = 0; b < QB; ++b) {
+                const uint32_t cols = hd_not_finite(s[b], see[b] >= 0);
+                if (lane == 0) s_again[b] |= cols;
+                if (see[b] >= 0 && grp == 0) {
+                    s_pos[16 * b + col] = see[b];
+                    s_owner[16 * b + col] = who;
+                }
+                if (see[b] >= 0 && !(cols >> col & 1))
                     hd_store(a.out, a.out_f16, (int64_t)row[b] * stride + (int64_t)h * HD, s[b], grp);
+            }
     }
+    // Rows whose state was not finite (an infinite or NaN V value that they see, or that a later
+    // row of the tile sees) are attended once more on their own.
+    if (wave == 0 && grp == 0)
+#pragma unroll
+        for (int b = 0; b < QB; ++b) s_row[16 * b + col] = row[b];
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < QB; ++b)
+        for (uint32_t left = s_again[b]; left != 0; left &= left - 1) {
+            const int c = 16 * b + __builtin_ctz(left);
+            prefill_generic_row<QF32>(again, cold_args<PrefillArgs>(), HD, (int)blockIdx.x, blockIdx.z,
+                                      s_row[c], s_owner[c], s_pos[c]);
+        }
 }
 
 template <int HD, int W, int QB>

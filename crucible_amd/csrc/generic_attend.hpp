@@ -4,15 +4,16 @@
 // steps of the warp). The MFMA kernels of attn_decode.hip / attn_prefill.hip are built for
 // head_dim 64, the dimension of every preset; hd_attend.hpp has those of the other multiples of
 // 32. The remaining dimensions (multiples of 8 up to 256), and calls whose buffers are not
-// 16-byte aligned, run through this workgroup-level routine instead: plain wave64 code, f32 accumulation,
-// fp16 K/V read from the same pool layout, online softmax in base 2.
+// 16-byte aligned, run through this workgroup-level routine instead: plain wave64 code, f32
+// accumulation, fp16 K/V read from the same pool layout, online softmax in base 2. The kernels of
+// hd_attend.hpp come back to it for outputs that are not finite.
 //
 // One workgroup of kGenericThreads threads attends one (query row, query head) over keys
-// [0, n). Wave w takes the 64-key blocks w, w + 4, ...: lane k scores key 64 * blk + k
-// (q from LDS, its K row in 16-byte loads), the wave's max and sum come from lane
-// shuffles, and for the P.V product the lanes switch to dimensions (lane d holds dims d,
-// d + 64, ...) and read each page's V^T rows (16 contiguous slots per dimension). The four
-// wave states merge through LDS at the end.
+// [0, n); the threads of a larger one past these only pass its barriers. Wave w takes the
+// 64-key blocks w, w + 4, ...: lane k scores key 64 * blk + k (q from LDS, its K row in 16-byte
+// loads), the wave's max and sum come from lane shuffles, and for the P.V product the lanes
+// switch to dimensions (lane d holds dims d, d + 64, ...) and read each page's V^T rows (16
+// contiguous slots per dimension). The four wave states merge through LDS at the end.
 #pragma once
 
 #include "common.hpp"
@@ -80,7 +81,7 @@ __device__ void attend_generic(GenericLds& lds, const GenericKeys& ks, int n, fl
     float m = -INFINITY;  // running max, log2-scaled
     float l = 0.0f;
     float o[kGenericMaxHeadDim / 64] = {};
-    for (int blk = wave; blk * 64 < n; blk += kGenericWaves) {
+    for (int blk = wave; blk * 64 < n && wave < kGenericWaves; blk += kGenericWaves) {
         const int key0 = blk * 64;
         // scores: lane k takes key key0 + k
         const int j = key0 + lane;
@@ -166,14 +167,14 @@ __device__ void attend_generic(GenericLds& lds, const GenericKeys& ks, int n, fl
     }
     // Merge the waves. A wave without keys has m = -inf, l = 0 and o = 0: weight 0. Wave 0
     // holds key 0, so the merged max is finite.
-    if (lane == 0) {
+    if (lane == 0 && wave < kGenericWaves) {
         lds.m[wave] = m;
         lds.l[wave] = l;
     }
 #pragma unroll
     for (int i = 0; i < kGenericMaxHeadDim / 64; ++i) {
         const int d = lane + 64 * i;
-        if (d < hd) lds.o[wave][d] = o[i];
+        if (d < hd && wave < kGenericWaves) lds.o[wave][d] = o[i];
     }
     __syncthreads();
     for (int d = threadIdx.x; d < hd; d += kGenericThreads) {

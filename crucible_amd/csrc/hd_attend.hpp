@@ -14,7 +14,9 @@
 //   one online-softmax update in base 2 for its 8 scores
 //   O^T[HD x 16] += V^T . P^T, HD / 16 blocks x (hi, lo); the lane's 8 scores are the k range
 //     8 grp .. +7 of the step, its V^T operand the two pages' quarters side by side
-// The waves' states then merge through LDS in halving rounds.
+// The waves' states then merge through LDS in halving rounds. Infinite or NaN values do not
+// survive masks (0 times an infinity is NaN) and hi + lo operands; a row that does not come out
+// finite goes through attend_generic again, on its own.
 #pragma once
 
 #include "common.hpp"
@@ -40,6 +42,14 @@ struct HdState {
         for (int d = 0; d < HD / 16; ++d) o[d] = float4_t{0.f, 0.f, 0.f, 0.f};
         m = -INFINITY;
         l = 0.0f;
+    }
+    template <class Lds>
+    __device__ __forceinline__ void read(const Lds& lds, int slot, int c, int grp) {
+#pragma unroll
+        for (int i = 0; i < HD / 16; ++i)
+            o[i] = *reinterpret_cast<const float4_t*>(&lds.o[slot][c][16 * i + 4 * grp]);
+        m = lds.m[slot][c];
+        l = lds.l[slot][c];
     }
     // Joins another state. Empty states (m = -inf, l = 0, o = 0) have weight 0.
     __device__ __forceinline__ void merge(const HdState& s) {
@@ -153,30 +163,6 @@ struct HdPair {
 #pragma unroll
                     for (int i = 0; i < HD / 16; ++i) v[p][i][r] = (half_t)0.0f;
     }
-    // Whether the lane holds an infinite or NaN V value.
-    __device__ __forceinline__ bool v_not_finite() const {
-        // an exponent of all ones carries into its half's top bit
-        uint32_t bad = 0;
-#pragma unroll
-        for (int p = 0; p < 2; ++p)
-#pragma unroll
-            for (int i = 0; i < HD / 16; ++i) {
-                struct Words { uint32_t w[2]; };
-                const Words x = __builtin_bit_cast(Words, v[p][i]);
-                bad |= ((x.w[0] & 0x7c007c00u) + 0x04000400u) | ((x.w[1] & 0x7c007c00u) + 0x04000400u);
-            }
-        return (bad & 0x80008000u) != 0;
-    }
-    __device__ __forceinline__ void zero_not_finite() {
-#pragma unroll
-        for (int p = 0; p < 2; ++p)
-#pragma unroll
-            for (int i = 0; i < HD / 16; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if ((__builtin_bit_cast(uint16_t, (half_t)v[p][i][r]) & 0x7c00) == 0x7c00)
-                        v[p][i][r] = (half_t)0.0f;
-    }
 };
 
 // One pair into a column block's state: the column sees keys up to `last` (-1: none), or the
@@ -233,31 +219,6 @@ __device__ __forceinline__ void hd_attend_pair(HdState<HD>& s, const HdQuery<HD,
     }
 }
 
-// A masked key's weight of 0 does not cancel an infinite or NaN V. Where a pair has such values
-// and some columns see only a part of it, this makes the outputs NaN whose column sees one (the
-// count of those is a product of two 0/1 operands), and the values are zeroed before
-// hd_attend_pair.
-template <int HD>
-__device__ __forceinline__ void hd_spoil(HdState<HD>& s, const HdPair<HD>& kv, int key0, int last,
-                                         int grp) {
-    half8_t sees;
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-        sees[e] = key0 + 16 * (e >> 2) + 4 * grp + (e & 3) <= last ? (half_t)1.0f : (half_t)0.0f;
-#pragma unroll
-    for (int i = 0; i < HD / 16; ++i) {
-        half8_t bad;
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-            bad[e] = (__builtin_bit_cast(uint16_t, (half_t)kv.v[e >> 2][i][e & 3]) & 0x7c00) == 0x7c00
-                         ? (half_t)1.0f : (half_t)0.0f;
-        const float4_t n = mfma_16x16x32(bad, sees, float4_t{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (n[r] > 0.0f) s.o[i][r] = __builtin_nanf("");
-    }
-}
-
 // The merge buffer: states of half the waves, padded so that the 16 columns of a block start in
 // different banks.
 template <int HD, int W, int QB>
@@ -296,16 +257,33 @@ __device__ __forceinline__ void hd_merge_waves(HdLds<HD, W, QB>& lds, HdState<HD
                 const int c = 16 * b + col;
                 if (c >= n_cols) continue;
                 HdState<HD> t;
-#pragma unroll
-                for (int i = 0; i < HD / 16; ++i)
-                    t.o[i] = *reinterpret_cast<const float4_t*>(&lds.o[wave][c][16 * i + 4 * grp]);
-                t.m = lds.m[wave][c];
-                t.l = lds.l[wave][c];
+                t.read(lds, wave, c, grp);
                 s[b].merge(t);
             }
         }
         __syncthreads();
     }
+}
+
+// The columns, as bits, whose merged state holds an infinity or a NaN (0 times it is not 0).
+template <int HD>
+__device__ __forceinline__ uint32_t hd_not_finite(const HdState<HD>& s, bool mine) {
+    float z = s.l * 0.0f;
+#pragma unroll
+    for (int i = 0; i < HD / 16; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z = __builtin_fmaf(s.o[i][r], 0.0f, z);
+    const uint64_t bad = __ballot(mine && !(z == 0.0f));
+    return (uint32_t)(bad | bad >> 16 | bad >> 32 | bad >> 48) & 0xffffu;
+}
+
+// The kernel's first argument read from the argument block where it is used, in a branch that
+// hardly runs: its fields would otherwise stay in scalar registers through the main loop.
+template <class Args>
+__device__ __forceinline__ const Args& cold_args() {
+    const void* p = (const void*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *static_cast<const Args*>(p);
 }
 
 // 8 consecutive values of a query row as f32.

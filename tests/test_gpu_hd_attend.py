@@ -188,6 +188,86 @@ def test_prefill_rows_before_an_infinite_value(gpu, dev, hd, bad):
     assert float((got[~sees] - want[~sees]).abs().max()) <= TOL
 
 
+def _same_special(got, want):
+    """NaN and infinities in the same places, the rest to TOL."""
+    assert torch.equal(got.isnan(), want.isnan())
+    inf = want.isinf()
+    assert torch.equal(got.isinf(), inf) and torch.equal(got[inf], want[inf])
+    fine = want.isfinite()
+    assert float((got[fine] - want[fine]).abs().max()) <= TOL
+
+
+def _spoil(pools, tables, layer, kv, request, key, what, value):
+    """`value` into one key of a request: its whole V row, the first half of it, or one K element."""
+    page = tables[request, key // 16].long()
+    if what == "k":
+        pools[0].view(-1, 2, 16, kv)[page, layer, key % 16, ::32] = value
+    else:
+        pools[1].view(-1, 2, kv, 16)[page, layer, :kv // (2 if what == "half" else 1), key % 16] = value
+
+
+SPECIAL = [("v", 3, float("inf")), ("half", 290, float("-inf")), ("half", 40, float("nan")),
+           ("k", 5, float("inf")), ("k", 299, float("-inf"))]
+
+
+@pytest.mark.parametrize("hd", [32, 96, 128, 160, 192, 224, 256])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("what,key,value", SPECIAL)
+def test_decode_of_infinite_values(gpu, dev, hd, dtype, what, key, value):
+    """A visible infinity gives what the generic kernels' f32 sums give: an infinite V value an
+    infinite output, and NaN only where they have one."""
+    from crucible_amd import _lib
+    lib = _lib.load()
+    lens, n_head, n_kv, layer = [300, 70, 600, 17], 4, 2, 1
+    g, stride, kv, pools, tables, q = _case(dev, hd + 7, hd, n_head, n_kv, lens, dtype=dtype)
+    _spoil(pools, tables, layer, kv, 0, key, what, value)
+    _spoil(pools, tables, layer, kv, 2, key, what, value)
+    _spoil(pools, tables, layer, kv, 2, 555, "half", float("inf"))
+    d_len = torch.tensor(lens, dtype=torch.int32, device=dev)
+    outs = []
+    for x in (q, _unaligned(q)):
+        out = torch.full((4, n_head * hd), 7.0, device=dev)
+        gpu.attention_decode_paged(x, *pools, out, tables, d_len, 4, n_head, n_kv, hd, stride, 2, layer,
+                                   kv, stride * 16)
+        outs.append(out)
+    _same_special(*outs)
+    alone = torch.full_like(outs[0], 7.0)
+    _lib.check(lib.crucible_attention_decode_paged(
+        q.data_ptr(), 0 if dtype == torch.float32 else 1, pools[0].data_ptr(), pools[1].data_ptr(),
+        alone.data_ptr(), 0, tables.data_ptr(), d_len.data_ptr(), 4, n_head, n_kv, hd, stride, 2,
+        layer, kv, stride * 16, None, 0, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(alone.nan_to_num(nan=5.0), outs[0].nan_to_num(nan=5.0))
+
+
+@pytest.mark.parametrize("hd", [32, 96, 128, 160, 192, 224, 256])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("hybrid", [False, True])
+@pytest.mark.parametrize("what,key,value", SPECIAL)
+def test_prefill_of_infinite_values(gpu, dev, hd, dtype, hybrid, what, key, value):
+    """The same for prefill rows before, at and after the key, in pairs of pages that a tile's
+    rows see whole and in part; hybrid chunks also bring a V value past fp16's range."""
+    starts, lens = [250, 0], [60, 45]
+    n_head, n_kv, layer = 4, 2, 1
+    g, stride, kv, pools, tables, _ = _case(dev, hd + 9, hd, n_head, n_kv,
+                                            [s + n for s, n in zip(starts, lens)])
+    _spoil(pools, tables, layer, kv, 0, key, what, value)
+    if key < 45:
+        _spoil(pools, tables, layer, kv, 1, key, what, value)
+    rows = sum(lens)
+    segments = torch.tensor([[0, lens[0], starts[0], 0], [lens[0], lens[1], starts[1], 1]],
+                            dtype=torch.int32, device=dev)
+    q = torch.randn(rows, n_head * hd, generator=g, device=dev).to(dtype)
+    cur = [torch.randn(rows, kv, generator=g, device=dev) for _ in "kv"]
+    cur[1][40, :kv // 4] = 1e6
+    outs = []
+    for x in (q, _unaligned(q)):
+        out = torch.full((rows, n_head * hd), 7.0, device=dev)
+        gpu.attention_prefill_tiled(x, *pools, *(cur if hybrid else (None, None)), out, tables, segments,
+                                    2, max(lens), stride, n_head, n_kv, hd, 2, layer, kv, hybrid=hybrid)
+        outs.append(out)
+    _same_special(*outs)
+
+
 def test_large_and_tiny_f32_queries(gpu, dev):
     """f32 queries outside fp16's range: the operands are scaled by a power of two."""
     hd, n_head, n_kv, lens = 128, 4, 2, [70, 33]
