@@ -85,11 +85,10 @@ struct HdQuery {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(x[k][i]));
             mx = group_max4(mx);
-            const int e = (int)(__builtin_bit_cast(uint32_t, mx) >> 23) - 127;
-            if (e >= -90 && e <= 90) {
-                up = __builtin_bit_cast(float, (uint32_t)(8 - e + 127) << 23);
-                scale *= __builtin_bit_cast(float, (uint32_t)(e - 8 + 127) << 23);
-            }
+            // up to the largest f32; smaller than 2^-118, both powers of two would not be normal
+            const int e = min(max((int)(__builtin_bit_cast(uint32_t, mx) >> 23) - 127, -118), 127);
+            up = __builtin_bit_cast(float, (uint32_t)(8 - e + 127) << 23);
+            scale *= __builtin_bit_cast(float, (uint32_t)(e - 8 + 127) << 23);
         }
 #pragma unroll
         for (int k = 0; k < HD / 32; ++k)
@@ -198,7 +197,13 @@ __device__ __forceinline__ void hd_attend_pair(HdState<HD>& s, const HdQuery<HD,
     for (int p = 0; p < 2; ++p) {
         float pf[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) pf[r] = fast_exp2(__builtin_fmaf(st[p][r], q.scale, -at));
+        for (int r = 0; r < 4; ++r) {
+            // rounded as the largest score was, so the difference is at most 0 (an FMA's is not,
+            // and past 2^28 its weight leaves fp16's range)
+#pragma clang fp contract(off)
+            const float t = st[p][r] * q.scale;
+            pf[r] = fast_exp2(t - at);
+        }
         sum += (pf[0] + pf[1]) + (pf[2] + pf[3]);
         const uint32_t h01 = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(pf[0], pf[1]));
         const uint32_t h23 = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(pf[2], pf[3]));

@@ -287,6 +287,38 @@ def test_large_and_tiny_f32_queries(gpu, dev):
         assert float((outs[0] - outs[1]).abs().max()) <= (1e-4 if factor > 1 else TOL)
 
 
+@pytest.mark.parametrize("hd", [32, 128])
+@pytest.mark.parametrize("power", [-140, -119, -100, 22, 26, 28, 30, 40, 80, 91, 110, 119])
+def test_f32_queries_over_the_whole_range(gpu, dev, hd, power):
+    """Scores past 2^18 put all the weight on the largest, scores below 2^-80 weigh every key the
+    same: either way the outputs are the generic kernels' (their largest two scores are 2^-12
+    apart or more), in decode and in prefill."""
+    n_head, n_kv, lens = 4, 2, [70, 33]
+    g, stride, kv, (kp, vp), tables, q = _case(dev, 5, hd, n_head, n_kv, lens)
+    q = torch.ldexp(q, torch.tensor(power, device=dev)) if power > -126 else \
+        torch.ldexp(torch.ldexp(q, torch.tensor(-100, device=dev)), torch.tensor(power + 100, device=dev))
+    assert q.isfinite().all() and bool((q != 0).any())
+    if power > 0:
+        k = kp.view(-1, 2, 16, n_kv, hd)
+        for b, n in enumerate(lens):
+            keys = k[tables[b].long(), 0].reshape(-1, n_kv, hd)[:n].double()
+            s = (q[b].double().view(1, n_head, hd) * keys.repeat_interleave(2, 1)).sum(2).t().sort(1).values
+            assert bool(((s[:, -1] - s[:, -2]) > s.abs().amax(1) * 2.0 ** -12).all())
+    d_len = torch.tensor(lens, dtype=torch.int32, device=dev)
+    d_own = torch.tensor([0, 1], dtype=torch.int32, device=dev)
+    outs = []
+    for x in (q, _unaligned(q)):
+        a, b = torch.zeros(2, n_head * hd, device=dev), torch.zeros(2, n_head * hd, device=dev)
+        gpu.attention_decode_paged(x, kp, vp, a, tables, d_len, 2, n_head, n_kv, hd, stride, 2, 0, kv,
+                                   stride * 16)
+        gpu.attention_prefill_packed(x, kp, vp, b, tables, d_own, d_len - 1, 2, stride, n_head, n_kv, hd,
+                                     2, 0, kv, stride * 16)
+        outs.append((a, b))
+    for got, want in zip(*outs):
+        assert want.isfinite().all()
+        assert float((got - want).abs().max()) <= TOL
+
+
 @pytest.mark.parametrize("hd", [128, 256])
 def test_workspace_shared_with_head_dim_64(gpu, dev, hd):
     """Calls of other head dimensions leave the counters and the unit plan of a workspace alone,
