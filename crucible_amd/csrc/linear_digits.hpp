@@ -264,7 +264,8 @@ __global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
     // Usual magnitudes only: every power of two below is a normal f32, and the scaling up exact.
     // x * norm_w below the normal range bounds nothing: the row's scale may lift h out of it.
     const bool usual = mx >= 0x00800000u && mx < 0x7f800000u && e >= -60 && e <= 21;  // up >= 1
-    const bool zero = mx == 0 && (!NORM || tot == 0.0);
+    // a zero row stays one unless eps lets its scale be infinite
+    const bool zero = mx == 0 && (!NORM || (tot == 0.0 && scale < (double)INFINITY));
     const float up = usual ? __builtin_bit_cast(float, (uint32_t)(21 - e + 127) << 23) : 0.0f;
     unsigned char* blk = a.ws + (int64_t)(row >> 5) * steps * kXBlk + (row & 31) * 16;
     auto write = [&](int g, const Group& v) {

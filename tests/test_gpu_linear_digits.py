@@ -193,6 +193,26 @@ def test_columns_that_see_only_small_elements(gpu, dev, tune, small, count, norm
     assert np.array_equal(got, _run(gpu, dev, x, w, nw)), "not deterministic"
 
 
+@pytest.mark.parametrize("eps", [0.0, 1e-6])
+def test_zero_rows_under_the_norm(gpu, dev, tune, eps):
+    """A zero row normalised with eps = 0 is 0 times infinity, NaN as in the f64 forms; other
+    rows of its block are untouched."""
+    x = torch.randn(40, 128, device=dev)
+    x[7] = 0
+    w = torch.randn(64, 128, device=dev).mul_(0.02).half()
+    nw = torch.ones(128, device=dev)
+    outs = []
+    for tile in (64, 32):
+        tune(linear_tile=tile)
+        out = torch.zeros(40, 64, device=dev)
+        gpu.linear_f64acc(x, w, out, norm_w=nw, eps=eps)
+        outs.append(out)
+    assert bool(outs[1][7].isnan().all()) == (eps == 0.0)
+    assert torch.equal(outs[0].isnan(), outs[1].isnan())
+    d = _ulps(*(o.nan_to_num(nan=0.0).cpu().numpy() for o in outs))
+    assert d.max() <= 1
+
+
 @pytest.mark.parametrize("rows", [40, 130])
 def test_identity_weights_give_the_rows_back(gpu, dev, tune, rows):
     """One-hot columns: every element of every row is an exact product by itself, whatever its
