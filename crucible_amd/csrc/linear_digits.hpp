@@ -257,8 +257,9 @@ __global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
         mx = max(mx, s_mx[i][r]);
     }
     const double scale = NORM ? 1.0 / sqrt(tot / (double)p.k_in + p.eps) : 1.0;
-    // |h| <= bound (1 + 2^-18 covers the roundings of h), so |h| 2^(21 - e) < 2^22 with e
-    // the exponent of 2^e > bound / 2
+    // |h| <= bound (1 + 2^-18 covers the roundings of h, unless x * scale is subnormal: those
+    // rows are found by their values below), so |h| 2^(21 - e) < 2^22 with e the exponent of
+    // 2^e > bound / 2
     const float bound = (float)((double)__builtin_bit_cast(float, mx) * scale * 1.00001);
     const int e = (int)((__builtin_bit_cast(uint32_t, bound) >> 23) & 255) - 127;
     // Usual magnitudes only: every power of two below is a normal f32, and the scaling up exact.
@@ -277,6 +278,8 @@ __global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
                 float h = v.x[q][i];
                 if constexpr (NORM) h = (float)((double)h * scale) * v.nw[q][i];
                 const float t = ok && usual ? h * up : 0.0f;        // exact
+                if constexpr (NORM)
+                    if (fabsf(t) >= 4194304.0f) s_flag = 1;
                 const float th = rintf(t);
                 const float tl = (t - th) * 16777216.0f;            // exact, |tl| <= 2^23
                 const float tr = rintf(tl);                         // rounds below 2^-22 of the largest

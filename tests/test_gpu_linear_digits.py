@@ -228,6 +228,25 @@ def test_identity_weights_give_the_rows_back(gpu, dev, tune, rows):
     assert np.array_equal(_run(gpu, dev, x, w), x)
 
 
+def test_subnormal_rows_that_round_past_the_bound(gpu, dev, tune):
+    """x * scale = 0.5000001 steps of f32's smallest rounds up to one, and a huge norm weight
+    lifts it: twice what x * norm_w * scale says."""
+    tune(linear_tile=64)
+    eps = np.float32(3.999999)
+    x = np.full((40, 64), 2.0 ** -149, np.float32)
+    x[::3, ::5] *= -1
+    nw = np.full(64, 1.99995 * 2.0 ** 99, np.float32)
+    w = np.random.default_rng(29).uniform(0.5, 1, (40, 64)).astype(np.float16)
+    x64 = x.astype(np.float64)
+    scale = 1.0 / np.sqrt((x64 * x64).mean(axis=1, keepdims=True) + np.float64(eps))
+    h = (x64 * scale).astype(np.float32) * nw
+    assert np.abs(h).max() > 1.9 * np.abs(x * nw).max() * scale.max()
+    out = torch.zeros(40, 40, device=dev)
+    gpu.linear_f64acc(*(torch.from_numpy(a).to(dev) for a in (x, w)), out,
+                      norm_w=torch.from_numpy(nw).to(dev), eps=float(eps))
+    _check(out.cpu().numpy(), (h.astype(np.float64) @ w.astype(np.float64).T).astype(np.float32))
+
+
 def test_workspace_is_checked(gpu, dev):
     """A workspace below the size asked for is refused before any launch; a null one means the
     plain product."""
