@@ -54,7 +54,7 @@ struct DigitLinear {
     int k_in;
 };
 
-
+typedef double double4_t __attribute__((ext_vector_type(4)));
 typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
 typedef int32_t i32x16_t __attribute__((ext_vector_type(16)));
 
@@ -342,6 +342,117 @@ constexpr int kStageK = 64;                // K of a stage: two MFMA steps
 constexpr int kStageX = 2 * 2 * kXBlk;     // 2 row blocks x 2 steps: 24 KiB
 constexpr int kStage = kStageX + 2 * 2 * 3 * kFrag;  // 2 column blocks x 2 steps, 3 digits
 
+// 32 x 32 outputs of one wave as f64 sums, for the rows and columns that the digits do not hold:
+// linear_gemm_kernel's wave (the f64 MFMA, operands from L2 into registers two 32-key chunks
+// ahead, the same keys a step), with the rows' scales from the workspace. MFMA-bound: 1,024 f64
+// products of 64 cycles for 1,024 keys. One element at a time a lane (2-byte loads, a serial
+// sum) took 60 ms for a layer's four products of 4,713 rows with one such row in 32, these 1.13,
+// linear_gemm_kernel alone 1.09; 13.3, 0.31 and 0.29 at 1,003 rows.
+template <int MODE, bool NORM>
+struct F64Block {
+    struct Chunk {
+        float4_t x[2][2], nw[NORM ? 2 : 1];
+        half8_t w[2];
+    };
+    const float* xp[2];
+    const float* nwp;
+    const half_t* wp[2];
+    double scale[2];
+    bool col_ok[2];
+    double4_t acc[2][2];
+
+    __device__ __forceinline__ void init(const DigitArgs& a, int row_blk, int col_blk, int lane) {
+        const DigitLinear& p = a.p;
+        const int col = lane & 15, g = lane >> 4;
+        nwp = NORM ? p.norm_w + 8 * g : nullptr;
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {  // past the end: the last row, and the first weight row
+            const int row = row_blk * kBlk + 16 * b + col;
+            xp[b] = p.x + (int64_t)min(row, p.rows - 1) * p.ldx + 8 * g;
+            scale[b] = reinterpret_cast<const double*>(a.ws + a.l.norm_off)[row];
+            wp[b] = weight_row(p, col_blk * kBlk + 16 * b + col, col_ok[b]) + 8 * g;
+            acc[b][0] = acc[b][1] = double4_t{0.0, 0.0, 0.0, 0.0};
+        }
+    }
+    __device__ __forceinline__ void load(int k0, Chunk& c) const {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            c.x[b][0] = *reinterpret_cast<const float4_t*>(xp[b] + k0);
+            c.x[b][1] = *reinterpret_cast<const float4_t*>(xp[b] + k0 + 4);
+            c.w[b] = *reinterpret_cast<const half8_t*>(wp[b] + k0);
+            if constexpr (NORM) c.nw[b] = *reinterpret_cast<const float4_t*>(nwp + k0 + 4 * b);
+        }
+    }
+    __device__ __forceinline__ void feed(const Chunk& c) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            double x[2], w[2];
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                float h = c.x[b][i >> 2][i & 3];
+                if constexpr (NORM) h = (float)((double)h * scale[b]) * c.nw[i >> 2][i & 3];
+                x[b] = (double)h;
+                w[b] = (double)(float)c.w[b][i];
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                acc[j >> 1][j & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[j >> 1], w[j & 1],
+                                                                         acc[j >> 1][j & 1], 0, 0, 0);
+        }
+    }
+    __device__ __forceinline__ void run(int k_in) {  // a multiple of 64
+        Chunk c0, c1;
+        load(0, c0);
+        __builtin_amdgcn_sched_barrier(0);
+        load(32, c1);
+        __builtin_amdgcn_sched_barrier(0);
+        for (int k0 = 0; k0 < k_in; k0 += 64) {  // the last loads are made again, unused
+            feed(c0);
+            __builtin_amdgcn_sched_barrier(0);
+            load(min(k0 + 64, k_in - 64), c0);
+            __builtin_amdgcn_sched_barrier(0);
+            feed(c1);
+            __builtin_amdgcn_sched_barrier(0);
+            load(min(k0 + 96, k_in - 32), c1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    __device__ __forceinline__ void store(const DigitLinear& p, int row_blk, int col_blk, int lane) const {
+        const int col = lane & 15, g = lane >> 4;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int row = row_blk * kBlk + 16 * (i >> 2) + g + 4 * (i & 3);
+            if (row >= p.rows) continue;
+            float* out = p.out + (int64_t)row * p.ldo;
+            if constexpr (MODE == kDigitSwiGLU) {
+                const float gate = (float)acc[i >> 2][0][i & 3], up = (float)acc[i >> 2][1][i & 3];
+                if (col_ok[0]) out[col_blk * 16 + col] = gate / (1.0f + expf(-gate)) * up;
+            } else {
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    const int n = col_blk * kBlk + 16 * b + col;
+                    const float y = (float)acc[i >> 2][b][i & 3];
+                    if (!col_ok[b]) continue;
+                    // out may alias resid: each element is read and written by the same lane
+                    out[n] = MODE == kDigitResidual ? p.resid[(int64_t)row * p.ldo + n] + y : y;
+                }
+            }
+        }
+    }
+};
+
+template <int MODE>
+__device__ __forceinline__ void f64_block(const DigitArgs& a, int row_blk, int col_blk, int lane) {
+    auto go = [&](auto norm_tag) {
+        F64Block<MODE, decltype(norm_tag)::value> f;
+        f.init(a, row_blk, col_blk, lane);
+        f.run(a.p.k_in);
+        f.store(a.p, row_blk, col_blk, lane);
+    };
+    if (a.p.norm_w) go(std::true_type{});
+    else go(std::false_type{});
+}
+
 // A 64 x 64 output tile per workgroup of 4 waves, 32 x 32 a wave. MFMA-bound: 18 products of
 // 32x32x32 a wave and step (24 with the fourth weight digit) against 9 KiB of LDS reads.
 // Stages of 64 keys stream into two LDS buffers with direct-to-LDS loads, the next stage's
@@ -385,15 +496,24 @@ __global__ __launch_bounds__(kDigitGemmThreads, 2) void digits_gemm_kernel(Digit
 
     // Flags: f64 for the wave's outputs if its row or column block needs it, a fourth weight
     // digit if one is nonzero anywhere in the wave's columns.
-    const int* xf = reinterpret_cast<const int*>(a.ws + a.l.xflag_off) + (2 * rt + wr) * kRowWgs;
-    const int* wf = reinterpret_cast<const int*>(a.ws + a.l.wflag_off) +
-                    (int64_t)(2 * ct + wc) * a.l.parts;
-    int wflag = 0;
-    for (int i = 0; i < (int)a.l.parts; ++i) wflag |= wf[i];
-    wflag = __builtin_amdgcn_readfirstlane(wflag);
-    const int xflag = __builtin_amdgcn_readfirstlane(xf[0] | xf[1] | xf[2] | xf[3]);
+    const int* xf = reinterpret_cast<const int*>(a.ws + a.l.xflag_off) + 2 * rt * kRowWgs;
+    const int* wf = reinterpret_cast<const int*>(a.ws + a.l.wflag_off) + (int64_t)(2 * ct) * a.l.parts;
+    int xflags[2], wflags[2] = {0, 0};  // of the tile's row and column blocks
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        const int* f = xf + b * kRowWgs;
+        xflags[b] = __builtin_amdgcn_readfirstlane(f[0] | f[1] | f[2] | f[3]);
+        for (int i = 0; i < (int)a.l.parts; ++i) wflags[b] |= wf[b * a.l.parts + i];
+        wflags[b] = __builtin_amdgcn_readfirstlane(wflags[b]);
+    }
+    const int xflag = wr ? xflags[1] : xflags[0], wflag = wc ? wflags[1] : wflags[0];
     const bool plain = (xflag & 1) != 0 || (wflag & 2) != 0;
     const bool four = (wflag & 1) != 0;
+    // every wave's outputs are f64 sums: no digit is needed
+    if ((xflags[0] & xflags[1] & 1) != 0 || (wflags[0] & wflags[1] & 2) != 0) {
+        f64_block<MODE>(a, 2 * rt + wr, 2 * ct + wc, lane);
+        return;
+    }
 
     // One stage: 24 + 12 blocks of 1 KiB. x block (row block b, step q, digit i) goes to LDS
     // slot (b * 2 + q) * 6 + i, w block (b, q, j) to 24 + (b * 2 + q) * 3 + j. Wave w loads
@@ -477,7 +597,25 @@ __global__ __launch_bounds__(kDigitGemmThreads, 2) void digits_gemm_kernel(Digit
     };
 #pragma unroll
     for (int i = 0; i < 9; ++i) issue_one(i, 0);
-    // The choice is per wave, and both loops pass the same barriers.
+    // The choice is per wave, and the loops pass the same barriers.
+    if (plain) {
+        // Only its share of the other waves' stages, then the f64 sums. (Taking 64 keys to each
+        // stage instead was no faster: the digits of the CU's other workgroup take turns with
+        // the f64 products on the matrix unit either way.)
+        for (int st = 0; st < n_stage; ++st) {
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            const bool more = st + 1 < n_stage;
+            xsrc += more ? 2 * kXBlk : 0;
+            wsrc += more ? 2 * kWBlk : 0;
+#pragma unroll
+            for (int i = 0; i < 9; ++i) issue_one(i, (st & 1) ^ 1);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        f64_block<MODE>(a, 2 * rt + wr, 2 * ct + wc, lane);
+        return;
+    }
     if (four) loop(std::true_type{});
     else loop(std::false_type{});
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into LDS outlives the workgroup
@@ -525,17 +663,7 @@ __global__ __launch_bounds__(kDigitGemmThreads, 2) void digits_gemm_kernel(Digit
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const int row = r0 + 8 * (i >> 2) + (i & 3);
-        float y = (float)(sums[i] * scales[row]);
-        if (plain) {
-            const double ns = reinterpret_cast<const double*>(a.ws + a.l.norm_off)[row];
-            const float* xr = p.x + (int64_t)min(row, p.rows - 1) * p.ldx;
-            double sum = 0.0;
-            for (int k = 0; k < p.k_in; ++k) {
-                const float h = p.norm_w ? (float)((double)xr[k] * ns) * p.norm_w[k] : xr[k];
-                sum += (double)h * (double)(float)wrow[k];
-            }
-            y = (float)sum;
-        }
+        const float y = (float)(sums[i] * scales[row]);
         const bool ok = row < p.rows && col_ok;
         if constexpr (MODE == kDigitSwiGLU) {
             const float u = __shfl_xor(y, 16);  // lanes 0..15 gate, 16..31 up

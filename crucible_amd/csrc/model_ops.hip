@@ -31,7 +31,6 @@
 namespace crucible {
 namespace {
 
-typedef double double4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kLinWaves = 8;               // the K range is split over the 8 waves
 constexpr int kLinThreads = 64 * kLinWaves;

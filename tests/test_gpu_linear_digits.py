@@ -247,6 +247,40 @@ def test_subnormal_rows_that_round_past_the_bound(gpu, dev, tune):
     _check(out.cpu().numpy(), (h.astype(np.float64) @ w.astype(np.float64).T).astype(np.float32))
 
 
+@pytest.mark.parametrize("mode", ["plain", "residual", "swiglu"])
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("rows,n_out,k_in", [(1, 1, 64), (100, 72, 192), (130, 200, 1088)])
+@pytest.mark.parametrize("bad_rows", [(), (3,), (40,), (3, 40), (99, 129)])
+@pytest.mark.parametrize("bad_cols", [(), (1,), (33, 70)])
+def test_blocks_of_f64_sums_beside_digits(gpu, dev, tune, mode, norm, rows, n_out, k_in, bad_rows, bad_cols):
+    """Row blocks and column blocks outside the digits, alone and beside others in a 64 x 64 tile:
+    the f64 kernel's outputs, bit for bit in those blocks."""
+    rng = np.random.default_rng(31)
+    x = rng.standard_normal((rows, k_in), dtype=np.float32)
+    w, up = ((rng.standard_normal((n_out, k_in)) * 0.02).astype(np.float16) for _ in range(2))
+    nw = (1 + 0.1 * rng.standard_normal(k_in)).astype(np.float32) if norm else None
+    bad_rows = [r for r in bad_rows if r < rows]
+    bad_cols = [c for c in bad_cols if c < n_out]
+    for r in bad_rows:  # one in four elements is rounded
+        x[r, ::4] = (rng.uniform(0.5, 1, x[r, ::4].shape) * 1e-12).astype(np.float32)
+    for c in bad_cols:
+        (up if mode == "swiglu" else w)[c, 5] = 200.0
+    resid = rng.standard_normal((rows, n_out), dtype=np.float32) if mode == "residual" else None
+    outs = []
+    for tile in (64, 32):
+        tune(linear_tile=tile)
+        outs.append(_run(gpu, dev, x, w, nw, resid=resid, w_up=up if mode == "swiglu" else None))
+    d = _ulps(*outs)
+    same = np.zeros((rows, n_out), bool)
+    for r in bad_rows:
+        same[r // 32 * 32:r // 32 * 32 + 32] = True
+    per = 16 if mode == "swiglu" else 32
+    for c in bad_cols:
+        same[:, c // per * per:c // per * per + per] = True
+    assert not d[same].any()
+    assert d.max() <= (8 if mode == "swiglu" else 1) and int((d > 0).sum()) <= max(2, d.size // 5000)
+
+
 def test_workspace_is_checked(gpu, dev):
     """A workspace below the size asked for is refused before any launch; a null one means the
     plain product."""
