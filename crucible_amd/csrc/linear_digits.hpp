@@ -14,7 +14,9 @@
 //     elements a row, and multiplied in f64 with the sums (of rows of 768 N(0,1) values about
 //     one in three thousand has such an element, of SwiGLU outputs one in thirty);
 //   - digit products of equal weight, s = i + j, share an accumulator: 18 products (i, j)
-//     in 8 accumulators (a ninth with the fourth weight digit).
+//     in 8 accumulators (a ninth with the fourth weight digit), 15 where the last activation
+//     digit is zero over 32 rows and 32 keys: it holds bits only of elements 2^14 below their
+//     row's largest (about one in twelve such pieces of N(0,1) rows of 768 has any).
 // So every product is exact, and the sums are joined in f64. Rows that this does not fit (a
 // non-finite value, a largest value outside 2^-60 .. 2^22, more than 16 rounded elements) and
 // columns with a weight over 127 or not finite take plain f64 sums instead, 32 x 32 outputs at
@@ -78,11 +80,12 @@ struct Rest {
 };
 
 // Workspace: the planes' blocks first (1 KiB aligned), then the rows' scales and rests, then
-// flags (rows: 1 f64 sums, 2 some row has rests; columns: 1 a fourth digit, 2 f64 sums).
+// flags (rows: 1 f64 sums, 2 some row has rests; columns: 1 a fourth digit, 2 f64 sums; a byte
+// for 8 rows and 32 keys: their last digit holds something).
 //   x planes [row block][K / 32][6][1024], w planes [column block][K / 32][4][1024]
 struct Layout {
     int64_t row_blks, col_blks, parts;
-    int64_t w_off, scale_off, norm_off, rest_off, count_off, xflag_off, wflag_off, bytes;
+    int64_t w_off, scale_off, norm_off, rest_off, count_off, last_off, xflag_off, wflag_off, bytes;
 };
 
 Layout make_layout(int64_t rows, int64_t cols, int64_t k_in) {
@@ -97,7 +100,8 @@ Layout make_layout(int64_t rows, int64_t cols, int64_t k_in) {
     l.norm_off = l.scale_off + l.row_blks * kBlk * 8;
     l.rest_off = l.norm_off + l.row_blks * kBlk * 8;
     l.count_off = l.rest_off + l.row_blks * kBlk * kRests * (int64_t)sizeof(Rest);
-    l.xflag_off = l.count_off + l.row_blks * kBlk * 4;
+    l.last_off = l.count_off + l.row_blks * kBlk * 4;
+    l.xflag_off = l.last_off + l.row_blks * steps * kRowWgs;
     l.wflag_off = l.xflag_off + l.row_blks * kRowWgs * 4;
     l.bytes = l.wflag_off + l.col_blks * l.parts * 4;
     return l;
@@ -270,27 +274,44 @@ __global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
     const float up = usual ? __builtin_bit_cast(float, (uint32_t)(21 - e + 127) << 23) : 0.0f;
     unsigned char* blk = a.ws + (int64_t)(row >> 5) * steps * kXBlk + (row & 31) * 16;
     auto write = [&](int g, const Group& v) {
-        uint32_t hi[16], lo[16];
+        uint32_t hi[16], lo[16], rounded = 0;
+        auto scaled = [&](int e) {
+            float h = v.x[e >> 2][e & 3];
+            if constexpr (NORM) h = (float)((double)h * scale) * v.nw[e >> 2][e & 3];
+            return ok && usual ? h * up : 0.0f;                     // exact
+        };
 #pragma unroll
         for (int q = 0; q < 4; ++q)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                float h = v.x[q][i];
-                if constexpr (NORM) h = (float)((double)h * scale) * v.nw[q][i];
-                const float t = ok && usual ? h * up : 0.0f;        // exact
+                const float t = scaled(4 * q + i);
                 if constexpr (NORM)
                     if (fabsf(t) >= 4194304.0f) s_flag = 1;
                 const float th = rintf(t);
                 const float tl = (t - th) * 16777216.0f;            // exact, |tl| <= 2^23
                 const float tr = rintf(tl);                         // rounds below 2^-22 of the largest
                 const uint32_t l = (uint32_t)((int)tr + 0x808080);  // 25 bits, carry on top
-                if (tl != tr) {
-                    const int at = atomicAdd(&s_rests[r], 1);
-                    if (at < kRests) s_rest[r][at] = {g * 16 + 4 * q + i, tl - tr};  // exact
-                }
+                rounded |= tl != tr ? 1u << (4 * q + i) : 0u;
                 hi[4 * q + i] = ((uint32_t)((int)th + (int)(l >> 24) + 0x808080)) ^ 0x808080u;
                 lo[4 * q + i] = l ^ 0x808080u;
             }
+        if (rounded) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                if (!(rounded >> i & 1)) continue;
+                const float t = scaled(i), tl = (t - rintf(t)) * 16777216.0f;
+                const int at = atomicAdd(&s_rests[r], 1);
+                if (at < kRests) s_rest[r][at] = {g * 16 + i, tl - rintf(tl)};  // exact
+            }
+        }
+        uint32_t last = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) last |= lo[i];
+        // 16 neighbouring lanes hold the 8 rows' 32 keys
+        const uint64_t some = __ballot((last & 255u) != 0) >> (tid & 48);
+        if ((tid & 15) == 0)
+            a.ws[a.l.last_off + ((int64_t)(row >> 5) * steps + (g >> 1)) * kRowWgs + (blockIdx.x & (kRowWgs - 1))] =
+                (some & 0xffffu) != 0;
         unsigned char* dst = blk + (int64_t)(g >> 1) * kXBlk + ((g & 1) ? 512 : 0);
 #pragma unroll
         for (int i = 0; i < kXDigits; ++i) {
@@ -498,13 +519,16 @@ __global__ __launch_bounds__(kDigitGemmThreads, 2) void digits_gemm_kernel(Digit
     // digit if one is nonzero anywhere in the wave's columns.
     const int* xf = reinterpret_cast<const int*>(a.ws + a.l.xflag_off) + 2 * rt * kRowWgs;
     const int* wf = reinterpret_cast<const int*>(a.ws + a.l.wflag_off) + (int64_t)(2 * ct) * a.l.parts;
-    int xflags[2], wflags[2] = {0, 0};  // of the tile's row and column blocks
+    const int parts = (int)a.l.parts;
+    const int x_lane = xf[lane & (2 * kRowWgs - 1)];
+    int w_lane = 0;  // the second block's flags two bits up
+    for (int i = lane; i < 2 * parts; i += 64) w_lane |= wf[i] << (i < parts ? 0 : 2);
+    int xflags[2], wflags[2];  // of the tile's row and column blocks
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-        const int* f = xf + b * kRowWgs;
-        xflags[b] = __builtin_amdgcn_readfirstlane(f[0] | f[1] | f[2] | f[3]);
-        for (int i = 0; i < (int)a.l.parts; ++i) wflags[b] |= wf[b * a.l.parts + i];
-        wflags[b] = __builtin_amdgcn_readfirstlane(wflags[b]);
+        const uint64_t lanes = ((1ull << kRowWgs) - 1) << (b * kRowWgs);
+        xflags[b] = ((__ballot(x_lane & 1) & lanes) ? 1 : 0) | ((__ballot(x_lane & 2) & lanes) ? 2 : 0);
+        wflags[b] = (__ballot(w_lane & (1 << 2 * b)) ? 1 : 0) | (__ballot(w_lane & (2 << 2 * b)) ? 2 : 0);
     }
     const int xflag = wr ? xflags[1] : xflags[0], wflag = wc ? wflags[1] : wflags[0];
     const bool plain = (xflag & 1) != 0 || (wflag & 2) != 0;
@@ -538,6 +562,10 @@ __global__ __launch_bounds__(kDigitGemmThreads, 2) void digits_gemm_kernel(Digit
     struct Frag {
         i32x4_t x[kXDigits], w[3];
     };
+    // a step's flags of the last digit as one word
+    typedef const __attribute__((address_space(4))) uint32_t* uniform_u32_ptr;
+    const uniform_u32_ptr lasts =
+        (uniform_u32_ptr)(a.ws + a.l.last_off + (int64_t)(2 * rt + wr) * steps * kRowWgs);
     auto read = [&](int buf, int q, Frag& f) {
         const unsigned char* base = &s_buf[buf][0] + lane * 16;
 #pragma unroll
@@ -549,6 +577,7 @@ __global__ __launch_bounds__(kDigitGemmThreads, 2) void digits_gemm_kernel(Digit
     };
     auto loop = [&](auto four_tag) {
         constexpr bool kFour = decltype(four_tag)::value;
+        uint32_t last[2] = {lasts[0], lasts[1]};
         for (int st = 0; st < n_stage; ++st) {
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
@@ -562,6 +591,8 @@ __global__ __launch_bounds__(kDigitGemmThreads, 2) void digits_gemm_kernel(Digit
             const bool more = st + 1 < n_stage;
             xsrc += more ? 2 * kXBlk : 0;
             wsrc += more ? 2 * kWBlk : 0;
+            const int ahead = 2 * (more ? st + 1 : st);
+            const uint32_t next[2] = {lasts[ahead], lasts[ahead + 1]};
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
@@ -569,27 +600,35 @@ __global__ __launch_bounds__(kDigitGemmThreads, 2) void digits_gemm_kernel(Digit
                 if constexpr (kFour)
                     w4 = *reinterpret_cast<const i32x4_t*>(
                         wp + ((int64_t)wc * steps + 2 * st + q) * kWBlk + 3 * kFrag + lane * 16);
+                auto product = [&](int i, int j, i32x4_t w) {
+                    acc[i + j + 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f[q].x[i], w, acc[i + j + 1], 0, 0, 0);
+                };
                 // j outer: consecutive products go to different accumulators
-                int n = 0;
+                int n = 0, issued = 0;
 #pragma unroll
                 for (int j = 0; j < 3; ++j)
 #pragma unroll
-                    for (int i = 0; i < kXDigits; ++i) {
-                        acc[i + j + 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
-                            f[q].x[i], f[q].w[j], acc[i + j + 1], 0, 0, 0);
-                        if (!kFour && q == 0 && (n & 1) == 0 && n < 18) {
+                    for (int i = 0; i < kXDigits - 1; ++i) {
+                        product(i, j, f[q].w[j]);
+                        if (!kFour && q == 0 && n * 3 % 5 < 3) {  // 9 of the 15
                             __builtin_amdgcn_sched_barrier(0);
-                            issue_one(n >> 1, buf ^ 1);
+                            issue_one(issued++, buf ^ 1);
                             __builtin_amdgcn_sched_barrier(0);
                         }
                         ++n;
                     }
                 if constexpr (kFour) {
 #pragma unroll
-                    for (int i = 0; i < kXDigits; ++i)
-                        acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f[q].x[i], w4, acc[i], 0, 0, 0);
+                    for (int i = 0; i < kXDigits - 1; ++i) product(i, -1, w4);
+                }
+                if (last[q]) {
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) product(kXDigits - 1, j, f[q].w[j]);
+                    if constexpr (kFour) product(kXDigits - 1, -1, w4);
                 }
             }
+            last[0] = next[0];
+            last[1] = next[1];
             if constexpr (kFour)
 #pragma unroll
                 for (int i = 0; i < 9; ++i) issue_one(i, buf ^ 1);
