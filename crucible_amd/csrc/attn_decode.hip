@@ -1137,13 +1137,21 @@ __global__ __launch_bounds__(kGenericThreads) void decode_generic_kernel(DecodeA
 // callers of these dimensions never had to clear or own one. HBM-bound at large batches,
 // latency-bound below; the split is small because one CU streams only 25-50 GB/s. 16 requests
 // of 64..2048 tokens, 12/3 heads of 128, fused append (26 MB): 70 us a layer with
-// attend_generic, 22.2 here with the append and the combine launches. Up to
-// 128 dims the registers are capped at 128, so that two workgroups share a CU (a few of the
-// f32-query form spill; uncapped it took 22 us against 19).
+// attend_generic, 22.2 here with the append and the combine launches. Up to 128 dims the
+// registers of the one-split forms are capped at 128, so that two workgroups share a CU (20 bytes
+// a lane spill at 128 dims; uncapped it took 22 us against 19). The walk's second state does not
+// fit there (300 to 400 bytes a lane spilled), so it takes what it needs; it is bound by its CU's
+// stream: 1 x 2,048 tokens 38 us, 16 x 1,000 22, 128 x 100 9.8 (12/3 heads of 128; the generic
+// kernel 35, 22 and 16; 76, 44 and 21 against 69, 36 and 25 at 256 dims).
 constexpr int kHdSplitPages = 16;
 
-template <int HD, bool QF32, bool WHOLE>
-__global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 ? 4 : 1) void decode_hd_kernel(DecodeArgs a, int col_blocks) {
+// A workgroup's share of a unit: one split, its partial to the scratch; the only split there can
+// be, straight to the output; or, without scratch, all of them.
+enum HdShare { kHdSplit, kHdOnly, kHdWalk };
+
+template <int HD, bool QF32, int SHARE>
+__global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 && SHARE != kHdWalk ? 4 : 1) void decode_hd_kernel(
+    DecodeArgs a, int col_blocks) {
     constexpr int W = hd_waves(HD);
     __shared__ HdLds<HD, W, 1> lds;
     const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
@@ -1155,7 +1163,7 @@ __global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 ? 4 : 1) void decode_h
     const uniform_i32_ptr table =
         a.tables ? (uniform_i32_ptr)(a.tables + (int64_t)b * a.table_stride) : nullptr;
     auto page_of = [&](int i) { return table ? (int64_t)table[min(i, a.max_pages - 1)] : (int64_t)i; };
-    const int s0 = WHOLE ? 0 : (int)blockIdx.z;
+    const int s0 = SHARE == kHdSplit ? (int)blockIdx.z : 0;
     const int first = s0 * kHdSplitPages + 2 * wave;
     int id0 = (int)page_of(first), id1 = (int)page_of(first + 1);
     asm volatile("" : "+s"(id0), "+s"(id1));  // issued with the length's load, not behind its branch
@@ -1210,7 +1218,7 @@ __global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 ? 4 : 1) void decode_h
 #pragma unroll
         for (int i = 0; i < kHdSplitPages / 2; i += W) {
             const int p = sp * kHdSplitPages + 2 * (i + wave);
-            if ((WHOLE && sp > 0) || i > 0) {
+            if (i > 0) {
                 page0 = page_of(p);
                 page1 = page_of(p + 1);
                 load(p);
@@ -1220,22 +1228,29 @@ __global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 ? 4 : 1) void decode_h
             if (key0 + 2 * kPageTokens > len) kv.zero_tail(key0, len, grp);
             hd_attend_pair(s[0], q, kv, key0, len - 1, grp);
         }
+        if (SHARE == kHdWalk && sp + 1 < n_active) {  // the next split's pages, beside the merge
+            const int p = (sp + 1) * kHdSplitPages + 2 * wave;
+            page0 = page_of(p);
+            page1 = page_of(p + 1);
+            load(p);
+        }
         hd_merge_waves<HD, W, 1>(lds, s, wave, col, grp, n_cols);
-        if constexpr (!WHOLE) break;
+        if constexpr (SHARE != kHdWalk) break;
         if (sp == 0) total = s[0];
         else total.merge(s[0]);
         if (sp + 1 == n_active) break;
     }
+    if constexpr (SHARE != kHdWalk) total = s[0];
     const bool mine = wave == 0 && col < n_cols;
-    if constexpr (!WHOLE) {
+    if constexpr (SHARE == kHdSplit) {
         if (!mine) return;
         const int64_t slot = ((int64_t)b * a.n_head + h) * a.n_splits + s0;
 #pragma unroll
         for (int i = 0; i < HD / 16; ++i)
-            *reinterpret_cast<float4_t*>(a.po + slot * HD + 16 * i + 4 * grp) = s[0].o[i];
+            *reinterpret_cast<float4_t*>(a.po + slot * HD + 16 * i + 4 * grp) = total.o[i];
         if (grp == 0) {
-            a.pm[slot] = s[0].m;
-            a.pl[slot] = s[0].l;
+            a.pm[slot] = total.m;
+            a.pl[slot] = total.l;
         }
     } else {
         __shared__ GenericLds again;
@@ -1560,6 +1575,26 @@ DecodeArgs common_args(const void* q, const void* k, const void* v, void* out, i
     return a;
 }
 
+// Where decode_generic_kernel, one workgroup of 4 waves a query head, is the faster form. What
+// decode_hd_kernel gains is one K/V read for the heads of a group and workgroups for every split;
+// with one or two heads a group and enough requests, or contexts of one split, neither counts, and
+// its wide workgroups and their merge cost more. us with scratch against generic, at full contexts:
+//   one head a group, 512 units (request, kv head) or more: 55.7 / 43.4 (128 dims, 128 x 500 keys,
+//     8 kv heads), 43.3 / 34.2 (96); 256 or more from 160 dims on: 44.6 / 34.8 (64 x 1,000, 4);
+//     at 16 x 2,000 keys the other way: 33.9 / 50.9 (128), 28.3 / 47.8 (96)
+//   one head a group, one split, 128 dims or more: 8.4 / 7.3 (16 x 200, 128), 24.6 / 11.7 (128 x 60, 160)
+//   two heads, one split, 160 dims or more: 16.3 / 13.0 (64 x 100, 160), 22.1 / 16.4 (256)
+//   few units, one split, 192 dims or more: 9.7 / 8.3 (1 x 100, 12/3 heads of 256)
+// By the shape alone, so that calls with and without scratch, and the separate and fused entries,
+// give the same bits.
+bool generic_decode_faster(const DecodeArgs& a, int hd) {
+    const int64_t units = (int64_t)a.batch * a.n_kv_head;
+    const bool one_split = a.max_pages <= kHdSplitPages;
+    if (a.n_rep == 1 && (units >= (hd >= 160 ? 256 : 512) || (one_split && hd >= 128))) return true;
+    if (a.n_rep == 2 && one_split && hd >= 160) return true;
+    return one_split && hd >= 192 && units < 32;
+}
+
 // Whether decode_hd_kernel takes the call: its vector accesses need 16-byte rows, its grid
 // the counts below. Everything else stays with decode_generic_kernel.
 bool hd_decode_fits(const DecodeArgs& a, int hd, bool q_f32) {
@@ -1567,7 +1602,7 @@ bool hd_decode_fits(const DecodeArgs& a, int hd, bool q_f32) {
            aligned16(a.rope_sin) &&
            a.q_row_stride % (q_f32 ? 4 : 8) == 0 &&
            a.batch <= 65535 && a.n_kv_head <= 65535 &&
-           a.max_pages <= kHdSplitPages * 65535;
+           a.max_pages <= kHdSplitPages * 65535 && !generic_decode_faster(a, hd);
 }
 
 template <int HD>
@@ -1577,12 +1612,13 @@ void launch_decode_hd(const DecodeArgs& a, bool q_f32, hipStream_t stream) {
                     (unsigned)(a.po ? a.n_splits : 1));
     auto go = [&](auto f32_tag) {
         constexpr bool kF32 = decltype(f32_tag)::value;
-        if (a.po)
-            hipLaunchKernelGGL((decode_hd_kernel<HD, kF32, false>), grid, dim3(64 * hd_waves(HD)),
-                               0, stream, a, blocks);
-        else
-            hipLaunchKernelGGL((decode_hd_kernel<HD, kF32, true>), grid, dim3(64 * hd_waves(HD)),
-                               0, stream, a, blocks);
+        auto launch = [&](auto share_tag) {
+            hipLaunchKernelGGL((decode_hd_kernel<HD, kF32, decltype(share_tag)::value>), grid,
+                               dim3(64 * hd_waves(HD)), 0, stream, a, blocks);
+        };
+        if (a.po) launch(std::integral_constant<int, kHdSplit>{});
+        else if (a.n_splits == 1) launch(std::integral_constant<int, kHdOnly>{});
+        else launch(std::integral_constant<int, kHdWalk>{});
     };
     if (q_f32) go(std::true_type{});
     else go(std::false_type{});

@@ -268,6 +268,36 @@ def test_prefill_of_infinite_values(gpu, dev, hd, dtype, hybrid, what, key, valu
     _same_special(*outs)
 
 
+@pytest.mark.parametrize("hd,n_head,n_kv,lens", [
+    (128, 2, 2, [200, 16]), (160, 4, 2, [256, 1]), (256, 4, 1, [100]), (96, 8, 8, [40] * 64),
+    (160, 4, 4, [300] * 64), (128, 8, 8, [300] * 64), (128, 8, 8, [300] * 63), (160, 4, 2, [257, 8])])
+def test_decode_forms_by_shape(gpu, dev, hd, n_head, n_kv, lens):
+    """Shapes on both sides of the line between the one-head and the shared-K/V kernels: outputs
+    to TOL of the generic kernel's, equal bits with and without scratch and from the fused entry."""
+    from crucible_amd import _lib
+    lib = _lib.load()
+    b, layer = len(lens), 1
+    g, stride, kv, (kp, vp), tables, q = _case(dev, hd + b, hd, n_head, n_kv, lens)
+    d_len = torch.tensor(lens, dtype=torch.int32, device=dev)
+    max_seq = 16 * -(-max(lens) // 16)
+    geometry = (b, n_head, n_kv, hd, stride, 2, layer, kv, max_seq)
+    outs = [torch.full((b, n_head * hd), 7.0, device=dev) for _ in range(4)]
+    gpu.attention_decode_paged(q, kp, vp, outs[0], tables, d_len, *geometry)
+    gpu.attention_decode_paged(_unaligned(q), kp, vp, outs[1], tables, d_len, *geometry)
+    stream = torch.cuda.current_stream().cuda_stream
+    _lib.check(lib.crucible_attention_decode_paged(
+        q.data_ptr(), 0, kp.data_ptr(), vp.data_ptr(), outs[2].data_ptr(), 0, tables.data_ptr(),
+        d_len.data_ptr(), *geometry, None, 0, stream))
+    k = kp.view(-1, 2, 16, kv)
+    v = vp.view(-1, 2, kv, 16)
+    last = d_len.long() - 1
+    page = tables.gather(1, (last // 16)[:, None])[:, 0].long()
+    k_new, v_new = k[page, layer, last % 16].contiguous(), v[page, layer, :, last % 16].contiguous()
+    gpu.attention_decode_paged_append(q, k_new, v_new, kp, vp, outs[3], tables, last.int(), d_len, *geometry)
+    assert float((outs[0] - outs[1]).abs().max()) <= TOL
+    assert torch.equal(outs[2], outs[0]) and torch.equal(outs[3], outs[0])
+
+
 def test_large_and_tiny_f32_queries(gpu, dev):
     """f32 queries outside fp16's range: the operands are scaled by a power of two."""
     hd, n_head, n_kv, lens = 128, 4, 2, [70, 33]
