@@ -298,6 +298,32 @@ def test_decode_forms_by_shape(gpu, dev, hd, n_head, n_kv, lens):
     assert torch.equal(outs[2], outs[0]) and torch.equal(outs[3], outs[0])
 
 
+@pytest.mark.parametrize("hd", [32, 96, 128, 160, 192, 224, 256])
+@pytest.mark.parametrize("n_head,n_kv", [(4, 2), (40, 2)])
+@pytest.mark.parametrize("kind", ["distinct", "alternating", "runs"])
+def test_prefill_tiles_of_many_owners(gpu, dev, hd, n_head, n_kv, kind):
+    """Packed rows of as many requests as rows, of three requests in turn, and of runs longer and
+    shorter than a tile: a tile's owners are dealt out over workgroups (more of them with few
+    heads), and every row is its request's alone."""
+    rng = np.random.default_rng(37)
+    owners = {"distinct": rng.permutation(70), "alternating": np.arange(70) % 3,
+              "runs": np.repeat(np.arange(5), [1, 40, 2, 24, 3])}[kind].astype(np.int32)
+    lens = rng.integers(1, 90, owners.max() + 1).tolist()
+    positions = np.array([rng.integers(0, lens[o]) for o in owners], np.int32)
+    positions[5] = -1
+    g, stride, kv, (kp, vp), tables, _ = _case(dev, hd + 11, hd, n_head, n_kv, lens)
+    q = torch.randn(70, n_head * hd, generator=g, device=dev).half()
+    d_own, d_pos = (torch.from_numpy(a).to(dev) for a in (owners, positions))
+    outs = []
+    for x in (q, _unaligned(q)):
+        out = torch.full((70, n_head * hd), 7.0, device=dev)
+        gpu.attention_prefill_packed(x, kp, vp, out, tables, d_own, d_pos, 70, stride, n_head, n_kv, hd,
+                                     2, 1, kv, stride * 16)
+        outs.append(out)
+    assert bool((outs[0][5] == 7.0).all())
+    assert float((outs[0] - outs[1]).abs().max()) <= TOL
+
+
 def test_large_and_tiny_f32_queries(gpu, dev):
     """f32 queries outside fp16's range: the operands are scaled by a power of two."""
     hd, n_head, n_kv, lens = 128, 4, 2, [70, 33]
