@@ -12,7 +12,9 @@ Differences from the reference, all from the allowed page-layout change:
   * pools are fp16 (reference: f32) and V pools store each (page, layer) block
     transposed, so the append methods take ``kind="k"`` or ``kind="v"``;
   * split-K decode needs a workspace; pass one (graph capture) or let the Gpu keep
-    a cached one per (batch, n_head, max_seq).
+    a cached one per (batch, n_head, max_seq). Launches that share a workspace must be
+    ordered. At a head_dim other than 64, calls without one take scratch from torch's
+    allocator.
 """
 from __future__ import annotations
 
@@ -155,15 +157,29 @@ class Gpu:
         graph) can take it, so calls on several streams and threads never share one."""
         return torch.empty(nbytes, dtype=torch.uint8, device=self.device)
 
-    def _decode_scratch(self, workspace, batch, n_head, head_dim, max_seq, pools=None):
-        """The workspace of a decode call: the caller's or the cached one for head_dim 64. The
-        other dimensions keep nothing between calls and never needed calls to be ordered, so
-        theirs is scratch of the call's own."""
-        if head_dim != 64:
-            # one split more than head_dim 64's need: wider heads round up to larger splits
-            return self._scratch(max(16, self.lib.crucible_attention_decode_workspace_bytes(
-                batch, n_head, max_seq) + 4 * batch * n_head * (head_dim + 2)))
-        return workspace if workspace is not None else self.workspace(batch, n_head, max_seq, pools)
+    def _decode_workspace(self, workspace, batch, n_head, head_dim, max_seq, pools=None):
+        """(tensor kept for the call, pointer, bytes) of a decode call's workspace: the caller's,
+        else for head_dim 64 the cached one. The kernels of the other multiples of 32 keep nothing
+        between calls, and calls on several streams never had to be ordered, so without a
+        caller's workspace that holds their partials they get scratch of the call's own; the
+        remaining dimensions use none."""
+        if workspace is not None:
+            _need(workspace, "workspace")
+        if head_dim == 64:
+            ws = workspace if workspace is not None else self.workspace(batch, n_head, max_seq, pools)
+        elif head_dim % 32:
+            return None, None, 0
+        else:
+            need = self.lib.crucible_attention_decode_workspace_bytes(batch, n_head, max_seq)
+            if head_dim > 160:  # wider partials round up to one split more than that holds
+                need += 4 * batch * n_head * (head_dim + 2)
+            ws = workspace
+            if ws is None or ws.numel() * ws.element_size() < need:
+                # a shape past the limits is the library's to refuse
+                ws = self._scratch(need) if 0 < need < 1 << 62 else None
+            if ws is None:
+                return None, None, 0
+        return ws, _ptr(ws), ws.numel() * ws.element_size()
 
     @staticmethod
     def version() -> str:
@@ -223,13 +239,12 @@ class Gpu:
         _need(v_pool, "v_pool", dtype=torch.float16)
         _need(page_tables, "page_tables", dtype=torch.int32, numel=batch * table_stride)
         _need(seq_lens, "seq_lens", dtype=torch.int32, numel=batch)
-        ws = self._decode_scratch(workspace, batch, n_head, head_dim, max_seq, (k_pool, v_pool))
-        _need(ws, "workspace")
+        ws, ws_ptr, ws_bytes = self._decode_workspace(workspace, batch, n_head, head_dim, max_seq,
+                                                      (k_pool, v_pool))
         _lib.check(self.lib.crucible_attention_decode_paged(
             _ptr(q), _dtype(q, "q"), _ptr(k_pool), _ptr(v_pool), _ptr(out), _dtype(out, "out"),
             _ptr(page_tables), _ptr(seq_lens), batch, n_head, n_kv_head, head_dim, table_stride,
-            n_layer, layer, kv_dim, max_seq, _ptr(ws), ws.numel() * ws.element_size(),
-            self._stream()))
+            n_layer, layer, kv_dim, max_seq, ws_ptr, ws_bytes, self._stream()))
 
     def attention_decode_paged_append(self, q, k_new, v_new, k_pool, v_pool, out, page_tables,
                                       positions, seq_lens, batch, n_head, n_kv_head, head_dim,
@@ -247,13 +262,13 @@ class Gpu:
         _need(page_tables, "page_tables", dtype=torch.int32, numel=batch * table_stride)
         _need(positions, "positions", dtype=torch.int32, numel=batch)
         _need(seq_lens, "seq_lens", dtype=torch.int32, numel=batch)
-        ws = self._decode_scratch(workspace, batch, n_head, head_dim, max_seq, (k_pool, v_pool))
+        ws, ws_ptr, ws_bytes = self._decode_workspace(workspace, batch, n_head, head_dim, max_seq,
+                                                      (k_pool, v_pool))
         _lib.check(self.lib.crucible_attention_decode_paged_append(
             _ptr(q), _dtype(q, "q"), _ptr(k_new), _ptr(v_new), _dtype(k_new, "k_new"),
             _ptr(k_pool), _ptr(v_pool), _ptr(out), _dtype(out, "out"), _ptr(page_tables),
             _ptr(positions), _ptr(seq_lens), batch, n_head, n_kv_head, head_dim, table_stride,
-            n_layer, layer, kv_dim, max_seq, _ptr(ws), ws.numel() * ws.element_size(),
-            self._stream()))
+            n_layer, layer, kv_dim, max_seq, ws_ptr, ws_bytes, self._stream()))
 
     def attention_decode_qkv_paged_append(self, qkv, rope_cos, rope_sin, k_pool, v_pool, out,
                                           page_tables, positions, seq_lens, batch, n_head,
@@ -275,12 +290,13 @@ class Gpu:
             _need(rope_cos, "rope_cos", dtype=torch.float32)
             _need(rope_sin, "rope_sin", dtype=torch.float32, numel=rope_cos.numel())
             max_pos = rope_cos.shape[0]
-        ws = self._decode_scratch(workspace, batch, n_head, head_dim, max_seq, (k_pool, v_pool))
+        ws, ws_ptr, ws_bytes = self._decode_workspace(workspace, batch, n_head, head_dim, max_seq,
+                                                      (k_pool, v_pool))
         _lib.check(self.lib.crucible_attention_decode_qkv_paged_append(
             _ptr(qkv), row_stride, _ptr(rope_cos), _ptr(rope_sin), max_pos, _ptr(k_pool),
             _ptr(v_pool), _ptr(out), _dtype(out, "out"), _ptr(page_tables), _ptr(positions),
             _ptr(seq_lens), batch, n_head, n_kv_head, head_dim, table_stride, n_layer, layer,
-            kv_dim, max_seq, _ptr(ws), ws.numel() * ws.element_size(), self._stream()))
+            kv_dim, max_seq, ws_ptr, ws_bytes, self._stream()))
 
     def attention_decode(self, q, k_cache, v_cache, out, n_head, n_kv_head, head_dim, params,
                          max_seq, cache_stride, layer_base, workspace=None):
@@ -290,11 +306,11 @@ class Gpu:
         _need(k_cache, "k_cache", dtype=torch.float16)
         _need(v_cache, "v_cache", dtype=torch.float16)
         _need(params, "params", dtype=torch.int32, numel=6)
-        ws = self._decode_scratch(workspace, 1, n_head, head_dim, max_seq)
+        ws, ws_ptr, ws_bytes = self._decode_workspace(workspace, 1, n_head, head_dim, max_seq)
         _lib.check(self.lib.crucible_attention_decode(
             _ptr(q), _dtype(q, "q"), _ptr(k_cache), _ptr(v_cache), _ptr(out), _dtype(out, "out"),
             n_head, n_kv_head, head_dim, _ptr(params), max_seq, cache_stride, layer_base,
-            _ptr(ws), ws.numel() * ws.element_size(), self._stream()))
+            ws_ptr, ws_bytes, self._stream()))
 
     def attention_split(self, q, k_cache, v_cache, partial_o, partial_m, partial_l, out, n_head,
                         n_kv_head, head_dim, params, capacity, cache_stride, layer_base):

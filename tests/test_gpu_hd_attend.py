@@ -406,3 +406,34 @@ def test_workspace_shared_with_head_dim_64(gpu, dev, hd):
     want = run(usual, 64)
     assert torch.equal(run(wide, hd), first)
     assert torch.equal(run(usual, 64), want)
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+def test_the_callers_workspace_is_used(gpu, dev, hd):
+    """A call that brings a workspace which holds its partials allocates nothing and writes them
+    there; one that is too small is left alone; one that is not on the device is refused."""
+    from crucible_amd._lib import CrucibleError
+    lens, n_head, n_kv = [600, 33, 257], 12, 3
+    b = len(lens)
+    g, stride, kv, (kp, vp), tables, q = _case(dev, hd, hd, n_head, n_kv, lens)
+    d_len = torch.tensor(lens, dtype=torch.int32, device=dev)
+    max_seq = stride * 16
+    need = gpu.lib.crucible_attention_decode_workspace_bytes(b, n_head, max_seq) + 4 * b * n_head * (hd + 2)
+
+    def run(ws):
+        out = torch.zeros(b, n_head * hd, device=dev)
+        before = torch.cuda.memory_stats(dev)["allocation.all.allocated"]
+        gpu.attention_decode_paged(q, kp, vp, out, tables, d_len, b, n_head, n_kv, hd, stride, 2, 1, kv,
+                                   max_seq, workspace=ws)
+        return out, torch.cuda.memory_stats(dev)["allocation.all.allocated"] - before
+
+    want, allocated = run(None)
+    assert allocated > 0
+    ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+    out, allocated = run(ws)
+    assert allocated == 0 and bool(ws.any()) and torch.equal(out, want)
+    small = torch.zeros(1 << 20, dtype=torch.uint8, device=dev)
+    out, _ = run(small)
+    assert not small.any() and torch.equal(out, want)
+    with pytest.raises(CrucibleError):
+        run(torch.zeros(need, dtype=torch.uint8))
