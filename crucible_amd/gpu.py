@@ -151,11 +151,22 @@ class Gpu:
             self._bindings[key] = binding
         return ws
 
-    def _scratch(self, nbytes: int) -> torch.Tensor:
+    def _scratch(self, nbytes: int) -> torch.Tensor | None:
         """Scratch of one call, from torch's caching allocator on the current stream: the
         block goes back when the call returns and only later work of the same stream (or
-        graph) can take it, so calls on several streams and threads never share one."""
-        return torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+        graph) can take it, so calls on several streams and threads never share one. None
+        where the device has no room for it: the call then takes its form without scratch."""
+        try:
+            return torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+        except torch.OutOfMemoryError:
+            return None
+
+    def _digit_scratch(self, rows, n_out, k_in, norm, swiglu, prefetch):
+        """(scratch, bytes) of a projection on int8 digits; (None, 0): it takes another form."""
+        nbytes = self.lib.crucible_linear_workspace_bytes(rows, n_out, k_in, norm, swiglu)
+        if not nbytes or (prefetch is not None and _prefetch_region(prefetch)[0] % 4):
+            return None, 0
+        return self._scratch(nbytes), nbytes
 
     def _decode_workspace(self, workspace, batch, n_head, head_dim, max_seq, pools=None):
         """(tensor kept for the call, pointer, bytes) of a decode call's workspace: the caller's,
@@ -398,9 +409,8 @@ class Gpu:
         args = (_ptr(x), k_in, _ptr(norm_w) if norm_w is not None else None, float(eps),
                 _ptr(w), n_out, k_in, _ptr(resid) if resid is not None else None, _ptr(out),
                 n_out, rows)
-        nbytes = self.lib.crucible_linear_workspace_bytes(rows, n_out, k_in, norm_w is not None, 0)
-        if nbytes and (prefetch is None or _prefetch_region(prefetch)[0] % 4 == 0):
-            ws = self._scratch(nbytes)
+        ws, nbytes = self._digit_scratch(rows, n_out, k_in, norm_w is not None, 0, prefetch)
+        if ws is not None:
             _lib.check(self.lib.crucible_linear_f64acc_ws(*args, _ptr(ws), nbytes,
                                                           self._stream()))
         elif prefetch is None:
@@ -424,9 +434,8 @@ class Gpu:
             _need(norm_w, "norm_w", dtype=torch.float32, numel=k_in)
         args = (_ptr(x), k_in, _ptr(norm_w) if norm_w is not None else None, float(eps),
                 _ptr(w_gate), _ptr(w_up), hidden, k_in, _ptr(out), hidden, rows)
-        nbytes = self.lib.crucible_linear_workspace_bytes(rows, hidden, k_in, norm_w is not None, 1)
-        if nbytes and (prefetch is None or _prefetch_region(prefetch)[0] % 4 == 0):
-            ws = self._scratch(nbytes)
+        ws, nbytes = self._digit_scratch(rows, hidden, k_in, norm_w is not None, 1, prefetch)
+        if ws is not None:
             _lib.check(self.lib.crucible_linear_swiglu_f64acc_ws(*args, _ptr(ws), nbytes,
                                                                  self._stream()))
         elif prefetch is None:

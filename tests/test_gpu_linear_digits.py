@@ -304,3 +304,33 @@ def test_workspace_is_checked(gpu, dev):
     assert lib.crucible_linear_f64acc_ws(*args, ws.data_ptr(), need, stream) == 0
     d = (out.view(torch.int32).long() - plain.view(torch.int32).long()).abs()
     assert int(d.max()) <= 1 and int((d > 0).sum()) <= out.numel() // 20000
+
+
+def test_no_room_for_the_digits(gpu, dev):
+    """Where the digits' scratch does not fit the device's memory, the product is made without
+    it, as it was before it took any."""
+    rows, hidden, k_in = 2048, 2048, 768
+    need = gpu.lib.crucible_linear_workspace_bytes(rows, hidden, k_in, 1, 1)
+    assert need > 20 << 20
+    x = torch.randn(rows, k_in, device=dev)
+    w, up = (torch.randn(hidden, k_in, device=dev).mul_(0.02).half() for _ in range(2))
+    nw = torch.ones(k_in, device=dev)
+    outs = [torch.zeros(rows, hidden, device=dev) for _ in range(4)]
+
+    def both(a, b):
+        gpu.linear_f64acc(x, w, a, norm_w=nw)
+        gpu.linear_swiglu_f64acc(x, w, up, b, norm_w=nw)
+
+    both(*outs[:2])
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(dev).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(dev) + (4 << 20)) / total, dev)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(need, dtype=torch.uint8, device=dev)
+        both(*outs[2:])
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, dev)
+    assert int((outs[0] - outs[2]).abs().gt(0).sum()) <= outs[0].numel() // 20000
+    torch.testing.assert_close(outs[1], outs[3], rtol=1e-6, atol=1e-9)
