@@ -40,6 +40,7 @@ namespace {
 enum DigitMode { kDigitPlain = 0, kDigitResidual = 1, kDigitSwiGLU = 2 };
 
 constexpr int kDecodeRows = 32;  // batches up to here keep the decode tilings
+constexpr int64_t kWideOutputs = 16 * 1024;  // decode tilings: several column blocks a workgroup
 
 struct DigitLinear {
     const float* x;
@@ -716,24 +717,35 @@ __global__ __launch_bounds__(kDigitGemmThreads, 2) void digits_gemm_kernel(Digit
     }
 }
 
-// Which form a product takes, by what each costs. The lines are fits, in us, to graph replays
-// of the 120m and 350m decoders' four products (768 and 1024 wide) at 64 to 1,024 rows, within
-// about 15% there; G = 10^9 multiply-adds:
-//   decode tilings     5 + 52 G, with a fused norm or SwiGLU 5 + 115 G (every workgroup
-//                      normalises its rows again; half-width tiles): 512 x 768 x 768 21.4,
-//                      192 x 1152 x 768 with norm 27.0
-//   int8 digits        a digit and a product launch each as long as K: 11 + 0.0155 K, the
-//                      weights' digits 2e-6 a weight, 10 G once the CUs are full:
-//                      24.6 and 21.9 there, 4,713 rows of gate/up 208
-//   f64 output tiles   one workgroup's whole K, 3 + 0.0345 K, or 39 G: 29.5 and 34.0, 554
+// Which form a product takes, by what each costs. The lines are fits, in us, to graph replays of
+// 18 products at 33 to 8,000 rows: 64 to 50,304 outputs, K of 64 to 16,384, the 120m decoder's
+// four among them. W are the weights, 10^9 G the multiply-adds with the rows rounded up to the
+// form's tile, out the outputs (gate and up):
+//   decode tilings     5 + the longer of 0.0035 K and 52 G (rows to 16), 100 G where every
+//                      workgroup normalises its rows again or holds gate and up, up to 16K outputs
+//   int8 digits        10, the planes (6 bytes a weight, 10 an activation at 4.5 TB/s), and the
+//                      longer of a tile's K, 0.0145 K, and 10 G (rows to 64), and 2.2e-6 out for
+//                      the joining of the sums
+//   f64 output tiles   3.5 + 0.035 K for each round of workgroups over the CUs + 0.5e-6 out
+// What it picks is within 4% of the form each product had by a fixed 128 rows, or faster, and
+// within 15% of the best of the three (36% at 33 to 64 rows of 32,000 x 768). Lines without
+// the rounding, the planes and the joining, fitted at 768 and 1,024 wide alone, took 125 us for
+// 33 rows of 50,304 x 768 (tilings 104, now 80), 172 for 8,000 of 64 x 4,096 (f64 tiles 138, now
+// the tilings' 115), 113 for 8,000 of 4,096 x 64 (f64 tiles 100, now those).
 struct LinearCost {
     double tiles, digits, gemm;
 };
 LinearCost linear_cost(int64_t rows, int64_t n_out, int64_t k_in, bool norm, bool swiglu) {
-    const double k = (double)k_in, weights = (double)n_out * k * (swiglu ? 2 : 1);
-    const double g = weights * (double)rows * 1e-9;
-    return {5.0 + (norm || swiglu ? 115.0 : 52.0) * g, 11.0 + 0.0155 * k + 2e-6 * weights + 10.0 * g,
-            std::max(3.0 + 0.0345 * k, 39.0 * g)};
+    const double k = (double)k_in, cols = (double)n_out * (swiglu ? 2 : 1);
+    const double weights = cols * k, outputs = (double)rows * cols;
+    auto g = [&](int64_t tile) { return weights * (double)((rows + tile - 1) / tile * tile) * 1e-9; };
+    const bool rows_again = (norm || swiglu) && (swiglu || n_out < kWideOutputs);
+    const int64_t cus = device_cu_count(), wg_cols = swiglu ? 64 : 128;
+    const int64_t wgs = (n_out + wg_cols - 1) / wg_cols * ((rows + 31) / 32);
+    return {5.0 + std::max(0.0035 * k, (rows_again ? 100.0 : 52.0) * g(16)),
+            10.0 + 1.33e-6 * weights + 2.2e-6 * (double)rows * k + std::max(0.0145 * k, 10.0 * g(64)) +
+                2.2e-6 * outputs,
+            3.5 + 0.035 * k * (double)((wgs + cus - 1) / cus) + 0.5e-6 * outputs};
 }
 
 // Whether a product takes the digits, given a workspace. Decode-sized batches never do: k_in

@@ -1133,7 +1133,7 @@ int linear_f64acc(const char* what, const float* x, int64_t ldx, const float* no
     // Wide outputs (the vocabulary projection): the persistent tile walk when the K range
     // fits its registers, else 4 column blocks per workgroup so each activation fragment
     // feeds 4 MFMAs; narrow ones keep a workgroup per 16 columns.
-    const bool wide = n_out >= 16 * 1024;
+    const bool wide = n_out >= kWideOutputs;
     const int64_t wide_rc = (k_in / kLinK + kLinWaves - 1) / kLinWaves;
     // the buffer ranges of the persistent walk are 32-bit
     const bool wide_fits = (int64_t)n_out * k_in * 2 < (1LL << 31) &&
