@@ -327,10 +327,13 @@ def test_no_room_for_the_digits(gpu, dev):
     total = torch.cuda.get_device_properties(dev).total_memory
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(dev) + (4 << 20)) / total, dev)
     try:
+        held = []  # blocks that the allocator still had
         with pytest.raises(torch.OutOfMemoryError):
-            torch.empty(need, dtype=torch.uint8, device=dev)
+            for _ in range(1000):
+                held.append(torch.empty(need, dtype=torch.uint8, device=dev))
         both(*outs[2:])
     finally:
+        held = None
         torch.cuda.set_per_process_memory_fraction(1.0, dev)
     assert int((outs[0] - outs[2]).abs().gt(0).sum()) <= outs[0].numel() // 20000
     torch.testing.assert_close(outs[1], outs[3], rtol=1e-6, atol=1e-9)
