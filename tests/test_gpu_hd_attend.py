@@ -375,6 +375,57 @@ def test_f32_queries_over_the_whole_range(gpu, dev, hd, power):
         assert float((got - want).abs().max()) <= TOL
 
 
+@pytest.mark.parametrize("hd,n_head,n_kv", [(32, 12, 3), (96, 12, 3), (128, 12, 3), (160, 6, 2), (192, 6, 2),
+                                            (224, 6, 2), (256, 6, 2)])
+def test_decode_of_long_contexts(gpu, dev, hd, n_head, n_kv):
+    """Nine and seventeen splits: the combine takes its partials in two and three batches."""
+    from crucible_amd import _lib
+    lib = _lib.load()
+    lens = [2048, 2049, 4200, 100]
+    g, stride, kv, (kp, vp), tables, q = _case(dev, hd + 13, hd, n_head, n_kv, lens)
+    d_len = torch.tensor(lens, dtype=torch.int32, device=dev)
+    geometry = (4, n_head, n_kv, hd, stride, 2, 1, kv, stride * 16)
+    outs = [torch.zeros(4, n_head * hd, device=dev) for _ in range(3)]
+    gpu.attention_decode_paged(q, kp, vp, outs[0], tables, d_len, *geometry)
+    gpu.attention_decode_paged(_unaligned(q), kp, vp, outs[1], tables, d_len, *geometry)
+    _lib.check(lib.crucible_attention_decode_paged(
+        q.data_ptr(), 0, kp.data_ptr(), vp.data_ptr(), outs[2].data_ptr(), 0, tables.data_ptr(),
+        d_len.data_ptr(), *geometry, None, 0, torch.cuda.current_stream().cuda_stream))
+    assert float((outs[0] - outs[1]).abs().max()) <= TOL
+    assert torch.equal(outs[2], outs[0])
+
+
+@pytest.mark.parametrize("hd", [32, 96, 128, 160, 192, 224, 256])
+@pytest.mark.parametrize("kv_dtype", [torch.float32, torch.float16])
+def test_fused_entries_at_every_dimension(gpu, dev, hd, kv_dtype):
+    """RoPE and both appends: pools byte for byte those of the RoPE split and the appends, outputs
+    to TOL of the generic kernel's on them."""
+    lens = [1, 16, 17, 300, 40, 0]
+    pos = [0, 15, 16, 299, 10, 3]
+    b, n_head, n_kv, layer = len(lens), 6, 2, 1
+    g, stride, kv, (kp, vp), tables, _ = _case(dev, hd + 15, hd, n_head, n_kv, lens)
+    d_len, d_pos = (torch.tensor(x, dtype=torch.int32, device=dev) for x in (lens, pos))
+    angle = torch.randn(stride * 16, hd // 2, generator=g, device=dev)
+    cos, sin = angle.cos().contiguous(), angle.sin().contiguous()
+    qkv = torch.randn(b, n_head * hd + 2 * kv, generator=g, device=dev)
+    q = torch.empty(b, n_head * hd, device=dev)
+    k, v = torch.empty(b, kv, device=dev), torch.empty(b, kv, device=dev)
+    gpu.rope_split_qkv(qkv, q, k, v, cos, sin, d_pos, n_head, n_kv, hd)
+    k, v = k.to(kv_dtype), v.to(kv_dtype)
+    geometry = (b, n_head, n_kv, hd, stride, 2, layer, kv, stride * 16)
+    pools = [[kp.clone(), vp.clone()] for _ in range(3)]
+    outs = [torch.full((b, n_head * hd), 7.0, device=dev) for _ in range(3)]
+    for src, pool, kind in ((k, pools[0][0], "k"), (v, pools[0][1], "v")):
+        gpu.cache_store_rows_paged(src, pool, tables, d_pos, b, kv, stride, 2, layer, kind=kind)
+    gpu.attention_decode_paged(_unaligned(q), *pools[0], outs[0], tables, d_len, *geometry)
+    gpu.attention_decode_paged_append(q, k, v, *pools[1], outs[1], tables, d_pos, d_len, *geometry)
+    gpu.attention_decode_qkv_paged_append(qkv, cos, sin, *pools[2], outs[2], tables, d_pos, d_len, *geometry)
+    for i in (1, 2):
+        assert torch.equal(pools[i][0], pools[0][0]) and torch.equal(pools[i][1], pools[0][1])
+        assert float((outs[i] - outs[0]).abs().max()) <= TOL
+        assert bool((outs[i][5] == 7.0).all())
+
+
 @pytest.mark.parametrize("hd", [128, 256])
 def test_workspace_shared_with_head_dim_64(gpu, dev, hd):
     """Calls of other head dimensions leave the counters and the unit plan of a workspace alone,
