@@ -1339,27 +1339,28 @@ __global__ __launch_bounds__(kGenericThreads) void decode_hd_combine_kernel(Deco
 template <bool F16>
 __global__ __launch_bounds__(256) void append_new_rows_kernel(DecodeArgs a, int hd) {
     const int half = hd >> 1;
-    const int64_t per_row = (int64_t)a.n_kv_head * half;
+    const uint32_t per_row = (uint32_t)a.n_kv_head * half;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (int64_t)a.batch * per_row) return;
-    const int b = (int)(i / per_row);
+    const int b = i <= UINT32_MAX ? (int)((uint32_t)i / per_row) : (int)(i / per_row);
     const int r = (int)(i - (int64_t)b * per_row);
     const int g = r / half;
     const int e = r - g * half;
+    const int c = g * hd + e;  // channel of the pair's first element
+    using T = std::conditional_t<F16, half_t, float>;
+    const T* kr = static_cast<const T*>(a.k_new) + (int64_t)b * a.kv_new_stride + c;
+    const T* vr = static_cast<const T*>(a.v_new) + (int64_t)b * a.kv_new_stride + c;
     const int pos = a.positions[b];
+    const T x0 = kr[0], x1 = kr[half], v0 = vr[0], v1 = vr[half];  // beside the position's load
     if (pos < 0 || (pos >> kPageShift) >= a.table_stride) return;
     const int64_t base = block_base(a.addr, a.tables[(int64_t)b * a.table_stride + (pos >> kPageShift)]);
     const int slot = pos & kPageMask;
-    const int c = g * hd + e;  // channel of the pair's first element
-    using T = std::conditional_t<F16, half_t, float>;
-    const T* kr = static_cast<const T*>(a.k_new) + (int64_t)b * a.kv_new_stride;
-    const T* vr = static_cast<const T*>(a.v_new) + (int64_t)b * a.kv_new_stride;
     half_t k0, k1;
     if constexpr (F16) {  // copied, not converted: the bytes of a NaN stay
-        k0 = kr[c];
-        k1 = kr[c + half];
+        k0 = x0;
+        k1 = x1;
     } else {
-        float lo = kr[c], hi = kr[c + half];
+        float lo = x0, hi = x1;
         if (a.rope_cos) {
             const int p = min(pos, a.rope_max_pos - 1);
             rope_pair(lo, hi, a.rope_cos[(int64_t)p * half + e], a.rope_sin[(int64_t)p * half + e]);
@@ -1370,8 +1371,8 @@ __global__ __launch_bounds__(256) void append_new_rows_kernel(DecodeArgs a, int 
     const int kv_dim = a.addr.kv_dim;
     a.k_pool[base + (int64_t)slot * kv_dim + c] = k0;
     a.k_pool[base + (int64_t)slot * kv_dim + c + half] = k1;
-    a.v_pool[base + (int64_t)c * kPageTokens + slot] = (half_t)vr[c];
-    a.v_pool[base + (int64_t)(c + half) * kPageTokens + slot] = (half_t)vr[c + half];
+    a.v_pool[base + (int64_t)c * kPageTokens + slot] = (half_t)v0;
+    a.v_pool[base + (int64_t)(c + half) * kPageTokens + slot] = (half_t)v1;
 }
 
 struct DecodeShape {
