@@ -1149,8 +1149,14 @@ constexpr int kHdSplitPages = 16;
 // be, straight to the output; or, without scratch, all of them.
 enum HdShare { kHdSplit, kHdOnly, kHdWalk };
 
+// Waves a SIMD that the registers leave room for: three workgroups of 32 dims a CU (684 units of one
+// split: 7.2 us a launch, 8.2 at two), two up to 128.
+constexpr int hd_min_waves(int hd, int share) {
+    return share == kHdWalk || hd > 128 ? 1 : hd == 32 ? 6 : 4;
+}
+
 template <int HD, bool QF32, int SHARE>
-__global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 && SHARE != kHdWalk ? 4 : 1) void decode_hd_kernel(
+__global__ __launch_bounds__(64 * hd_waves(HD), hd_min_waves(HD, SHARE)) void decode_hd_kernel(
     DecodeArgs a, int col_blocks) {
     constexpr int W = hd_waves(HD);
     __shared__ HdLds<HD, W, 1> lds;
@@ -1243,8 +1249,16 @@ __global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 && SHARE != kHdWalk ? 
     if constexpr (SHARE != kHdWalk) total = s[0];
     const bool mine = wave == 0 && col < n_cols;
     if constexpr (SHARE == kHdSplit) {
-        if (!mine) return;
+        if (wave != 0) return;
         const int64_t slot = ((int64_t)b * a.n_head + h) * a.n_splits + s0;
+        if (n_active == 1) {  // the output itself; the combine only asks whether it is finite
+            const uint32_t cols = hd_not_finite(total, mine);
+            if (!mine) return;
+            hd_store(a.out, a.out_f16, (int64_t)b * a.out_row_stride + (int64_t)h * HD, total, grp);
+            if (grp == 0) a.pl[slot] = cols >> col & 1 ? __builtin_nanf("") : 1.0f;
+            return;
+        }
+        if (!mine) return;
 #pragma unroll
         for (int i = 0; i < HD / 16; ++i)
             *reinterpret_cast<float4_t*>(a.po + slot * HD + 16 * i + 4 * grp) = total.o[i];
@@ -1260,7 +1274,9 @@ __global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 && SHARE != kHdWalk ? 
             if (lane == 0) s_again = cols;
         }
         if (mine) hd_store(a.out, a.out_f16, (int64_t)b * a.out_row_stride + (int64_t)h * HD, total, grp);
-        __syncthreads();
+        lds_barrier();
+        if (s_again == 0) return;
+        __syncthreads();  // the stores above before those below
         for (uint32_t left = s_again; left != 0; left &= left - 1) {
             const DecodeArgs& c = cold_args<DecodeArgs>();
             decode_generic_head<QF32>(again, c, HD, blockIdx.y, g * c.n_rep + c0 + __builtin_ctz(left), len);
@@ -1275,14 +1291,13 @@ __global__ __launch_bounds__(64 * hd_waves(HD), HD <= 128 && SHARE != kHdWalk ? 
 template <bool QF32>
 __global__ __launch_bounds__(kGenericThreads) void decode_hd_combine_kernel(DecodeArgs a, int hd) {
     __shared__ GenericLds again;
-    __shared__ uint32_t s_again;  // of the workgroup's rows, at most 32
+    __shared__ uint64_t s_again[kGenericWaves];  // the threads whose quad is not finite
     const int quads = hd >> 2;
     const int rows = kGenericThreads / quads;
     const int mine = threadIdx.x / quads;
     const int64_t row0 = (int64_t)blockIdx.x * rows;
     const int64_t row = row0 + mine;  // b * n_head + h
-    if (threadIdx.x == 0) s_again = 0;
-    __syncthreads();
+    bool again_mine = false;
     if (mine < rows && row < (int64_t)a.batch * a.n_head) {
         const int d = 4 * (threadIdx.x - mine * quads);
         const int b = (int)(row / a.n_head);
@@ -1302,8 +1317,11 @@ __global__ __launch_bounds__(kGenericThreads) void decode_hd_combine_kernel(Deco
         };
         load(0);
         const int len = request_len(a, b);
-        if (len > 0) {
-            const int n_active = ((len + kPageMask) / kPageTokens + kHdSplitPages - 1) / kHdSplitPages;
+        const int n_active =
+            len > 0 ? ((len + kPageMask) / kPageTokens + kHdSplitPages - 1) / kHdSplitPages : 0;
+        if (n_active == 1) {  // written by its only split
+            again_mine = !(t[0].l == 1.0f);
+        } else if (n_active > 1) {
             HdState<16> total;  // one quad of dims
             for (int j0 = 0; j0 < n_active; j0 += kAhead) {
                 if (j0 > 0) load(j0);
@@ -1317,13 +1335,23 @@ __global__ __launch_bounds__(kGenericThreads) void decode_hd_combine_kernel(Deco
             const float4_t v = total.o[0] * (1.0f / total.l);
             store_out4(a, (int64_t)b * a.out_row_stride + (row - (int64_t)b * a.n_head) * hd + d, v);
             const float z = ((v[0] * 0.0f + v[1] * 0.0f) + v[2] * 0.0f) + v[3] * 0.0f;
-            if (!(z == 0.0f)) atomicOr(&s_again, 1u << mine);
+            again_mine = !(z == 0.0f);
         }
     }
-    __syncthreads();
-    for (uint32_t left = s_again; left != 0; left &= left - 1) {
+    const uint64_t bad = __ballot(again_mine);
+    if ((threadIdx.x & 63) == 0) s_again[threadIdx.x >> 6] = bad;
+    lds_barrier();
+    uint64_t any = 0;
+#pragma unroll
+    for (int w = 0; w < kGenericWaves; ++w) any |= s_again[w];
+    if (any == 0) return;
+    __syncthreads();  // the stores above before those below
+    for (int r = 0; r < rows; ++r) {
+        bool again_row = false;
+        for (int t = r * quads; t < (r + 1) * quads; ++t) again_row |= (s_again[t >> 6] >> (t & 63) & 1) != 0;
+        if (!again_row) continue;
         const DecodeArgs& c = cold_args<DecodeArgs>();
-        const int64_t at = (int64_t)blockIdx.x * rows + __builtin_ctz(left);
+        const int64_t at = (int64_t)blockIdx.x * rows + r;
         const int b = (int)(at / c.n_head);
         decode_generic_head<QF32>(again, c, hd, b, (int)(at - (int64_t)b * c.n_head), request_len(c, b));
     }
@@ -1580,20 +1608,26 @@ DecodeArgs common_args(const void* q, const void* k, const void* v, void* out, i
 // decode_hd_kernel gains is one K/V read for the heads of a group and workgroups for every split;
 // with one or two heads a group and enough requests, or contexts of one split, neither counts, and
 // its wide workgroups and their merge cost more. us with scratch against generic, at full contexts:
-//   one head a group, 512 units (request, kv head) or more: 55.7 / 43.4 (128 dims, 128 x 500 keys,
-//     8 kv heads), 43.3 / 34.2 (96); 256 or more from 160 dims on: 44.6 / 34.8 (64 x 1,000, 4);
-//     at 16 x 2,000 keys the other way: 33.9 / 50.9 (128), 28.3 / 47.8 (96)
+//   one head a group, 96 or 128 dims, 512 units (request, kv head) or more, up to 1,024 tokens of
+//     capacity: 55.7 / 43.4 (128 x 500 keys, 8 kv heads of 128), 88 / 78 (102 ragged requests, 12
+//     of 128), 43.3 / 34.2 (96); at 1,696 tokens of capacity, ragged, the other way: 79 / 87 (55
+//     requests, 12 of 96), and at 16 x 2,000: 33.9 / 50.9 (128), 28.3 / 47.8 (96)
+//   one head a group, 160 dims or more, 256 units or more: 44.6 / 34.8 (64 x 1,000, 4 of 160)
 //   one head a group, one split, 128 dims or more: 8.4 / 7.3 (16 x 200, 128), 24.6 / 11.7 (128 x 60, 160)
 //   two heads, one split, 160 dims or more: 16.3 / 13.0 (64 x 100, 160), 22.1 / 16.4 (256)
 //   few units, one split, 192 dims or more: 9.7 / 8.3 (1 x 100, 12/3 heads of 256)
+// Not at 32 dims, whose 1 KB blocks of a pool of several layers cost the generic kernel more: 13.0
+// / 17.0 a layer (122 ragged requests, 12 heads).
 // By the shape alone, so that calls with and without scratch, and the separate and fused entries,
 // give the same bits.
 bool generic_decode_faster(const DecodeArgs& a, int hd) {
     const int64_t units = (int64_t)a.batch * a.n_kv_head;
     const bool one_split = a.max_pages <= kHdSplitPages;
-    if (a.n_rep == 1 && (units >= (hd >= 160 ? 256 : 512) || (one_split && hd >= 128))) return true;
-    if (a.n_rep == 2 && one_split && hd >= 160) return true;
-    return one_split && hd >= 192 && units < 32;
+    if (a.n_rep == 1 && hd >= 128 && one_split) return true;
+    if (a.n_rep == 1 && hd >= 160 && units >= 256) return true;
+    if (a.n_rep == 1 && hd >= 96 && units >= 512 && a.max_pages <= 4 * kHdSplitPages) return true;
+    if (a.n_rep == 2 && hd >= 160 && one_split) return true;
+    return hd >= 192 && one_split && units < 32;
 }
 
 // Whether decode_hd_kernel takes the call: its vector accesses need 16-byte rows, its grid

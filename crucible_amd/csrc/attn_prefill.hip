@@ -1908,7 +1908,11 @@ __global__ __launch_bounds__(64 * W, W == 8 ? 4 : 1) void prefill_hd_kernel(Pref
     if (wave == 0 && grp == 0)
 #pragma unroll
         for (int b = 0; b < QB; ++b) s_row[16 * b + col] = row[b];
-    __syncthreads();
+    lds_barrier();
+    uint32_t any_again = 0;
+#pragma unroll
+    for (int b = 0; b < QB; ++b) any_again |= s_again[b];
+    if (any_again == 0) return;
 #pragma unroll
     for (int b = 0; b < QB; ++b)
         for (uint32_t left = s_again[b]; left != 0; left &= left - 1) {

@@ -282,6 +282,13 @@ __device__ __forceinline__ uint32_t hd_not_finite(const HdState<HD>& s, bool min
     return (uint32_t)(bad | bad >> 16 | bad >> 32 | bad >> 48) & 0xffffu;
 }
 
+// A barrier for LDS alone: __syncthreads would also wait for the outputs' stores on their way.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // The kernel's first argument read from the argument block where it is used, in a branch that
 // hardly runs: its fields would otherwise stay in scalar registers through the main loop.
 template <class Args>
