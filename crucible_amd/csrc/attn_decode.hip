@@ -1137,12 +1137,13 @@ __global__ __launch_bounds__(kGenericThreads) void decode_generic_kernel(DecodeA
 // callers of these dimensions never had to clear or own one. HBM-bound at large batches,
 // latency-bound below; the split is small because one CU streams only 25-50 GB/s. 16 requests
 // of 64..2048 tokens, 12/3 heads of 128, fused append (26 MB): 70 us a layer with
-// attend_generic, 22.2 here with the append and the combine launches. Up to 128 dims the
-// registers of the one-split forms are capped at 128, so that two workgroups share a CU (20 bytes
-// a lane spill at 128 dims; uncapped it took 22 us against 19). The walk's second state does not
-// fit there (300 to 400 bytes a lane spilled), so it takes what it needs; it is bound by its CU's
-// stream: 1 x 2,048 tokens 38 us, 16 x 1,000 22, 128 x 100 9.8 (12/3 heads of 128; the generic
-// kernel 35, 22 and 16; 76, 44 and 21 against 69, 36 and 25 at 256 dims).
+// attend_generic, 23 here with the append and the combine launches (traced 4.3, 13.0 and 5.0).
+// Up to 128 dims the registers of the one-split forms are capped (hd_min_waves), so that
+// workgroups share a CU (20 to 36 bytes a lane spill at 128 dims; uncapped it took 22 us against
+// 19). The walk's second state does not fit there (300 to 400 bytes a lane spilled), so it takes
+// what it needs; it is bound by its CU's stream: 1 x 2,048 tokens 38 us, 16 x 1,000 22, 128 x 100
+// in one split 9.8 (12/3 heads of 128; the generic kernel 35, 22 and 16; at 256 dims 76, 44 and 21
+// against 69, 36 and 25).
 constexpr int kHdSplitPages = 16;
 
 // A workgroup's share of a unit: one split, its partial to the scratch; the only split there can

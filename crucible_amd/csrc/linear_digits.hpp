@@ -145,8 +145,9 @@ constexpr int kDigitThreads = 256;
 // Memory-bound: 4 B read and 6 written per activation, 2 and 4 per weight. A thread
 // handles groups of 16 consecutive K of a row, the 16 bytes one lane supplies to an MFMA for
 // each digit; 8 neighbouring lanes hold 8 rows, so a digit's stores are 128-byte runs (8 rows
-// a workgroup against 16: 4,713 x 2048 22.4 -> 19.4 us, 1,003 x 768 12.6 -> 11.4). The digits need the row's norm and largest value first: with G > 0 (k_in <= 512 G) a thread's
-// groups wait in registers, loaded at once; G = 0 reads the row twice.
+// a workgroup against 16: 4,713 x 2048 22.4 -> 19.4 us, 1,003 x 768 12.6 -> 11.4). The digits
+// need the row's norm and largest value first: with G > 0 (k_in <= 512 G) a thread's groups wait
+// in registers, loaded at once; G = 0 reads the row twice.
 template <int G, bool NORM>
 __global__ __launch_bounds__(kDigitThreads) void digits_kernel(DigitArgs a) {
     __shared__ double s_ss[32][kWgRows];
@@ -475,8 +476,9 @@ __device__ __forceinline__ void f64_block(const DigitArgs& a, int row_blk, int c
     else go(std::false_type{});
 }
 
-// A 64 x 64 output tile per workgroup of 4 waves, 32 x 32 a wave. MFMA-bound: 18 products of
-// 32x32x32 a wave and step (24 with the fourth weight digit) against 9 KiB of LDS reads.
+// A 64 x 64 output tile per workgroup of 4 waves, 32 x 32 a wave. MFMA-bound: 15 products of
+// 32x32x32 a wave and step (18 with the last activation digit, up to 24 with the fourth weight
+// digit) against 9 KiB of LDS reads.
 // Stages of 64 keys stream into two LDS buffers with direct-to-LDS loads, the next stage's
 // issued between the products; the planes are stored in operand order, so both the copy and
 // the reads are linear in the lane and free of bank conflicts. Two workgroups a CU (73.7 KB
@@ -484,7 +486,7 @@ __device__ __forceinline__ void f64_block(const DigitArgs& a, int row_blk, int c
 // digit, rare, goes from global memory to registers.
 //
 // With every SIMD busy on random digits the part runs a 32x32x32 product in 20 ns (13.7 with
-// a few CUs busy): 150 us for the gate/up product of 4,713 rows (252 G multiply-adds).
+// a few CUs busy): 133 to 160 us for the gate/up product of 4,713 rows, traced 205.
 // Measured slower: steps of 32 in a ring of 4 (2 workgroups a CU) or 8 buffers, operands
 // double-buffered in registers, 32 x 64 outputs a wave (one wave a SIMD, 512 VGPRs), and, for
 // grids below the CU count, a second set of 4 waves on every other stage of K.

@@ -153,12 +153,13 @@ int crucible_cache_store_packed_paged(const void* src, int src_dtype, void* pool
  * when q, out and the RoPE tables are 16-byte aligned and rows of q start there: splits of 16 pages, joined by a second launch when the call brings a
  * workspace that holds them (uncleared; only its partials' part, behind the counters and the
  * plan described below, is written) and by the same workgroup, with the same bits, when it does
- * not. The remaining multiples of 8, and
- * unaligned buffers, run a generic kernel (one workgroup per request and query head, f32
- * arithmetic, no workspace). For every head_dim other than 64 the pool layout and the results
- * are the same to the tolerance of f32 accumulation, the fused entries write the bytes of the
- * separate appends, and attention_split leaves its partial buffers untouched. The same holds
- * for the prefill entries below.
+ * not. The remaining multiples of 8, unaligned buffers, and shapes where it is faster (one or
+ * two query heads a group with many requests or short capacities) run a generic kernel (one
+ * workgroup per request and query head, f32 arithmetic, no workspace). For every head_dim other
+ * than 64 the pool layout and the results are the same to the tolerance of f32 accumulation,
+ * infinities and NaN included, the fused entries write the bytes of the separate appends, and
+ * attention_split leaves its partial buffers untouched. The same holds for the prefill entries
+ * below.
  * The split-K partials live in a caller-provided workspace of at least
  * crucible_attention_decode_workspace_bytes(...) bytes (no allocation here; 0 for an
  * empty batch, SIZE_MAX for a shape past the entry points' limits), 16-byte aligned.
