@@ -488,3 +488,42 @@ def test_the_callers_workspace_is_used(gpu, dev, hd):
     assert not small.any() and torch.equal(out, want)
     with pytest.raises(CrucibleError):
         run(torch.zeros(need, dtype=torch.uint8))
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+def test_captured_calls_replay(gpu, dev, hd):
+    """The fused decode with scratch of its own, and a projection on digits, captured in a graph:
+    every replay on new inputs, with eager work between, gives the eager calls' outputs."""
+    lens, n_head, n_kv, layer = [600, 33, 257], 12, 3, 1
+    b = len(lens)
+    g, stride, kv, (kp, vp), tables, q = _case(dev, hd + 17, hd, n_head, n_kv, lens)
+    d_len = torch.tensor(lens, dtype=torch.int32, device=dev)
+    new = [torch.randn(b, kv, generator=g, device=dev) for _ in "kv"]
+    x = torch.randn(300, 768, generator=g, device=dev)
+    w = torch.randn(1152, 768, generator=g, device=dev).mul_(0.02).half()
+    nw = torch.ones(768, device=dev)
+    out, y = torch.zeros(b, n_head * hd, device=dev), torch.zeros(300, 1152, device=dev)
+    assert gpu.lib.crucible_linear_workspace_bytes(300, 1152, 768, 1, 0) > 0
+
+    def step(o, p):
+        gpu.attention_decode_paged_append(q, *new, kp, vp, o, tables, d_len - 1, d_len, b, n_head, n_kv, hd,
+                                          stride, 2, layer, kv, stride * 16)
+        gpu.linear_f64acc(x, w, p, norm_w=nw)
+
+    step(out, y)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step(out, y)
+    for _ in range(4):
+        for t in (q, *new, x):
+            t.copy_(torch.randn(t.shape, generator=g, device=dev))
+        x[5] *= 1e-3
+        x[5, 0] = float("inf")  # f64 sums for its block
+        want, wy = torch.zeros_like(out), torch.zeros_like(y)
+        step(want, wy)
+        torch.cuda.synchronize()
+        out.zero_(), y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert torch.equal(y.nan_to_num(nan=7.0), wy.nan_to_num(nan=7.0))
